@@ -1130,10 +1130,6 @@ int lp_convex_hulls(lp_context* c, const double* x, const double* y, const int32
     if (total) {
         LP_HIP(hipMemcpyAsync(c->d.hcx, x, total * sizeof(double), hipMemcpyHostToDevice, c->stream));
         LP_HIP(hipMemcpyAsync(c->d.hcy, y, total * sizeof(double), hipMemcpyHostToDevice, c->stream));
-        // (x, y) pairs kept for the canonical index among identical points.
-        LP_HIP(hipMemcpy2DAsync(c->d.dsort, 16, x, 8, 8, total, hipMemcpyHostToDevice, c->stream));
-        LP_HIP(hipMemcpy2DAsync(reinterpret_cast<char*>(c->d.dsort) + 8, 16, y, 8, 8, total, hipMemcpyHostToDevice,
-                                c->stream));
     }
     launch_hull_lists(c, num_lists, total);
     LP_HIP(hipGetLastError());
