@@ -11,15 +11,19 @@
 // the float-rounded value exactly as the reference does.
 //
 // Polygons of up to 64 vertices (nearly all hulls) take one wavefront each,
-// larger ones a workgroup.  One lane walks the antipodal pairs and the
-// centroid is summed in the reference's order.  The candidates (i, -1) and
-// (i - 1, +1) share one edge with opposite directions, which negates every
-// rotated coordinate exactly and leaves the area bit-identical, so one area
-// is evaluated per edge, O(n) each, a lane per edge; one wavefront then
-// applies the sequential selection rule over the candidates in the
-// reference's order (64 at a time, through a prefix minimum of the areas) and
-// recomputes the chosen candidate's extents in its own direction for the
-// corners.
+// larger ones a workgroup, in one launch.  The antipodal walk is a serial
+// chain (about 2.5 steps per vertex, 300 cycles each: two thirds of the
+// stage's time when one lane walked it), but its state at every vertex i is
+// where the area of (i, i+1, j) stops growing, so all rows are found at once
+// by binary search and the whole walk is then checked step by step in
+// parallel with the reference's own comparisons; a walk that differs anywhere
+// (rounded ties, polygons that are not convex) is redone by one lane.  The
+// candidates (i, -1) and (i - 1, +1) share one edge with opposite directions,
+// which negates every rotated coordinate exactly and leaves the area
+// bit-identical, so one area is evaluated per edge, O(n) each, a lane per
+// edge; the sequential selection rule over the candidates is applied by two
+// reductions.  64x2048 frame of 40 cars: 96 -> 19 us (two launches before),
+// 331 polygons of 13 vertices on average: 81 -> 19 us.
 #include <algorithm>
 
 #include "lp_device.h"
@@ -34,85 +38,75 @@ namespace {
 
 constexpr int kBoxThreads = 256;
 // Polygons of up to kBoxVerts vertices are held in LDS (larger: capacity
-// error).  Antipodal pairs: at most 3n/2, room for 2n.
+// error).
 constexpr int kBoxVerts = 1024;
 
 // areaOfTriangle (polygonizer.hpp:228-231), same operand order.
-__device__ __forceinline__ double tri_area_xy(double ax, double ay, double bx, double by, double cx, double cy) {
-    return fabs((ax * (by - cy) + bx * (cy - ay) + cx * (ay - by)) * 0.5);
+__device__ __forceinline__ double tri_area(const double2& a, const double2& b, const double2& c) {
+    return fabs((a.x * (b.y - c.y) + b.x * (c.y - a.y) + c.x * (a.y - b.y)) * 0.5);
 }
 
 __device__ __forceinline__ int wrap(int k, int n) { return k >= n ? k - n : k; }
 
-// Antipodal pairs of polygon (n >= 3 vertices) in the reference's order
+// Antipodal pairs of polygon V (n >= 3 vertices) in the reference's order
 // (polygonizer.cpp:93-161), walked as one sequential chain with the areas of
-// the running pair carried from step to step.  vert(stream, k, x, y) fetches
-// vertex k; stream 0 serves i and stream 1 serves j, and each stream's
-// vertex indices advance by one (mod n) from call to call.  emit(c, i, j)
-// records pair c.  Returns the count, or -1 when the walk exceeds 4n + 8
-// steps or `cap` pairs (the reference's loop need not end on degenerate
-// input).
-template <typename Vert, typename Emit>
-__device__ __forceinline__ int antipodal_walk(int n, int cap, Vert vert, Emit emit) {
+// the running pair carried from step to step.  emit(i, j) receives the pairs.
+// Returns false when the walk exceeds 4n + 8 steps or `cap` pairs (the
+// reference's loop need not end on degenerate input).
+template <typename Emit>
+__device__ __forceinline__ bool antipodal_walk(const double2* V, int n, int cap, Emit emit) {
     const int i0 = n - 1;
     const int limit = 4 * n + 8;
     int guard = 0, count = 0;
     int i = 0, j = 1;
-    double xi, yi, xi1, yi1, xj, yj, xn, yn;
-    vert(0, 0, xi, yi);
-    vert(0, 1, xi1, yi1);
-    xj = xi1;
-    yj = yi1;
+    double2 vi = V[0], vi1 = V[1], vj = V[1];
     int jn = wrap(2, n);
-    vert(1, jn, xn, yn);
-    double a_cur = tri_area_xy(xi, yi, xi1, yi1, xj, yj);
+    double2 vn = V[jn];
+    double a_cur = tri_area(vi, vi1, vj);
     // while (area(i, i+1, j+1) > area(i, i+1, j)) ++j
     for (;;) {
-        const double a_nx = tri_area_xy(xi, yi, xi1, yi1, xn, yn);
+        const double a_nx = tri_area(vi, vi1, vn);
         if (!(a_nx > a_cur)) break;
         j = jn;
-        xj = xn;
-        yj = yn;
+        vj = vn;
         a_cur = a_nx;
         jn = wrap(j + 1, n);
-        vert(1, jn, xn, yn);
-        if (++guard > limit) return -1;
+        vn = V[jn];
+        if (++guard > limit) return false;
     }
     const int j0 = j;
     while (i != j0) {
         i = wrap(i + 1, n);
-        xi = xi1;
-        yi = yi1;
+        vi = vi1;
         const int i1 = wrap(i + 1, n);
-        vert(0, i1, xi1, yi1);
-        if (count >= cap) return -1;
-        emit(count++, i, j);
-        a_cur = tri_area_xy(xi, yi, xi1, yi1, xj, yj);
+        vi1 = V[i1];
+        if (count++ >= cap) return false;
+        emit(i, j);
+        a_cur = tri_area(vi, vi1, vj);
         for (;;) {
-            const double a_nx = tri_area_xy(xi, yi, xi1, yi1, xn, yn);
+            const double a_nx = tri_area(vi, vi1, vn);
             if (!(a_nx > a_cur)) break;
             j = jn;
-            xj = xn;
-            yj = yn;
+            vj = vn;
             a_cur = a_nx;
             jn = wrap(j + 1, n);
-            vert(1, jn, xn, yn);
-            if (i == j0 && j == i0) return count;
-            if (count >= cap) return -1;
-            emit(count++, i, j);
-            if (++guard > limit) return -1;
+            vn = V[jn];
+            if (i == j0 && j == i0) return true;
+            if (count++ >= cap) return false;
+            emit(i, j);
+            if (++guard > limit) return false;
         }
         // areaOfTriangle(j, i+1, j+1) == areaOfTriangle(i, i+1, j)
-        if (tri_area_xy(xj, yj, xi1, yi1, xn, yn) == a_cur) {
-            if (count >= cap) return -1;
+        if (tri_area(vj, vi1, vn) == a_cur) {
+            if (count++ >= cap) return false;
             if (i == j0 && j == i0)
-                emit(count++, i1, j);
+                emit(i1, j);
             else
-                emit(count++, i, jn);
+                emit(i, jn);
         }
-        if (++guard > limit) return -1;
+        if (++guard > limit) return false;
     }
-    return count;
+    return true;
 }
 
 // Extents of the polygon rotated into the frame of unit direction (ux, uy)
@@ -135,15 +129,14 @@ __device__ __forceinline__ Extent extent_init() {
 
 // Candidate edge (idx, idx + off) of the reference: unit direction, or
 // false when shorter than 1e-6.
-__device__ __forceinline__ bool cand_dir(const double* X, const double* Y, int n, int idx, int off, double& ux,
-                                         double& uy) {
+__device__ __forceinline__ bool cand_dir(const double2* V, int n, int idx, int off, double& ux, double& uy) {
     int nb = idx + off;
     if (nb < 0)
         nb += n;
     else if (nb >= n)
         nb -= n;
-    const double ex = X[nb] - X[idx];
-    const double ey = Y[nb] - Y[idx];
+    const double ex = V[nb].x - V[idx].x;
+    const double ey = V[nb].y - V[idx].y;
     const double len = sqrt(ex * ex + ey * ey);
     if (len < 1.0e-6) return false;
     ux = ex / len;
@@ -153,72 +146,239 @@ __device__ __forceinline__ bool cand_dir(const double* X, const double* Y, int n
 
 // Area of the box in the frame of edge e (e -> e+1), or NaN when the edge is
 // shorter than 1e-6.  The candidates (e, +1) and (e + 1, -1) share it.
-// vert(q, x, y) fetches vertex q for the extents (the same for every lane).
-template <typename Vert>
-__device__ __forceinline__ double edge_box_area(const double* X, const double* Y, int n, int e, double cx, double cy,
-                                                Vert vert) {
+// fmin / fmax keep the same extents as extent_add up to the sign of a zero,
+// which can only show in an area of zero: such an edge is evaluated again in
+// the reference's own order.
+__device__ __forceinline__ double edge_box_area(const double2* V, int n, int e, double cx, double cy) {
     double ux, uy;
-    if (!cand_dir(X, Y, n, e, 1, ux, uy)) return __builtin_nan("");
+    if (!cand_dir(V, n, e, 1, ux, uy)) return __builtin_nan("");
     Extent ex = extent_init();
-    // Unrolled so the vertex fetches of two steps are in flight together;
-    // the order of the updates stays.
-#pragma unroll 2
+#pragma unroll 4
     for (int q = 0; q < n; ++q) {
-        double xq, yq;
-        vert(q, xq, yq);
-        const double tx = xq - cx;
-        const double ty = yq - cy;
+        const double tx = V[q].x - cx;
+        const double ty = V[q].y - cy;
+        const double rx = tx * ux + ty * uy;
+        const double ry = -tx * uy + ty * ux;
+        ex.mnx = fmin(ex.mnx, rx);
+        ex.mxx = fmax(ex.mxx, rx);
+        ex.mny = fmin(ex.mny, ry);
+        ex.mxy = fmax(ex.mxy, ry);
+    }
+    const double area = (ex.mxx - ex.mnx) * (ex.mxy - ex.mny);
+    if (area != 0.0) return area;
+    ex = extent_init();
+    for (int q = 0; q < n; ++q) {
+        const double tx = V[q].x - cx;
+        const double ty = V[q].y - cy;
         extent_add(ex, tx * ux + ty * uy, -tx * uy + ty * ux);
     }
     return (ex.mxx - ex.mnx) * (ex.mxy - ex.mny);
 }
 
-// The reference's sequential choice among the 4 * np candidates of the
-// antipodal pairs, run by one whole wavefront (every lane returns the same
-// box).  Candidate c: pair c/4, vertex (c & 2 ? j : i), offset (c & 1 ? +1 :
-// -1); a candidate replaces the box when its area is below the float running
-// minimum (polygonizer.cpp:257).  `area` holds the area of every edge.
-__device__ void choose_box(const double* X, const double* Y, int n, const double* area, const int2* pairs, int np,
-                           double cx, double cy, lp_bounding_box& box) {
-    const int lane = lane_id();
-    // The running minimum after candidate c is float(min of the areas up to
-    // c): float rounding is monotone, so a candidate that does not replace
-    // the box lies between the smallest area so far and its float value and
-    // rounds to the same float.  So candidate c replaces the box exactly when
-    // its area is below float(min of the areas before it), which a prefix
-    // minimum over the lanes gives for 64 candidates at once; the box is the
-    // last replacing candidate.  NaN areas (short edges, no candidate) never
-    // replace and do not enter the minimum.
-    float best = __builtin_inff();  // float(DBL_MAX)
-    int sel = -1;
-    const int nc = 4 * np;
-    for (int base = 0; base < nc; base += kWave) {
-        const int c = base + lane;
-        double a = __builtin_nan("");
-        if (c < nc) {
-            const int2 pr = pairs[c >> 2];
-            const int idx = (c & 2) ? pr.y : pr.x;
-            a = area[(c & 1) ? idx : (idx == 0 ? n - 1 : idx - 1)];
-        }
-        double incl = (a == a) ? a : __builtin_inf();
-#pragma unroll
-        for (int o = 1; o < kWave; o <<= 1) {
-            const double u = __shfl_up(incl, o, kWave);
-            if (lane >= o) incl = fmin(incl, u);
-        }
-        double excl = __shfl_up(incl, 1, kWave);
-        if (lane == 0) excl = __builtin_inf();
-        const float before = fminf(best, static_cast<float>(excl));
-        const uint64_t rep = __ballot(a < static_cast<double>(before));
-        if (rep) sel = base + 63 - __clzll(static_cast<long long>(rep));
-        best = fminf(best, static_cast<float>(__shfl(incl, kWave - 1, kWave)));
+// A group of NT threads (a wavefront, or the whole workgroup).
+template <int NT>
+__device__ __forceinline__ void group_sync() {
+    if (NT == kWave)
+        wave_sync();
+    else
+        __syncthreads();
+}
+
+// Whether `v` holds on any thread of the group; the group is in step
+// afterwards.
+template <int NT>
+__device__ __forceinline__ bool group_any(bool v) {
+    if (NT == kWave) {
+        const bool r = __ballot(v) != 0;
+        wave_sync();
+        return r;
     }
-    if (sel < 0) return;
-    // The chosen candidate in its own direction.
-    const int2 pr = pairs[sel >> 2];
-    const int idx = (sel & 2) ? pr.y : pr.x;
+    return __syncthreads_or(v ? 1 : 0) != 0;
+}
+
+// The smallest (area, position) pair and the last position are kept with the
+// candidate they belong to: vertex * 2 + (offset + 1) / 2.
+struct CandMin {
+    double area;
+    int pos;
+    int cand;
+};
+
+__device__ __forceinline__ void cand_min(CandMin& m, double area, int pos, int cand) {
+    if (area < m.area || (area == m.area && pos < m.pos)) m = CandMin{area, pos, cand};
+}
+
+// The candidate that the reference's sequential rule ends with, for a walk
+// done by all NT threads: cand (as in CandMin) and the smallest area, or -1
+// when no candidate has an area, or kWalkSerial when the sequential walk has
+// to decide.  V, area in LDS; J (n entries), par (n / 32 + 1 words) and red
+// (NT / 64 entries) are LDS scratch.
+//
+// Walk: row i starts at j = J[i - 1] (row 0 at 1) and advances to J[i], the
+// first j whose next vertex does not enlarge the triangle (j runs on past n;
+// vertex j - n is meant); rows run to j0 = J[0].  Element t of the walk is
+// (i, t - i + 1) with i the first row with J[i] - 1 + i >= t.  Every element
+// but a row's last must advance and the last must not; with that the rows are
+// the sequential walk's, whatever guessed them.  Row j0 ends the walk when it
+// advances to vertex n - 1.
+//
+// Rule: a candidate replaces the box when its area is below the float of the
+// smallest area before it (float rounding is monotone, so that is the float
+// running minimum of polygonizer.cpp:257).  After the first candidate of the
+// overall smallest area m only areas below float(m) replace, so the last of
+// those is the answer; without one it is that first candidate, if m is below
+// the float of the smallest area before it.
+constexpr int kWalkSerial = -2;
+
+template <int NT>
+__device__ int choose_candidate(const double2* V, const double* area, int n, int cap, int tid, uint16_t* J,
+                                uint32_t* par, CandMin* red, double& smallest) {
+    auto advances = [&](int i, int j) {
+        const double2 a = V[i], b = V[wrap(i + 1, n)];
+        return tri_area(a, b, V[wrap(j + 1, n)]) > tri_area(a, b, V[wrap(j, n)]);
+    };
+    for (int i = tid; i < n; i += NT) {
+        int lo = i + 1, hi = i + n - 1;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (advances(i, mid))
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        J[i] = static_cast<uint16_t>(lo);
+    }
+    for (int q = tid; q <= n >> 5; q += NT) par[q] = 0;
+    group_sync<NT>();
+    const int j0 = J[0];  // 1 .. n - 1
+    const bool early = J[j0 - 1] < n - 1 && J[j0] >= n - 1;
+    const int jl = early ? n - 1 : J[j0];
+    bool bad = false;
+    for (int i = 1 + tid; i <= j0; i += NT) bad |= J[i] < J[i - 1];
+    if (group_any<NT>(bad)) return kWalkSerial;
+    if (tid == 0) J[j0] = static_cast<uint16_t>(jl);
+    group_sync<NT>();
+    const int elements = jl + j0;
+    auto row_of = [&](int t) {
+        int lo = 0, hi = j0;
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (J[mid] - 1 + mid >= t)
+                hi = mid;
+            else
+                lo = mid + 1;
+        }
+        return lo;
+    };
+    for (int t = tid; t < elements; t += NT) {
+        const int i = row_of(t), j = t - i + 1;
+        const bool end = j == J[i];
+        const bool last = end && early && i == j0;
+        bad |= !last && advances(i, j) == end;
+        if (end && !last && i > 0) {
+            const double2 vi1 = V[wrap(i + 1, n)];
+            const double2 vj = V[wrap(j, n)];
+            if (tri_area(vj, vi1, V[wrap(j + 1, n)]) == tri_area(V[i], vi1, vj))
+                atomicOr(&par[i >> 5], 1u << (i & 31));
+        }
+    }
+    if (group_any<NT>(bad)) return kWalkSerial;
+    int pairs = elements - j0 - (early ? 1 : 0);  // row 0 has j0 elements and no pairs
+    for (int q = 0; q <= j0 >> 5; ++q) pairs += __popc(par[q]);
+    if (pairs > cap) return kWalkSerial;
+    // Candidates of the walk's pairs: visit(position, vertex, offset bit).
+    auto candidates = [&](auto visit) {
+        for (int t = j0 + tid; t < elements; t += NT) {
+            const int i = row_of(t), j = t - i + 1;
+            if (early && i == j0 && j == n - 1) continue;
+            int before = t - j0;
+            for (int q = 0; q < i >> 5; ++q) before += __popc(par[q]);
+            before += __popc(par[i >> 5] & ((1u << (i & 31)) - 1u));
+            const bool twin = j == J[i] && ((par[i >> 5] >> (i & 31)) & 1u);
+            const bool wrapped = i == j0 && j == n - 1;
+            for (int p = 0; p <= (twin ? 1 : 0); ++p) {
+                const int a = p && wrapped ? wrap(i + 1, n) : i;
+                const int b = wrap(p && !wrapped ? j + 1 : j, n);
+                visit(4 * (before + p) + 0, a, 0);
+                visit(4 * (before + p) + 1, a, 1);
+                visit(4 * (before + p) + 2, b, 0);
+                visit(4 * (before + p) + 3, b, 1);
+            }
+        }
+    };
+    auto area_of = [&](int v, int up) { return area[up ? v : (v == 0 ? n - 1 : v - 1)]; };
+    // Candidate of the smallest area, the first of equal ones.
+    CandMin m{__builtin_inf(), 0x7fffffff, -1};
+    candidates([&](int pos, int v, int up) { cand_min(m, area_of(v, up), pos, 2 * v + up); });
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1)
+        cand_min(m, __shfl_xor(m.area, o, kWave), __shfl_xor(m.pos, o, kWave), __shfl_xor(m.cand, o, kWave));
+    if (NT > kWave) {
+        if (lane_id() == 0) red[tid / kWave] = m;
+        __syncthreads();
+        for (int q = 0; q < NT / kWave; ++q) cand_min(m, red[q].area, red[q].pos, red[q].cand);
+        __syncthreads();
+    }
+    smallest = m.area;
+    if (!(m.area < __builtin_inf())) return -1;
+    // The last later candidate below float(m), and the smallest area before.
+    const double fm = static_cast<double>(static_cast<float>(m.area));
+    CandMin later{__builtin_inf(), -1, -1};
+    double before = __builtin_inf();
+    candidates([&](int pos, int v, int up) {
+        const double a = area_of(v, up);
+        if (pos > m.pos && a < fm && pos > later.pos) {
+            later.pos = pos;
+            later.cand = 2 * v + up;
+        }
+        if (pos < m.pos) before = fmin(before, a);
+    });
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        const int p = __shfl_xor(later.pos, o, kWave), c = __shfl_xor(later.cand, o, kWave);
+        if (p > later.pos) {
+            later.pos = p;
+            later.cand = c;
+        }
+        before = fmin(before, __shfl_xor(before, o, kWave));
+    }
+    later.area = before;
+    if (NT > kWave) {
+        if (lane_id() == 0) red[tid / kWave] = later;
+        __syncthreads();
+        for (int q = 0; q < NT / kWave; ++q) {
+            if (red[q].pos > later.pos) later = CandMin{later.area, red[q].pos, red[q].cand};
+            later.area = fmin(later.area, red[q].area);
+        }
+        __syncthreads();
+    }
+    if (later.pos >= 0) return later.cand;
+    return m.area < static_cast<double>(static_cast<float>(later.area)) ? m.cand : kWalkSerial;
+}
+
+// The same by one lane: the reference's walk and its sequential rule.  False
+// when the walk does not end.
+__device__ bool choose_serial(const double2* V, const double* area, int n, int cap, int& cand, float& best) {
+    best = __builtin_inff();  // float(DBL_MAX)
+    cand = -1;
+    return antipodal_walk(V, n, cap, [&](int i, int j) {
+        for (int q = 0; q < 4; ++q) {
+            const int v = q < 2 ? i : j;
+            const double a = area[(q & 1) ? v : (v == 0 ? n - 1 : v - 1)];
+            if (a < static_cast<double>(best)) {
+                best = static_cast<float>(a);
+                cand = 2 * v + (q & 1);
+            }
+        }
+    });
+}
+
+// Box of the chosen candidate in its own direction, by one whole wavefront
+// (every lane returns the same box).
+__device__ void candidate_box(const double2* V, int n, int cand, double cx, double cy, lp_bounding_box& box) {
+    const int lane = lane_id();
     double ux = 0.0, uy = 0.0;
-    cand_dir(X, Y, n, idx, (sel & 1) ? 1 : -1, ux, uy);
+    cand_dir(V, n, cand >> 1, (cand & 1) ? 1 : -1, ux, uy);
     // Lanes take every 64th vertex; the reduction keeps, among equal values,
     // the one of the lowest vertex index, which is what the sequential
     // std::min / std::max keep (equal values differ at most in the sign of a
@@ -226,8 +386,8 @@ __device__ void choose_box(const double* X, const double* Y, int n, const double
     Extent ex = extent_init();
     int qa = n, qb = n, qc = n, qd = n;
     for (int q = lane; q < n; q += kWave) {
-        const double tx = X[q] - cx;
-        const double ty = Y[q] - cy;
+        const double tx = V[q].x - cx;
+        const double ty = V[q].y - cy;
         const double rx = tx * ux + ty * uy, ry = -tx * uy + ty * ux;
         if (rx < ex.mnx) { ex.mnx = rx; qa = q; }
         if (ex.mxx < rx) { ex.mxx = rx; qb = q; }
@@ -245,7 +405,6 @@ __device__ void choose_box(const double* X, const double* Y, int n, const double
         if (a2 < ex.mny || (a2 == ex.mny && b2 < qc)) { ex.mny = a2; qc = b2; }
         if (ex.mxy < a3 || (a3 == ex.mxy && b3 < qd)) { ex.mxy = a3; qd = b3; }
     }
-    box.area = best;
     box.corners[0] = ex.mnx * ux - ex.mny * uy + cx;
     box.corners[1] = ex.mnx * uy + ex.mny * ux + cy;
     box.corners[2] = ex.mxx * ux - ex.mny * uy + cx;
@@ -268,100 +427,81 @@ __device__ __forceinline__ lp_bounding_box empty_box() {
     return box;
 }
 
-// Polygons of up to one vertex per lane: one wavefront each, four per
-// workgroup (a grid-stride loop over the frame's polygons), the vertices in
-// the wavefront's own LDS slice.  Polygon k of frame f: vertices
-// VX/VY[ob + off[k] .. off[k+1]) with the offsets' end given by `total`.
-// Larger polygons are listed for k_boxes.
-constexpr int kBoxWaves = kBoxThreads / kWave;
+// LDS of one polygon of up to N vertices worked on by W wavefronts.
+template <int N, int W>
+struct BoxLds {
+    double2 V[N];
+    double area[N];  // per edge e (e -> e+1); NaN when too short
+    uint16_t J[N];
+    uint32_t par[N / 32 + 1];
+    CandMin red[W];
+    int cand;
+    float best;
+    int ok;
+};
 
-__global__ __launch_bounds__(kBoxThreads) void k_boxes_wave(DevBuf d, Layout L, const double* VX, const double* VY,
-                                                            const uint32_t* off) {
-    __shared__ double Xs[kBoxWaves][kWave];
-    __shared__ double Ys[kBoxWaves][kWave];
-    __shared__ double areas[kBoxWaves][kWave];
-    __shared__ int2 pairs_s[kBoxWaves][2 * kWave];
-    int tile, f;
-    xcd_tile_frame(tile, f);
-    const int w = threadIdx.x / kWave;
-    const int lane = lane_id();
-    double* X = Xs[w];
-    double* Y = Ys[w];
-    double* area = areas[w];
-    int2* pairs = pairs_s[w];
-    const uint32_t* fs = d.fs + f * kFsCount;
-    const int K = static_cast<int>(fs[kFsClusters]);
-    const uint32_t total = fs[kFsHullTotal];
-    const size_t ob = (size_t)f * L.N;
-    if (K > L.box_stride) {
-        if (tile == 0 && threadIdx.x == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
-        return;
+// Box of polygon k of frame f, vertices VX/VY[v0 .. v0 + n), 3 <= n <= N, by
+// the group's NT threads.
+template <int NT, int N>
+__device__ __forceinline__ void polygon_box(const DevBuf& d, const Layout& L, int f, int k, const double* VX,
+                                            const double* VY, int n, int tid, BoxLds<N, NT / kWave>& s) {
+    for (int q = tid; q < n; q += NT) s.V[q] = make_double2(VX[q], VY[q]);
+    group_sync<NT>();
+    // Centroid: the vertices summed in order, as the reference does.
+    double cx = 0.0, cy = 0.0;
+#pragma unroll 4
+    for (int q = 0; q < n; ++q) {
+        cx += s.V[q].x;
+        cy += s.V[q].y;
     }
-    for (int k = tile * kBoxWaves + w; k < K; k += gridDim.x * kBoxWaves) {
-        const uint32_t v0 = off[ob + k];
-        const uint32_t v1 = k + 1 < K ? off[ob + k + 1] : total;
-        const int n = static_cast<int>(v1 - v0);
-        if (n > kWave) {
-            if (lane == 0) {
-                const uint32_t q = atomicAdd(&d.fs[f * kFsCount + kFsBoxLarge], 1u);
-                d.box_large[(size_t)f * L.box_stride + q] = k;
-            }
-            continue;
-        }
+    cx /= n;
+    cy /= n;
+    for (int e = tid; e < n; e += NT) s.area[e] = edge_box_area(s.V, n, e, cx, cy);
+    group_sync<NT>();
+    double smallest = 0.0;
+    int cand = choose_candidate<NT>(s.V, s.area, n, 2 * N, tid, s.J, s.par, s.red, smallest);
+    float best = static_cast<float>(smallest);
+    bool ok = true;
+    if (cand == kWalkSerial) {
+        if (tid == 0) s.ok = choose_serial(s.V, s.area, n, 2 * N, s.cand, s.best) ? 1 : 0;
+        group_sync<NT>();
+        cand = s.cand;
+        best = s.best;
+        ok = s.ok != 0;
+    }
+    if (!ok && tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
+    if (tid < kWave) {
         lp_bounding_box box = empty_box();
-        if (n >= 3) {
-            if (lane < n) {
-                X[lane] = VX[ob + v0 + lane];
-                Y[lane] = VY[ob + v0 + lane];
-            }
-            wave_sync();
-            int np = 0;
-            if (lane == 0)
-                np = antipodal_walk(
-                    n, 2 * kWave, [&](int, int q, double& vx, double& vy) { vx = X[q]; vy = Y[q]; },
-                    [&](int c, int a, int b) { pairs[c] = make_int2(a, b); });
-            np = __shfl(np, 0, kWave);
-            wave_sync();
-            // Centroid: the vertices summed in order, as the reference does.
-            double cx = 0.0, cy = 0.0;
-            for (int q = 0; q < n; ++q) {
-                cx += X[q];
-                cy += Y[q];
-            }
-            cx /= n;
-            cy /= n;
-            if (np < 0) {
-                if (lane == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
-            } else {
-                if (lane < n)
-                    area[lane] = edge_box_area(X, Y, n, lane, cx, cy, [&](int q, double& vx, double& vy) {
-                        vx = X[q];
-                        vy = Y[q];
-                    });
-                wave_sync();
-                choose_box(X, Y, n, area, pairs, np, cx, cy, box);
-            }
+        if (ok && cand >= 0) {
+            box.area = best;
+            candidate_box(s.V, n, cand, cx, cy, box);
         }
-        if (lane == 0) {
+        if (tid == 0) {
             d.boxes[(size_t)f * L.box_stride + k] = box;
             if (box.is_valid) atomicAdd(&d.fs[f * kFsCount + kFsBoxes], 1u);
         }
-        wave_sync();
     }
+    group_sync<NT>();
 }
 
-// Polygons of more than one vertex per lane, one workgroup each (up to
-// kBoxVerts vertices; larger: capacity error): workgroup `tile` takes the
-// entries tile, tile + gridDim.x, ... of the frame's list written by
-// k_boxes_wave.
+// One launch for all polygons.  Polygon k of frame f: vertices
+// VX/VY[ob + off[k] .. off[k+1]) with the offsets' end given by `total`.  The
+// first `large_tiles` workgroups of a frame take its polygons of more than 64
+// vertices (up to kBoxVerts; larger: capacity error): each lists them all
+// from the offsets, in order, and takes every large_tiles-th, so the few long
+// polygons start at once and run beside the small ones.  The other workgroups
+// take the small polygons, a wavefront each, in a grid-stride loop.
+constexpr int kBoxWaves = kBoxThreads / kWave;
+
 __global__ __launch_bounds__(kBoxThreads) void k_boxes(DevBuf d, Layout L, const double* VX, const double* VY,
-                                                      const uint32_t* off) {
-    __shared__ double X[kBoxVerts];
-    __shared__ double Y[kBoxVerts];
-    __shared__ double area[kBoxVerts];  // per edge e (e -> e+1); NaN when too short
-    __shared__ int2 pairs[2 * kBoxVerts];
-    __shared__ int np_s;
-    __shared__ double cen_s[2];
+                                                       const uint32_t* off, int large_tiles) {
+    union Lds {
+        BoxLds<kBoxVerts, kBoxWaves> large;
+        BoxLds<kWave, 1> small[kBoxWaves];
+        __device__ Lds() {}
+    };
+    __shared__ Lds lds;
+    __shared__ int row_cnt[kBoxWaves];
     int tile, f;
     xcd_tile_frame(tile, f);
     const int tid = threadIdx.x;
@@ -370,62 +510,72 @@ __global__ __launch_bounds__(kBoxThreads) void k_boxes(DevBuf d, Layout L, const
     const uint32_t* fs = d.fs + f * kFsCount;
     const int K = static_cast<int>(fs[kFsClusters]);
     const uint32_t total = fs[kFsHullTotal];
-    const int m = static_cast<int>(fs[kFsBoxLarge]);
     const size_t ob = (size_t)f * L.N;
-    if (K > L.box_stride) return;  // flagged by k_boxes_wave
-    for (int j = tile; j < m; j += gridDim.x) {
-        const int k = d.box_large[(size_t)f * L.box_stride + j];
-        const uint32_t v0 = off[ob + k];
-        const uint32_t v1 = k + 1 < K ? off[ob + k + 1] : total;
-        const int n = static_cast<int>(v1 - v0);
-        lp_bounding_box box = empty_box();
-        if (n > kBoxVerts) {
-            if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
-        } else {
-            for (int q = tid; q < n; q += kBoxThreads) {
-                X[q] = VX[ob + v0 + q];
-                Y[q] = VY[ob + v0 + q];
+    if (K > L.box_stride) {
+        if (tile == 0 && tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
+        return;
+    }
+    auto range = [&](int k, uint32_t& v0) {
+        v0 = off[ob + k];
+        return static_cast<int>((k + 1 < K ? off[ob + k + 1] : total) - v0);
+    };
+    if (tile >= large_tiles) {
+        const int tiles = static_cast<int>(gridDim.x) - large_tiles;
+        for (int k = (tile - large_tiles) * kBoxWaves + w; k < K; k += tiles * kBoxWaves) {
+            uint32_t v0;
+            const int n = range(k, v0);
+            if (n > kWave) continue;
+            if (n < 3) {
+                if (lane == 0) d.boxes[(size_t)f * L.box_stride + k] = empty_box();
+                continue;
             }
-            __syncthreads();
-            // The first wavefront walks the antipodal pairs while the
-            // others sum the centroid (each on its own, in the
-            // reference's order) and evaluate the edge areas.
-            if (w == 0) {
-                if (lane == 0)
-                    np_s = antipodal_walk(
-                        n, 2 * kBoxVerts, [&](int, int q, double& x, double& y) { x = X[q]; y = Y[q]; },
-                        [&](int c, int a, int b) { pairs[c] = make_int2(a, b); });
-            } else {
-                double cx = 0.0, cy = 0.0;
-                for (int q = 0; q < n; ++q) {
-                    cx += X[q];
-                    cy += Y[q];
-                }
-                cx /= n;
-                cy /= n;
-                if (tid == kWave) {
-                    cen_s[0] = cx;
-                    cen_s[1] = cy;
-                }
-                for (int e = tid - kWave; e < n; e += kBoxThreads - kWave)
-                    area[e] = edge_box_area(X, Y, n, e, cx, cy, [&](int q, double& vx, double& vy) {
-                        vx = X[q];
-                        vy = Y[q];
-                    });
-            }
-            __syncthreads();
-            const int np = np_s;
-            if (np < 0) {
-                if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
-            } else if (w == 0) {
-                choose_box(X, Y, n, area, pairs, np, cen_s[0], cen_s[1], box);
-            }
+            polygon_box<kWave, kWave>(d, L, f, k, VX + ob + v0, VY + ob + v0, n, lane, lds.small[w]);
         }
-        if (tid == 0) {
-            d.boxes[(size_t)f * L.box_stride + k] = box;
-            if (box.is_valid) atomicAdd(&d.fs[f * kFsCount + kFsBoxes], 1u);
-        }
+        return;
+    }
+    int seen = 0;  // large polygons before this row of 256
+    for (int k0 = 0; k0 < K; k0 += kBoxThreads) {
+        uint32_t v0 = 0;
+        const int k = k0 + tid;
+        const int n = k < K ? range(k, v0) : 0;
+        const uint64_t big = __ballot(n > kWave);
+        if (lane == 0) row_cnt[w] = __popcll(big);
         __syncthreads();
+        int before = seen;
+        for (int q = 0; q < w; ++q) before += row_cnt[q];
+        int all = 0;
+        for (int q = 0; q < kBoxWaves; ++q) all += row_cnt[q];
+        before += static_cast<int>(lanes_below(big));
+        // This workgroup's polygons of the row, one after the other: `before`
+        // is the polygon's number among the large ones.
+        const uint64_t mine = __ballot(n > kWave && before % large_tiles == tile);
+        __syncthreads();
+        seen += all;
+        if (all == 0) continue;
+        // Every wavefront goes through every wavefront's polygons.
+        for (int q = 0; q < kBoxWaves; ++q) {
+            if (w == q && lane == 0) {
+                lds.large.par[0] = static_cast<uint32_t>(mine);
+                lds.large.par[1] = static_cast<uint32_t>(mine >> 32);
+            }
+            __syncthreads();
+            uint64_t todo = lds.large.par[0] | (static_cast<uint64_t>(lds.large.par[1]) << 32);
+            __syncthreads();
+            while (todo) {
+                const int kk = k0 + q * kWave + __ffsll(static_cast<unsigned long long>(todo)) - 1;
+                todo &= todo - 1;
+                uint32_t vv;
+                const int nn = range(kk, vv);
+                if (nn > kBoxVerts) {
+                    if (tid == 0) {
+                        atomicOr(&d.fs[f * kFsCount + kFsErr], kErrBoxCapacity);
+                        d.boxes[(size_t)f * L.box_stride + kk] = empty_box();
+                    }
+                    continue;
+                }
+                polygon_box<kBoxThreads, kBoxVerts>(d, L, f, kk, VX + ob + vv, VY + ob + vv, nn, tid, lds.large);
+            }
+        }
     }
 }
 
@@ -727,15 +877,14 @@ void launch_boxes(lp_context* c, int B) {
     hipStream_t st = c->stream;
     const size_t BN = (size_t)L.B * L.N;
     stage_mark(c, "boxes");
-    // Four polygons per workgroup; about 128 wavefronts per frame on large
-    // batches, more for few frames (standalone polygon lists).
-    const int tiles = std::min(1024, std::max(32, 4096 / B));
-    hipLaunchKernelGGL(k_boxes_wave, dim3(tiles, B), dim3(kBoxThreads), 0, st, d, L, d.hcx + BN, d.hcy + BN,
-                       d.hull_off);
-    // Enough workgroups that each takes at most one of a frame's few large
-    // polygons, whose walk is the longest chain of the stage.
-    hipLaunchKernelGGL(k_boxes, dim3(std::min(256, std::max(4, 1024 / B)), B), dim3(kBoxThreads), 0, st, d, L,
-                       d.hcx + BN, d.hcy + BN, d.hull_off);
+    // Four small polygons per workgroup, about 128 wavefronts per frame on
+    // large batches, more for few frames (standalone polygon lists); ahead of
+    // them enough workgroups that each takes at most one of a frame's few
+    // large polygons.
+    const int small_tiles = std::min(1024, std::max(32, 4096 / B));
+    const int large_tiles = std::min(256, std::max(8, 1024 / B));
+    hipLaunchKernelGGL(k_boxes, dim3(large_tiles + small_tiles, B), dim3(kBoxThreads), 0, st, d, L, d.hcx + BN,
+                       d.hcy + BN, d.hull_off, large_tiles);
 }
 
 }  // namespace lp
