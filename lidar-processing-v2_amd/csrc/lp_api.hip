@@ -120,11 +120,215 @@ __global__ void k_deinterleave(const uint8_t* raw, int n, int stride, int ox, in
     }
 }
 
+// Frames one staging launch describes: their descriptors travel as kernel
+// arguments (2.7 KB of the 4 KB a launch may carry).
+constexpr int kStageFrames = 16;
+
+// A frame's points where the gather reads them: n points, `stride` bytes
+// apart; n = 0 when they are copied by other means.
+struct StageCloud {
+    const uint8_t* x;
+    const uint8_t* y;
+    const uint8_t* z;
+    const uint8_t* ring;
+    int32_t stride, ring_stride;
+    int32_t n;
+};
+
+struct StageArgs {
+    FrameDesc fd[kStageFrames];
+    StageCloud cl[kStageFrames];
+    CluConst cc;
+    NoiseConst nc;
+    int32_t first;  // index of fd[0] in the batch
+};
+
+constexpr int kStageRows = 4;  // points per thread, 256 apart
+
+__device__ __forceinline__ float load_f32(const uint8_t* p) {
+    float v;
+    memcpy(&v, p, 4);
+    return v;
+}
+
+__device__ __forceinline__ uint16_t load_u16(const uint8_t* p) {
+    uint16_t v;
+    memcpy(&v, p, 2);
+    return v;
+}
+
+// Stages a batch: descriptors and constants from the arguments, and the
+// points of the clouds that are in this device's memory, whatever their
+// strides.  One launch for up to 16 frames instead of four copies per frame
+// and three for the descriptors (a copy costs 3 to 5 us of host time and a
+// gap on the stream; the points themselves move at memory speed): the pass
+// over 128 frames @STAGE128@, over one @STAGE1@.
+__global__ __launch_bounds__(256) void k_stage(StageArgs a, float* x, float* y, float* z, uint16_t* ring,
+                                               FrameDesc* frames, CluConst* cc, NoiseConst* nc) {
+    const int f = blockIdx.y;
+    if (blockIdx.x == 0) {
+        constexpr int kWords = sizeof(FrameDesc) / 4;
+        static_assert(sizeof(FrameDesc) % 4 == 0 && kWords <= 256, "one thread per descriptor word");
+        if (threadIdx.x < kWords)
+            reinterpret_cast<uint32_t*>(frames + a.first + f)[threadIdx.x] =
+                reinterpret_cast<const uint32_t*>(&a.fd[f])[threadIdx.x];
+        if (f == 0 && threadIdx.x == 0) {
+            *cc = a.cc;
+            *nc = a.nc;
+        }
+    }
+    const StageCloud& c = a.cl[f];
+    const int off = a.fd[f].pt_off;
+    const int base = blockIdx.x * (256 * kStageRows) + threadIdx.x;
+    float vx[kStageRows], vy[kStageRows], vz[kStageRows];
+    uint16_t vr[kStageRows];
+#pragma unroll
+    for (int k = 0; k < kStageRows; ++k) {
+        const int i = base + k * 256;
+        if (i >= c.n) continue;
+        const size_t o = static_cast<size_t>(i) * c.stride;
+        vx[k] = load_f32(c.x + o);
+        vy[k] = load_f32(c.y + o);
+        vz[k] = load_f32(c.z + o);
+        if (c.ring) vr[k] = load_u16(c.ring + static_cast<size_t>(i) * c.ring_stride);
+    }
+#pragma unroll
+    for (int k = 0; k < kStageRows; ++k) {
+        const int i = base + k * 256;
+        if (i >= c.n) continue;
+        x[off + i] = vx[k];
+        y[off + i] = vy[k];
+        z[off + i] = vz[k];
+        if (c.ring) ring[off + i] = vr[k];
+    }
+}
+
+// One array on its way to the host: `elem` bytes times a count, which is
+// fs[frame][slot] (at most `count`) or `count` itself (slot < 0).  The unknown
+// cloud (kUnknownCloud) follows the ground cloud in memory and holds what the
+// ground and obstacle points leave of that count.
+struct OutItem {
+    const uint8_t* src;
+    uint8_t* dst;   // where the kernel writes: the caller's page-locked memory or the bounce buffer
+    uint32_t elem;
+    int32_t count;
+    int32_t frame;
+    int16_t slot;
+    int16_t rules;  // OutRule bits
+    int32_t hull_capacity;
+};
+enum OutRule : int16_t {
+    kSkipFailed = 1,    // nothing when the frame failed
+    kSkipHullOver = 2,  // nothing when the frame has more than hull_capacity hull vertices
+    kUnknownCloud = 4
+};
+constexpr int kOutItems = 64;  // items of one launch (2.6 KB of arguments)
+struct OutArgs {
+    OutItem item[kOutItems];
+};
+
+// Bytes of an item, by the frame's scalars (the same on host and device).
+__host__ __device__ inline uint32_t out_bytes(const OutItem& it, const uint32_t* fs) {
+    const uint32_t* s = fs + static_cast<size_t>(it.frame) * kFsCount;
+    if ((it.rules & kSkipFailed) && (s[kFsErr] | s[kFsNoiseErr]) != 0) return 0;
+    const int32_t hull = static_cast<int32_t>(s[kFsHullTotal]);
+    if ((it.rules & kSkipHullOver) && hull > 0 && hull > it.hull_capacity) return 0;
+    const uint32_t cap = static_cast<uint32_t>(it.count);
+    uint32_t n = it.slot < 0 ? cap : (s[it.slot] < cap ? s[it.slot] : cap);
+    if (it.rules & kUnknownCloud) {
+        const uint32_t known = s[kFsGround] + s[kFsObstacles];
+        n = known < n ? n - known : 0u;
+    }
+    return n * it.elem;
+}
+
+__host__ __device__ inline const uint8_t* out_src(const OutItem& it, const uint32_t* fs) {
+    const uint32_t skipped = it.rules & kUnknownCloud ? fs[static_cast<size_t>(it.frame) * kFsCount + kFsGround] : 0u;
+    return it.src + static_cast<size_t>(skipped) * it.elem;
+}
+
+// Writes the outputs of a run straight into host memory: one launch for up to
+// 64 arrays, whose sizes it reads on the device, so the host waits once
+// instead of once for the counts and once more for a copy per array.  Link
+// bound: @FETCH@.
+__global__ __launch_bounds__(256) void k_copy_out(OutArgs a, const uint32_t* fs) {
+    const OutItem& it = a.item[blockIdx.y];
+    const uint32_t bytes = out_bytes(it, fs);
+    const uint8_t* src = out_src(it, fs);
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x;
+    const uint32_t step = gridDim.x * blockDim.x;
+    const uintptr_t mix = reinterpret_cast<uintptr_t>(src) | reinterpret_cast<uintptr_t>(it.dst);
+    uint32_t done = 0;
+    if ((mix & 15) == 0) {
+        const uint32_t n = bytes / 16;
+        for (uint32_t i = t; i < n; i += step)
+            reinterpret_cast<uint4*>(it.dst)[i] = reinterpret_cast<const uint4*>(src)[i];
+        done = n * 16;
+    } else if ((mix & 3) == 0) {
+        const uint32_t n = bytes / 4;
+        for (uint32_t i = t; i < n; i += step)
+            reinterpret_cast<uint32_t*>(it.dst)[i] = reinterpret_cast<const uint32_t*>(src)[i];
+        done = n * 4;
+    }
+    for (uint32_t i = done + t; i < bytes; i += step) it.dst[i] = src[i];
+}
+
 }  // namespace lp
 
 using namespace lp;
 
 namespace {
+
+// Kind of the memory around a pointer of the caller, and whether a kernel of
+// this device may touch all of [p, p + bytes).  Allocations seen are kept for
+// one call only (a batch's arrays mostly share a few allocations).
+class CallerMemory {
+   public:
+    enum Kind { kDevice, kPinned, kPageable, kOther };
+
+    explicit CallerMemory(int device) : device_(device) {}
+
+    // *dev receives the address to use on the device (kDevice, kPinned).
+    Kind find(const void* p, size_t bytes, uint8_t** dev) {
+        const uintptr_t a = reinterpret_cast<uintptr_t>(p);
+        for (const Range& r : ranges_)
+            if (a >= r.lo && a + bytes <= r.hi) {
+                *dev = reinterpret_cast<uint8_t*>(a + r.delta);
+                return r.kind;
+            }
+        hipPointerAttribute_t at{};
+        if (hipPointerGetAttributes(&at, p) != hipSuccess) {
+            (void)hipGetLastError();
+            return kPageable;  // not known to the runtime
+        }
+        if (at.type == hipMemoryTypeUnregistered) return kPageable;
+        if ((at.type != hipMemoryTypeDevice && at.type != hipMemoryTypeHost) || at.device != device_ ||
+            !at.devicePointer)
+            return kOther;
+        hipDeviceptr_t base = nullptr;
+        size_t size = 0;
+        if (hipMemGetAddressRange(&base, &size, reinterpret_cast<hipDeviceptr_t>(at.devicePointer)) != hipSuccess) {
+            (void)hipGetLastError();
+            return kOther;
+        }
+        const uintptr_t d = reinterpret_cast<uintptr_t>(at.devicePointer);
+        const uintptr_t b = reinterpret_cast<uintptr_t>(base);
+        if (d < b || d + bytes > b + size) return kOther;
+        const Kind kind = at.type == hipMemoryTypeDevice ? kDevice : kPinned;
+        ranges_.insert(ranges_.begin(), Range{a - (d - b), a - (d - b) + size, d - a, kind});
+        if (ranges_.size() > 16) ranges_.pop_back();
+        *dev = reinterpret_cast<uint8_t*>(d);
+        return kind;
+    }
+
+   private:
+    struct Range {
+        uintptr_t lo, hi, delta;
+        Kind kind;
+    };
+    int device_;
+    std::vector<Range> ranges_;
+};
 
 template <typename T>
 T* carve(char*& p, size_t count) {
@@ -302,16 +506,23 @@ int validate_frame(const lp_context* c, const lp_segmenter_config& cfg, const lp
 
 namespace {
 
-// Copies a cloud into the packed inputs (x, y, z, ring at offset `off`), or
-// into the noise filter's raw inputs when `raw_inputs`.
-int stage_cloud(lp_context* c, const lp_cloud& cl, int32_t off, uint8_t* raw_dev, bool raw_inputs = false) {
-    DevBuf d = c->d;
-    if (raw_inputs) {
-        d.x = d.rx;
-        d.y = d.ry;
-        d.z = d.rz;
-        d.ring = d.rring;
-    }
+// Whether k_stage may read the cloud where it is: device memory of this
+// device, every field inside its allocation.
+bool gathers(CallerMemory& mem, const lp_cloud& cl, StageCloud& g) {
+    if (!cl.on_device || cl.num_points == 0 || cl.xyz_stride < 4 || (cl.ring && cl.ring_stride < 2)) return false;
+    const size_t last = static_cast<size_t>(cl.num_points) - 1;
+    uint8_t *x, *y, *z, *r = nullptr;
+    const size_t span = last * static_cast<size_t>(cl.xyz_stride) + 4;
+    if (mem.find(cl.x, span, &x) != CallerMemory::kDevice || mem.find(cl.y, span, &y) != CallerMemory::kDevice ||
+        mem.find(cl.z, span, &z) != CallerMemory::kDevice ||
+        (cl.ring && mem.find(cl.ring, last * static_cast<size_t>(cl.ring_stride) + 2, &r) != CallerMemory::kDevice))
+        return false;
+    g = StageCloud{x, y, z, r, cl.xyz_stride, cl.ring_stride, cl.num_points};
+    return true;
+}
+
+// Copies a cloud into the packed inputs (x, y, z, ring at offset `off`) of d.
+int stage_cloud(lp_context* c, const DevBuf& d, const lp_cloud& cl, int32_t off, uint8_t* raw_dev) {
     const int n = cl.num_points;
     if (n == 0) return LP_OK;
     const hipMemcpyKind kind = cl.on_device ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
@@ -342,6 +553,54 @@ int stage_cloud(lp_context* c, const lp_cloud& cl, int32_t off, uint8_t* raw_dev
                            a.fx, a.fy, a.fz, a.fr, d.x + o, d.y + o, d.z + o, d.ring + o);
         LP_HIP(hipGetLastError());
     }
+    return LP_OK;
+}
+
+// Stages the clouds of c->frames (descriptors ready, constants given) into
+// the packed inputs, or into the noise filter's raw inputs when `raw_inputs`.
+// Clouds in host memory, or in memory a kernel may not read, are copied (AoS
+// records through a device area, free at this point of the pipeline).
+int stage_frames(lp_context* c, const lp_cloud* clouds, const CluConst& cc, const NoiseConst& nc, bool raw_inputs) {
+    DevBuf d = c->d;
+    if (raw_inputs) {
+        d.x = d.rx;
+        d.y = d.ry;
+        d.z = d.rz;
+        d.ring = d.rring;
+    }
+    uint8_t* raw = reinterpret_cast<uint8_t*>(c->d.slot_w);
+    CallerMemory mem(c->device);
+    const int B = static_cast<int>(c->frames.size());
+    for (int f0 = 0; f0 < B; f0 += kStageFrames) {
+        StageArgs a{};
+        a.cc = cc;
+        a.nc = nc;
+        a.first = f0;
+        const int cnt = std::min(kStageFrames, B - f0);
+        int most = 0;
+        for (int k = 0; k < cnt; ++k) {
+            const lp_cloud& cl = clouds[f0 + k];
+            a.fd[k] = c->frames[f0 + k];
+            std::string why;
+            AosLayout layout;
+            const bool soa = cl.xyz_stride == 4 && (cl.ring == nullptr || cl.ring_stride == 2);
+            if (cl.num_points > 0 && !soa) {
+                if (!aos_layout(cl, layout, why)) return fail(LP_ERR_INVALID_ARGUMENT, why);
+                if (raw_staging_bytes(c) < static_cast<size_t>(layout.stride))
+                    return fail(LP_ERR_CAPACITY, "point record larger than the staging area");
+            }
+            if (gathers(mem, cl, a.cl[k])) {
+                most = std::max(most, cl.num_points);
+                continue;
+            }
+            const int st = stage_cloud(c, d, cl, c->frames[f0 + k].pt_off, raw);
+            if (st != LP_OK) return st;
+        }
+        const int tiles = std::max(1, (most + 256 * kStageRows - 1) / (256 * kStageRows));
+        hipLaunchKernelGGL(k_stage, dim3(tiles, cnt), dim3(256), 0, c->stream, a, d.x, d.y, d.z, d.ring, d.frames, d.cc,
+                           d.nc);
+    }
+    LP_HIP(hipGetLastError());
     return LP_OK;
 }
 
@@ -527,7 +786,8 @@ int create_lane(const lp_capacity* cap, lp_context** out) {
     layout_bytes(L, &c->d, static_cast<char*>(c->arena));
     launch_mt19937(c->d.mt_raw, kMtRawCount, c->stream);
     launch_hash_init(c);
-    e = hipStreamSynchronize(c->stream);
+    e = hipMemsetAsync(c->d.fs, 0, L.B * kFsCount * sizeof(uint32_t), c->stream);
+    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         lp_context_destroy(c);
         return fail(LP_ERR_HIP, std::string("context init: ") + hipGetErrorString(e));
@@ -588,21 +848,12 @@ int stage_batch(lp_context* c, const lp_segmenter_config* seg_cfgs, int32_t num_
         fd.has_ring = cl.ring != nullptr ? 1 : 0;
         off += cl.num_points;
     }
-    // Inputs: SoA copies straight in; AoS records through a device staging
-    // area (the slot-weight arrays are free at this point of the pipeline).
-    // With the noise filter on they land in its raw inputs and the filter
-    // writes the kept points where the segmenter reads them.
-    uint8_t* raw = reinterpret_cast<uint8_t*>(c->d.slot_w);
-    for (int f = 0; f < num_frames; ++f) {
-        const int st = stage_cloud(c, clouds[f], c->frames[f].pt_off, raw, filter);
-        if (st != LP_OK) return st;
-    }
+    // With the noise filter on the points land in its raw inputs and the
+    // filter writes the kept ones where the segmenter reads them.
     derive_clu(*ccfg, c->cap.max_voxels, c->cc);
-    if (filter) LP_HIP(hipMemcpyAsync(c->d.nc, &c->nc, sizeof(NoiseConst), hipMemcpyHostToDevice, c->stream));
+    const int st = stage_frames(c, clouds, c->cc, c->nc, filter);
+    if (st != LP_OK) return st;
     c->staged_filtered = filter;
-    LP_HIP(hipMemcpyAsync(c->d.frames, c->frames.data(), sizeof(FrameDesc) * num_frames, hipMemcpyHostToDevice,
-                          c->stream));
-    LP_HIP(hipMemcpyAsync(c->d.cc, &c->cc, sizeof(CluConst), hipMemcpyHostToDevice, c->stream));
     c->num_frames = num_frames;
     c->staged_points = off;
     return LP_OK;
@@ -707,20 +958,155 @@ int lp_query(lp_context* c) {
 
 namespace {
 
-int fetch_lane(lp_context* c, const lp_frame_outputs* outputs, lp_frame_result* results) {
+// Host memory a context keeps for outputs that go to pageable memory: at
+// most this much, beyond it such arrays are copied one by one.
+constexpr size_t kBounceMax = size_t{64} << 20;
+
+// The arrays one call returns, and where each goes.  add() them, launch()
+// the copies behind the run, finish() waits and hands the pageable ones over.
+class Outputs {
+   public:
+    explicit Outputs(lp_context* c) : c_(c), mem_(c->device) {}
+
+    // `count` elements of `elem` bytes at src (fewer if fs[frame][slot] says so).
+    void add(void* user, const void* src, size_t elem, int count, int frame = 0, int slot = -1, int rules = 0,
+             int hull_capacity = 0) {
+        if (!user || count <= 0) return;
+        Entry e{};
+        e.it = OutItem{static_cast<const uint8_t*>(src), nullptr, static_cast<uint32_t>(elem), count, frame,
+                       static_cast<int16_t>(slot), static_cast<int16_t>(rules), hull_capacity};
+        e.user = user;
+        const size_t bytes = elem * static_cast<size_t>(count);
+        e.kind = mem_.find(user, bytes, &e.it.dst);
+        if (e.kind == CallerMemory::kDevice) e.kind = CallerMemory::kOther;
+        if (e.kind == CallerMemory::kPageable) {
+            e.bounce = (need_ + 255) & ~size_t{255};
+            if (e.bounce + bytes > kBounceMax)
+                e.kind = CallerMemory::kOther;
+            else
+                need_ = e.bounce + bytes;
+        }
+        entries_.push_back(e);
+    }
+
+    // Queues the copies and the scalars of `frames` frames.
+    int launch(int frames) {
+        const size_t scalars = (static_cast<size_t>(c_->L.B) * kFsCount * 4 + 255) & ~size_t{255};
+        const size_t want = scalars + need_;
+        if (want > c_->pinned_bytes) {
+            if (c_->pinned) (void)hipHostFree(c_->pinned);
+            c_->pinned = nullptr;
+            c_->pinned_bytes = 0;
+            LP_HIP(hipHostMalloc(&c_->pinned, want, hipHostMallocDefault));
+            c_->pinned_bytes = want;
+        }
+        bounce_ = static_cast<uint8_t*>(c_->pinned) + scalars;
+        OutArgs a{};
+        a.item[0] = OutItem{reinterpret_cast<const uint8_t*>(c_->d.fs), static_cast<uint8_t*>(c_->pinned), 4,
+                            frames * kFsCount, 0, -1, 0, 0};
+        int k = 1;
+        size_t most = 0;
+        auto flush = [&] {
+            // 16 bytes a thread, at most 64 workgroups an item: a few
+            // hundred KB in flight fill the host link.
+            const int tiles = static_cast<int>(std::min<size_t>(64, std::max<size_t>(1, (most + 4095) / 4096)));
+            hipLaunchKernelGGL(k_copy_out, dim3(tiles, k), dim3(256), 0, c_->stream, a, c_->d.fs);
+            k = 0;
+            most = 0;
+        };
+        for (Entry& e : entries_) {
+            if (e.kind == CallerMemory::kOther) continue;
+            if (e.kind == CallerMemory::kPageable) e.it.dst = bounce_ + e.bounce;
+            if (k == kOutItems) flush();
+            a.item[k++] = e.it;
+            most = std::max(most, static_cast<size_t>(e.it.elem) * e.it.count);
+        }
+        if (k) flush();
+        LP_HIP(hipGetLastError());
+        return LP_OK;
+    }
+
+    // The scalars, valid after finish().
+    const uint32_t* scalars() const { return static_cast<const uint32_t*>(c_->pinned); }
+
+    int finish() {
+        LP_HIP(hipStreamSynchronize(c_->stream));
+        bool more = false;
+        for (const Entry& e : entries_) {
+            const uint32_t bytes = e.kind == CallerMemory::kPinned ? 0 : out_bytes(e.it, scalars());
+            if (!bytes) continue;
+            if (e.kind == CallerMemory::kPageable) {
+                std::memcpy(e.user, bounce_ + e.bounce, bytes);
+            } else {
+                LP_HIP(hipMemcpyAsync(e.user, out_src(e.it, scalars()), bytes, hipMemcpyDeviceToHost, c_->stream));
+                more = true;
+            }
+        }
+        if (more) LP_HIP(hipStreamSynchronize(c_->stream));
+        return LP_OK;
+    }
+
+   private:
+    struct Entry {
+        OutItem it;
+        void* user;
+        size_t bounce;
+        CallerMemory::Kind kind;
+    };
+    lp_context* c_;
+    CallerMemory mem_;
+    std::vector<Entry> entries_;
+    size_t need_ = 0;
+    uint8_t* bounce_ = nullptr;
+};
+
+// Queues the outputs of a lane's frames behind its run.
+int queue_fetch(lp_context* c, const lp_frame_outputs* outputs, Outputs& out) {
     LP_HIP(hipSetDevice(c->device));
     const int B = c->num_frames;
     const Layout& L = c->L;
-    std::vector<uint32_t> fs(static_cast<size_t>(B) * kFsCount);
-    LP_HIP(hipMemcpyAsync(fs.data(), c->d.fs, fs.size() * 4, hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
+    const bool boxes = c->boxes_on || c->vehicles_on;
+    for (int f = 0; f < B && outputs; ++f) {
+        const FrameDesc& fd = c->frames[f];
+        const lp_frame_outputs& o = outputs[f];
+        const size_t ob = static_cast<size_t>(f) * L.N;
+        const size_t kb = static_cast<size_t>(f) * L.box_stride;
+        const int n = fd.n;
+        // Points the segmenter saw: the noise filter's kept count when it ran.
+        const int points = c->staged_filtered ? kFsKept : -1;
+        // A cluster has at least min_size of them.
+        const int k = n / std::max(1, static_cast<int>(std::min(c->cc.min_size, 1u << 30)));
+        if (c->staged_filtered) out.add(o.noise_labels, c->d.noise + ob, 1, fd.n_raw, f);
+        out.add(o.seg_labels, c->d.labels + fd.pt_off, 4, n, f, points);
+        out.add(o.obstacle_index, c->d.obs_src + ob, 4, n, f, kFsObstacles, kSkipFailed);
+        out.add(o.cluster_labels, c->d.clabel + ob, 4, n, f, kFsObstacles, kSkipFailed);
+        out.add(o.hull_offsets, c->d.hull_off + ob, 4, k, f, kFsClusters, kSkipFailed);
+        const int hc = o.hull_capacity;
+        const int rules = kSkipFailed | (o.hull_indices ? kSkipHullOver : 0);
+        out.add(o.hull_indices, c->d.hull_local + ob, 4, std::min(n, hc), f, kFsHullTotal, rules, hc);
+        if (boxes) out.add(o.boxes, c->d.boxes + kb, sizeof(lp_bounding_box), std::min(k, L.box_stride), f, kFsClusters,
+                           rules, hc);
+        if (c->vehicles_on) out.add(o.vehicle_class, c->d.vclass + kb, 4, std::min(k, L.box_stride), f, kFsClusters,
+                                    rules, hc);
+        if (c->clouds_on) {
+            out.add(o.ground_index, c->d.split_idx + ob, 4, n, f, kFsGround, rules, hc);
+            out.add(o.unknown_index, c->d.split_idx + ob, 4, n, f, points, rules | kUnknownCloud, hc);
+        }
+    }
+    return out.launch(B);
+}
+
+// Waits for a lane's outputs and reports its frames.
+int finish_fetch(lp_context* c, const lp_frame_outputs* outputs, lp_frame_result* results, Outputs& out) {
+    LP_HIP(hipSetDevice(c->device));
+    const int st = out.finish();
+    if (st != LP_OK) return st;
     int overall = LP_OK;
-    for (int f = 0; f < B; ++f) {
-        const uint32_t* s = fs.data() + static_cast<size_t>(f) * kFsCount;
+    for (int f = 0; f < c->num_frames; ++f) {
+        const uint32_t* s = out.scalars() + static_cast<size_t>(f) * kFsCount;
         const FrameDesc& fd = c->frames[f];
         lp_frame_result r{};
         r.status = status_of(s[kFsErr] | s[kFsNoiseErr]);
-        // Points the segmenter saw: the noise filter's kept count when it ran.
         const int n = c->staged_filtered ? static_cast<int>(s[kFsKept]) : fd.n;
         r.num_points = n;
         r.num_noise = c->staged_filtered ? static_cast<int32_t>(s[kFsNoise]) : 0;
@@ -750,45 +1136,14 @@ int fetch_lane(lp_context* c, const lp_frame_outputs* outputs, lp_frame_result* 
         std::memcpy(r.ransac.plane, pl, sizeof(pl));
         if (results) results[f] = r;
         if (r.status != LP_OK && overall == LP_OK) overall = r.status;
-        if (!outputs) continue;
+        if (!outputs || r.status != LP_OK) continue;
         const lp_frame_outputs& o = outputs[f];
-        const size_t ob = static_cast<size_t>(f) * L.N;
-        if (c->staged_filtered && o.noise_labels && fd.n_raw)
-            LP_HIP(hipMemcpyAsync(o.noise_labels, c->d.noise + ob, fd.n_raw, hipMemcpyDeviceToHost, c->stream));
-        if (o.seg_labels && n)
-            LP_HIP(hipMemcpyAsync(o.seg_labels, c->d.labels + fd.pt_off, n * 4, hipMemcpyDeviceToHost, c->stream));
-        if (r.status != LP_OK) continue;
-        const int no = r.num_obstacles, K = r.num_clusters, V = r.num_hull_vertices;
-        if (o.obstacle_index && no)
-            LP_HIP(hipMemcpyAsync(o.obstacle_index, c->d.obs_src + ob, no * 4, hipMemcpyDeviceToHost, c->stream));
-        if (o.cluster_labels && no)
-            LP_HIP(hipMemcpyAsync(o.cluster_labels, c->d.clabel + ob, no * 4, hipMemcpyDeviceToHost, c->stream));
-        if (o.hull_offsets) {
-            if (K) LP_HIP(hipMemcpyAsync(o.hull_offsets, c->d.hull_off + ob, K * 4, hipMemcpyDeviceToHost, c->stream));
-            o.hull_offsets[K] = V;
+        if (o.hull_offsets) o.hull_offsets[r.num_clusters] = r.num_hull_vertices;
+        if (o.hull_indices && r.num_hull_vertices > 0 && r.num_hull_vertices > o.hull_capacity) {
+            if (results) results[f].status = fail(LP_ERR_CAPACITY, "hull_capacity too small");
+            overall = LP_ERR_CAPACITY;
         }
-        if (o.hull_indices && V) {
-            if (V > o.hull_capacity) {
-                if (results) results[f].status = fail(LP_ERR_CAPACITY, "hull_capacity too small");
-                overall = LP_ERR_CAPACITY;
-                continue;
-            }
-            LP_HIP(hipMemcpyAsync(o.hull_indices, c->d.hull_local + ob, V * 4, hipMemcpyDeviceToHost, c->stream));
-        }
-        if (boxes && o.boxes && K)
-            LP_HIP(hipMemcpyAsync(o.boxes, c->d.boxes + static_cast<size_t>(f) * L.box_stride,
-                                  K * sizeof(lp_bounding_box), hipMemcpyDeviceToHost, c->stream));
-        if (c->vehicles_on && o.vehicle_class && K)
-            LP_HIP(hipMemcpyAsync(o.vehicle_class, c->d.vclass + static_cast<size_t>(f) * L.box_stride,
-                                  K * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-        if (c->clouds_on && o.ground_index && r.num_ground)
-            LP_HIP(hipMemcpyAsync(o.ground_index, c->d.split_idx + ob, r.num_ground * 4, hipMemcpyDeviceToHost,
-                                  c->stream));
-        if (c->clouds_on && o.unknown_index && r.num_unknown)
-            LP_HIP(hipMemcpyAsync(o.unknown_index, c->d.split_idx + ob + r.num_ground, r.num_unknown * 4,
-                                  hipMemcpyDeviceToHost, c->stream));
     }
-    LP_HIP(hipStreamSynchronize(c->stream));
     return overall;
 }
 
@@ -796,16 +1151,42 @@ int fetch_lane(lp_context* c, const lp_frame_outputs* outputs, lp_frame_result* 
 
 int lp_batch_fetch(lp_context* c, const lp_frame_outputs* outputs, lp_frame_result* results) {
     if (!c || c->num_frames < 1) return fail(LP_ERR_INVALID_ARGUMENT, "nothing staged");
-    if (c->lanes.empty()) return fetch_lane(c, outputs, results);
-    int overall = LP_OK, off = 0;
-    for (size_t k = 0; k < c->lane_frames.size(); ++k) {
-        const int cnt = c->lane_frames[k];
-        if (cnt == 0) continue;
-        lp_context* lane = k == 0 ? c : c->lanes[k - 1];
-        const int st = fetch_lane(lane, outputs ? outputs + off : nullptr, results ? results + off : nullptr);
-        if (st != LP_OK && overall == LP_OK) overall = st;
-        off += cnt;
+    if (c->lanes.empty()) {
+        Outputs out(c);
+        const int st = queue_fetch(c, outputs, out);
+        return st != LP_OK ? st : finish_fetch(c, outputs, results, out);
     }
+    // Every lane's copies are queued before the first is waited for, so a
+    // lane that is done sends its outputs while the others still run.
+    std::vector<Outputs> outs;
+    outs.reserve(c->lane_frames.size());
+    int overall = LP_OK, off = 0;
+    auto each = [&](auto step) {
+        off = 0;
+        for (size_t k = 0; k < c->lane_frames.size(); ++k) {
+            if (c->lane_frames[k] == 0) continue;
+            lp_context* lane = k == 0 ? c : c->lanes[k - 1];
+            const int st = step(lane, outputs ? outputs + off : nullptr, results ? results + off : nullptr);
+            if (st != LP_OK && overall == LP_OK) overall = st;
+            off += c->lane_frames[k];
+        }
+    };
+    each([&](lp_context* lane, const lp_frame_outputs* o, lp_frame_result*) {
+        outs.emplace_back(lane);
+        return queue_fetch(lane, o, outs.back());
+    });
+    if (overall != LP_OK) {
+        // A lane failed to queue: nothing is left writing to the caller's memory.
+        each([&](lp_context* lane, const lp_frame_outputs*, lp_frame_result*) -> int {
+            LP_HIP(hipStreamSynchronize(lane->stream));
+            return LP_OK;
+        });
+        return overall;
+    }
+    size_t next = 0;
+    each([&](lp_context* lane, const lp_frame_outputs* o, lp_frame_result* r) {
+        return finish_fetch(lane, o, r, outs[next++]);
+    });
     return overall;
 }
 
@@ -829,11 +1210,12 @@ int lp_segment(lp_context* c, const lp_segmenter_config* cfg, const lp_cloud* cl
     if (st != LP_OK) return st;
     st = run_pipeline(c, 1, true);
     if (st != LP_OK) return st;
-    uint32_t fs[kFsCount];
-    LP_HIP(hipMemcpyAsync(fs, c->d.fs, sizeof(fs), hipMemcpyDeviceToHost, c->stream));
-    if (cloud->num_points)
-        LP_HIP(hipMemcpyAsync(labels, c->d.labels, cloud->num_points * 4, hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
+    Outputs out(c);
+    out.add(labels, c->d.labels, 4, cloud->num_points);
+    st = out.launch(1);
+    if (st == LP_OK) st = out.finish();
+    if (st != LP_OK) return st;
+    const uint32_t* fs = out.scalars();
     st = status_of(fs[kFsErr] & ~(kErrVoxelOverflow | kErrHullCapacity));
     if (ransac) {
         ransac->candidates = fs[kFsCands];
@@ -864,23 +1246,21 @@ int lp_cluster(lp_context* c, const lp_clusterer_config* cfg, const lp_cloud* cl
     c->frames.assign(1, fd);
     lp_cloud xyz = *cloud;
     xyz.ring = nullptr;
-    int st = stage_cloud(c, xyz, 0, reinterpret_cast<uint8_t*>(c->d.slot_w));
-    if (st != LP_OK) return st;
     derive_clu(*cfg, c->cap.max_voxels, c->cc);
-    LP_HIP(hipMemcpyAsync(c->d.frames, c->frames.data(), sizeof(FrameDesc), hipMemcpyHostToDevice, c->stream));
-    LP_HIP(hipMemcpyAsync(c->d.cc, &c->cc, sizeof(CluConst), hipMemcpyHostToDevice, c->stream));
+    int st = stage_frames(c, &xyz, c->cc, c->nc, false);
+    if (st != LP_OK) return st;
     c->num_frames = 1;
     c->L.B_active = 1;
     launch_clear(c, 1);
     launch_cluster(c, 1, false);
     LP_HIP(hipGetLastError());
-    uint32_t fs[kFsCount];
-    LP_HIP(hipMemcpyAsync(fs, c->d.fs, sizeof(fs), hipMemcpyDeviceToHost, c->stream));
-    if (cloud->num_points)
-        LP_HIP(hipMemcpyAsync(labels, c->d.clabel, cloud->num_points * 4, hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
+    Outputs out(c);
+    out.add(labels, c->d.clabel, 4, cloud->num_points);
+    st = out.launch(1);
+    if (st == LP_OK) st = out.finish();
+    if (st != LP_OK) return st;
     c->num_frames = 0;  // the staged frame is not a full-pipeline batch
-    return status_of(fs[kFsErr]);
+    return status_of(out.scalars()[kFsErr]);
 }
 
 void lp_noise_config_default(lp_noise_config* cfg) {
@@ -1014,11 +1394,8 @@ int lp_remove_noise(lp_context* c, const lp_noise_config* cfg, const lp_cloud* c
     c->frames.assign(1, fd);
     lp_cloud xyz = *cloud;
     xyz.ring = nullptr;
-    int st = stage_cloud(c, xyz, 0, reinterpret_cast<uint8_t*>(c->d.slot_w), true);
+    int st = stage_frames(c, &xyz, c->cc, noise_const(*cfg), true);
     if (st != LP_OK) return st;
-    const NoiseConst nc = noise_const(*cfg);
-    LP_HIP(hipMemcpyAsync(c->d.frames, c->frames.data(), sizeof(FrameDesc), hipMemcpyHostToDevice, c->stream));
-    LP_HIP(hipMemcpyAsync(c->d.nc, &nc, sizeof(NoiseConst), hipMemcpyHostToDevice, c->stream));
     c->num_frames = 0;
     c->L.B_active = 1;
     if (c->noise_kdtree) {
@@ -1027,15 +1404,12 @@ int lp_remove_noise(lp_context* c, const lp_noise_config* cfg, const lp_cloud* c
         launch_noise(c, 1, false);
     }
     LP_HIP(hipGetLastError());
-    LP_HIP(hipMemcpyAsync(labels, c->d.noise, cloud->num_points, hipMemcpyDeviceToHost, c->stream));
-    uint32_t err = 0;
-    LP_HIP(hipMemcpyAsync(&err, c->d.fs + kFsNoiseErr, sizeof(err), hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
-    if (c->noise_kdtree) {
-        const int st2 = status_of(err);
-        if (st2 != LP_OK) return st2;
-    }
-    return LP_OK;
+    Outputs out(c);
+    out.add(labels, c->d.noise, 1, cloud->num_points);
+    st = out.launch(1);
+    if (st == LP_OK) st = out.finish();
+    if (st != LP_OK) return st;
+    return c->noise_kdtree ? status_of(out.scalars()[kFsNoiseErr]) : LP_OK;
 }
 
 namespace {
@@ -1068,11 +1442,12 @@ int polygon_boxes(lp_context* c, const double* x, const double* y, const int32_t
     c->L.B_active = 1;
     launch(c, num_polygons);
     LP_HIP(hipGetLastError());
-    LP_HIP(hipMemcpyAsync(fs.data(), c->d.fs, kFsCount * 4, hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipMemcpyAsync(boxes, c->d.boxes, num_polygons * sizeof(lp_bounding_box), hipMemcpyDeviceToHost,
-                          c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
-    if (fs[kFsErr] & kErrBoxCapacity) return fail(LP_ERR_CAPACITY, "a polygon exceeds the box kernel's capacity");
+    Outputs out(c);
+    out.add(boxes, c->d.boxes, sizeof(lp_bounding_box), num_polygons);
+    int st = out.launch(1);
+    if (st == LP_OK) st = out.finish();
+    if (st != LP_OK) return st;
+    if (out.scalars()[kFsErr] & kErrBoxCapacity) return fail(LP_ERR_CAPACITY, "a polygon exceeds the box kernel's capacity");
     return LP_OK;
 }
 
@@ -1132,16 +1507,17 @@ int lp_convex_hulls(lp_context* c, const double* x, const double* y, const int32
     }
     launch_hull_lists(c, num_lists, total);
     LP_HIP(hipGetLastError());
-    uint32_t fs[kFsCount];
-    LP_HIP(hipMemcpyAsync(fs, c->d.fs, sizeof(fs), hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
+    Outputs out(c);
+    out.add(hull_offsets, c->d.hull_off, sizeof(int32_t), num_lists);
+    out.add(hull_indices, c->d.hull_local, sizeof(int32_t), std::min(c->L.N, hull_capacity), 0, kFsHullTotal,
+            kSkipHullOver, hull_capacity);
+    int st = out.launch(1);
+    if (st == LP_OK) st = out.finish();
+    if (st != LP_OK) return st;
+    const uint32_t* fs = out.scalars();
     const int32_t V = static_cast<int32_t>(fs[kFsHullTotal]);
     if (fs[kFsErr] & kErrHullCapacity) return fail(LP_ERR_CAPACITY, "hull candidates exceed the device capacity");
     if (V > hull_capacity || (V > 0 && !hull_indices)) return fail(LP_ERR_CAPACITY, "hull_capacity too small");
-    LP_HIP(hipMemcpyAsync(hull_offsets, c->d.hull_off, num_lists * sizeof(int32_t), hipMemcpyDeviceToHost,
-                          c->stream));
-    if (V) LP_HIP(hipMemcpyAsync(hull_indices, c->d.hull_local, V * sizeof(int32_t), hipMemcpyDeviceToHost, c->stream));
-    LP_HIP(hipStreamSynchronize(c->stream));
     hull_offsets[num_lists] = V;
     c->num_frames = 0;
     return LP_OK;

@@ -305,7 +305,8 @@ struct lp_context {
     void* clouds_mem = nullptr;     // gnd_flag + split_idx
     uint8_t* image_dev = nullptr;   // one frame's label image (allocated on first use)
     bool staged_filtered = false;   // the staged batch went through the noise filter
-    // pinned host buffers for inputs / outputs
+    // page-locked host memory: the frames' scalars, then outputs on their way
+    // to pageable memory (grown on use)
     void* pinned = nullptr;
     size_t pinned_bytes = 0;
     // One captured graph per (batch size, optional-stage switches): every
