@@ -213,10 +213,12 @@ __global__ void k_jcp_slots(DevBuf d, Layout L) {
             // slot was inside the image.
             const int rlo = max(0, -dr), rhi = min(H, H - dr);
             const int clo = max(0, -dc), chi = min(W, W - dc);
-            int khi = j - 1;
+            // None in an image too small for the slot: rows rlo .. rhi - 1
+            // exist below.
+            int khi = rlo < rhi ? j - 1 : -1, klo = 0;
             // First queue index at or after a row's first pixel: qrow.
-            if (rhi < H) khi = min(khi, qrow[rhi] - 1);
-            const int klo = rlo > 0 ? qrow[rlo] : 0;
+            if (rlo < rhi && rhi < H) khi = min(khi, qrow[rhi] - 1);
+            if (rlo < rhi && rlo > 0) klo = qrow[rlo];
             int k = khi;
             for (; k >= klo; --k) {
                 const int qc = ql[k] % W;
