@@ -19,6 +19,7 @@ constexpr int kRansacIters = 60;      // segmenter.cpp:324
 constexpr int kRansacRadialBins = 4;  // segmenter.cpp:323
 constexpr int kMtRawCount = 4096;     // precomputed mt19937{42} outputs
 constexpr int kSmallCell = 512;       // cells up to this size are sorted by one wave
+constexpr int kSlotRecordBytes = 128;  // JCP slots of a queue pixel
 constexpr int kBigCell = 8192;        // larger cells: one workgroup; beyond: capacity error
 constexpr int kHullChunk = 256;       // points per chunk-hull wave
 constexpr int kHullFinal = 8192;      // candidates a final hull workgroup can hold
@@ -155,9 +156,7 @@ struct DevBuf {
     // JCP queue (frame stride pix_stride)
     int32_t* qlist;
     int32_t* qrow;           // [frame][H + 1] first queue index of each row
-    float* slot_w;           // [q][24]
-    int32_t* slot_src;       // [q][24]
-    uint8_t* qsum_ok;
+    uint4* slot_rec;         // [q] slot records of kSlotRecordBytes; before the run: staging area of AoS records
     uint8_t* fin;
     // voxel hash (frame stride hash_cap)
     HashSlot* hslot;

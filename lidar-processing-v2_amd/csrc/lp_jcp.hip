@@ -15,12 +15,14 @@
 //   * all of them lie in earlier image rows, except the two same-row
 //     neighbours (0,-1) and (0,-2) -- a stale slot's writer and the writer's
 //     neighbour are always in earlier rows or static;
-//   * so rows are solved in order, and inside a row the state of pixel j is
-//     T_j(state(j-2), state(j-1)) over 3 states {ground, obstacle, pending}:
-//     an associative scan of 9-entry transfer maps solves the row at once.
+//   * so rows are solved in order, and inside a row a pixel's label is a
+//     function of the labels of the two queue pixels before it: an
+//     associative scan of these maps solves the row at once.
 // The weights w_i = u_i / sum do not depend on labels and are precomputed
-// for all queue pixels in parallel (k_jcp_slots); the per-row solve only
-// re-runs the ordered float sums that the reference performs.
+// for all queue pixels in parallel (k_jcp_slots).  A label is the sign of
+// (obstacle weights - ground weights); the row solve forms that difference
+// once and only where it is within rounding of zero evaluates the reference's
+// ordered float sums.
 #include "lp_kernels.h"
 #include "lp_queue.h"
 
@@ -37,9 +39,6 @@ __constant__ static const int8_t kOffC[24] = {-2, -1, 0, 1, 2, -2, -1, 0, 1, 2, 
 constexpr int32_t kSrcUnknown = -1;
 constexpr int32_t kSrcGround = -2;
 constexpr int32_t kSrcObstacle = -3;
-
-// Internal solve states.
-constexpr uint32_t kSG = 0, kSO = 1, kSU = 2;
 
 // Queue membership: a ground pixel with an obstacle pixel in its clipped 5x5
 // window (cv::dilate of the red channel, then the raster scan of
@@ -80,9 +79,10 @@ __global__ __launch_bounds__(T) void k_jcp_mark(DevBuf d, Layout L) {
 // The queue in raster order, from the flags in two passes over tiles of 2048
 // pixels (eight rows of 256, coalesced): the queue count of every tile, then
 // each tile's compaction after the counts of the tiles before it.  qlist[j]
-// is the pixel of queue entry j, qmap[p] the queue index of pixel p (-1 when
-// not queued), qrow[r] the first queue index at or after row r's first pixel
-// (kept for the row solve); the last tile writes the queue length.
+// is the pixel of queue entry j, qmap[p] the queue index of pixel p or, for a
+// pixel that is not queued, its static label source (negative), qrow[r] the
+// first queue index at or after row r's first pixel (kept for the row solve);
+// the last tile writes the queue length.
 constexpr int kQueueThreads = 256;
 constexpr int kQueueRows = 8;
 constexpr int kQueueTile = kQueueThreads * kQueueRows;
@@ -141,12 +141,41 @@ __global__ __launch_bounds__(kQueueThreads) void k_jcp_fill(DevBuf d, Layout L) 
             d.qlist[po + j] = p;
             d.qmap[po + p] = j;
         } else {
-            d.qmap[po + p] = -1;
+            const uint8_t st = d.state[fd.pix_off + p];
+            d.qmap[po + p] = st == kGround ? kSrcGround : (st == kObstacle ? kSrcObstacle : kSrcUnknown);
         }
     }
     if (threadIdx.x == 0 && base + kQueueTile >= P) d.fs[f * kFsCount + kFsQueue] = pre_total + total;
 }
 
+
+// A queue pixel's slots, as the row solve reads them: the head slots 0..11
+// (rows -2, -1 and the two left neighbours) with their weights and label
+// entries, and the tail slots 12..23 (right neighbours, rows +1, +2).  A tail
+// slot names a neighbour raster-after its writer (the pixel itself or, stale,
+// an earlier queue pixel), so its label is static or pending and its weight is
+// stored with a sign: + obstacle, - ground, 0 neither.
+// A record is eight 16-byte parts, part k of queue pixel j at [k * P + j] of
+// the frame's records, so neighbouring lanes read neighbouring addresses:
+//   0..2  head weights 0..11 (float)
+//   3     head entries 0..7, 16 bits each (low half; see kLabelBase)
+//   4     head entries 8..11, the sum of the tail (float), flags
+//   5..7  tail weights 12..23 (float)
+// flags: bits 0..11 bit 16 of the entries; bits kRecScale.. log2 of the
+// weights' sum, rounded up; kRecTail, kRecOk.  The solve's fast path reads
+// parts 0 to 4.
+constexpr int kRecordParts = 8;
+static_assert(kRecordParts * 16 == kSlotRecordBytes, "slot records fill their array");
+constexpr int kRecScale = 12;
+constexpr uint32_t kRecTail = 1u << 30;  // some tail weight is not zero
+constexpr uint32_t kRecOk = 1u << 31;    // the weight sum passes the reference's test
+
+// Label entries: 0, 1, 2 are the static sources kSrcObstacle, kSrcGround and
+// kSrcUnknown, queue pixel j is entry j + kLabelBase.  A label is +1 for an
+// obstacle, -1 for ground and 0 for neither.
+constexpr int kLabelBase = 3;
+static_assert(kSrcObstacle + kLabelBase == 0 && kSrcGround + kLabelBase == 1 && kSrcUnknown + kLabelBase == 2,
+              "static sources are the first three label entries");
 
 struct SlotVal {
     float u;
@@ -155,12 +184,10 @@ struct SlotVal {
 };
 
 // Slot value computed by evaluator pixel `pe` (core point `core`) for its
-// neighbour pixel np (segmenter.cpp:558-606).
-__device__ __forceinline__ SlotVal eval_slot(const DevBuf& d, size_t po, size_t qo, const SegConst& s, int pe,
-                                             float4 core, int np) {
+// neighbour pixel np with record nb and source qm (segmenter.cpp:558-606).
+__device__ __forceinline__ SlotVal eval_slot(const SegConst& s, int pe, float4 core, int np, float4 nb, int qm) {
     SlotVal v{0.0f, kSrcUnknown, false};
-    const float4 nb = d.pxyz[po + np];  // w holds the pixel's winner, -1 when empty
-    if (__float_as_int(nb.w) == -1) return v;
+    if (__float_as_int(nb.w) == -1) return v;  // w holds the pixel's winner, -1 when empty
     const float dx = core.x - nb.x;
     const float dy = core.y - nb.y;
     const float dz = core.z - nb.z;
@@ -168,19 +195,17 @@ __device__ __forceinline__ SlotVal eval_slot(const DevBuf& d, size_t po, size_t 
     if (d2 > s.kthr2) return v;
     v.u = glibc_expf(s.neg_amp * sqrtf(d2));
     v.near = true;
-    const int qm = d.qmap[qo + np];
-    if (qm >= 0) {
-        v.src = (np < pe) ? qm : kSrcUnknown;  // later queue pixels are still pending
-    } else {
-        const uint8_t st = d.state[po + np];
-        v.src = st == kGround ? kSrcGround : (st == kObstacle ? kSrcObstacle : kSrcUnknown);
-    }
+    v.src = (qm >= 0 && np >= pe) ? kSrcUnknown : qm;  // later queue pixels are still pending
     return v;
 }
 
 // Per queue pixel: the 24 slot weights w_i = u_i / sum and label sources,
-// including stale slots resolved through their writer.
-__global__ void k_jcp_slots(DevBuf d, Layout L) {
+// including stale slots resolved through their writer.  Bound by the latency
+// of the neighbour reads, so all 24 records and sources of a pixel are
+// requested before the first is used (clamped into the image; a slot outside
+// it is stale and read again through its writer): 35 -> 22 us for one 64x2048
+// frame, 65 -> 49 us for 32.
+__global__ __launch_bounds__(256) void k_jcp_slots(DevBuf d, Layout L) {
     int tile, f;
     xcd_tile_frame(tile, f);
     const FrameDesc& fd = d.frames[f];
@@ -189,13 +214,22 @@ __global__ void k_jcp_slots(DevBuf d, Layout L) {
     const int j = tile * blockDim.x + threadIdx.x;
     if (j >= nq) return;
     const int H = s.H, W = s.W;
-    const size_t po = fd.pix_off;
+    const float4* px = d.pxyz + fd.pix_off;
     const size_t qo = (size_t)f * L.P;
+    const int32_t* qm = d.qmap + qo;
     const int32_t* ql = d.qlist + qo;
     const int32_t* qrow = d.qrow + (size_t)f * (L.H + 1);
     const int p = ql[j];
     const int r = p / W, c = p % W;
-    const float4 core = d.pxyz[po + p];
+    const float4 core = px[p];
+    float4 nb[24];
+    int32_t nq_src[24];
+#pragma unroll
+    for (int i = 0; i < 24; ++i) {
+        const int np = min(max(r + kOffR[i], 0), H - 1) * W + min(max(c + kOffC[i], 0), W - 1);
+        nb[i] = px[np];
+        nq_src[i] = qm[np];
+    }
     float u[24];
     int32_t src[24];
     float sum = 0.0f;
@@ -204,7 +238,7 @@ __global__ void k_jcp_slots(DevBuf d, Layout L) {
         const int dr = kOffR[i], dc = kOffC[i];
         const int nr = r + dr, nc = c + dc;
         if (nr >= 0 && nr < H && nc >= 0 && nc < W) {
-            const SlotVal v = eval_slot(d, po, qo, s, p, core, nr * W + nc);
+            const SlotVal v = eval_slot(s, p, core, nr * W + nc, nb[i], nq_src[i]);
             u[i] = v.u;
             src[i] = v.src;
             if (v.near) sum += v.u;
@@ -219,15 +253,14 @@ __global__ void k_jcp_slots(DevBuf d, Layout L) {
             // First queue index at or after a row's first pixel: qrow.
             if (rlo < rhi && rhi < H) khi = min(khi, qrow[rhi] - 1);
             if (rlo < rhi && rlo > 0) klo = qrow[rlo];
-            int k = khi;
-            for (; k >= klo; --k) {
-                const int qc = ql[k] % W;
-                if (qc >= clo && qc < chi) break;
+            int q = -1;
+            for (int k = khi; k >= klo && q < 0; --k) {
+                const int pk = ql[k], qc = pk % W;
+                if (qc >= clo && qc < chi) q = pk;
             }
-            if (k >= klo) {
-                const int q = ql[k];
-                const int qr = q / W, qc = q % W;
-                const SlotVal v = eval_slot(d, po, qo, s, q, d.pxyz[po + q], (qr + dr) * W + (qc + dc));
+            if (q >= 0) {
+                const int np = (q / W + dr) * W + q % W + dc;
+                const SlotVal v = eval_slot(s, q, px[q], np, px[np], qm[np]);
                 u[i] = v.u;
                 src[i] = v.src;
             } else {
@@ -237,294 +270,316 @@ __global__ void k_jcp_slots(DevBuf d, Layout L) {
         }
     }
     const bool ok = fabsf(sum) > 1.1920928955078125e-07f;  // FLT_EPSILON
-    float w[24];
+    // An infinite sum makes every weight 0 or NaN: the reference's comparison
+    // is false then, as it is without any weight.
+    const bool weigh = ok && sum < __builtin_inff();
+    float head[12], tail[12];
+    uint32_t entry[12];
+    uint32_t flags = ok ? kRecOk : 0u;
+    float tail_sum = 0.0f, total = 0.0f;
 #pragma unroll
-    for (int i = 0; i < 24; ++i) w[i] = ok ? u[i] / sum : 0.0f;
-    // Head slots 0..11 (rows -2, -1 and the two left neighbours): sources
-    // and weights as they are.  Tail slots 12..23 (right neighbours and rows
-    // +1, +2) name a neighbour raster-after their writer (the pixel itself
-    // or, stale, an earlier queue pixel), so their source is static or a
-    // pending queue pixel and their addends are known here: the ground
-    // addend (w or +0) and the obstacle addend of each tail slot.
-    float* wo = d.slot_w + ((size_t)f * L.P + j) * 24;
-    int32_t* so = d.slot_src + ((size_t)f * L.P + j) * 24;
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        wo[k] = src[12 + k] == kSrcGround ? w[12 + k] : 0.0f;
-        wo[12 + k] = src[12 + k] == kSrcObstacle ? w[12 + k] : 0.0f;
-        so[k] = src[k];
-        so[12 + k] = __float_as_int(w[k]);
+    for (int i = 0; i < 12; ++i) {
+        const float w = weigh ? u[i] / sum : 0.0f;
+        const uint32_t e = static_cast<uint32_t>((w > 0.0f ? src[i] : kSrcUnknown) + kLabelBase);
+        head[i] = w;
+        entry[i] = e & 0xffffu;
+        flags |= (e >> 16) << i;
+        const float t = weigh ? u[12 + i] / sum : 0.0f;
+        tail[i] = src[12 + i] == kSrcObstacle ? t : (src[12 + i] == kSrcGround ? -t : 0.0f);
+        tail_sum += tail[i];
+        if (tail[i] != 0.0f) flags |= kRecTail;
+        total += w + t;
     }
-    d.qsum_ok[(size_t)f * L.P + j] = ok ? 1 : 0;
+    // The pixel's own weights sum to 1; stale ones come on top, divided by a
+    // sum they are not part of.
+    if (total > 1.5f) flags |= min(((__float_as_uint(total) >> 23) & 0xffu) - 126u, 140u) << kRecScale;
+    uint4* rec = d.slot_rec + qo * kRecordParts + j;
+    const size_t P = static_cast<size_t>(L.P);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        rec[k * P] = make_uint4(__float_as_uint(head[4 * k]), __float_as_uint(head[4 * k + 1]),
+                                __float_as_uint(head[4 * k + 2]), __float_as_uint(head[4 * k + 3]));
+        rec[(5 + k) * P] = make_uint4(__float_as_uint(tail[4 * k]), __float_as_uint(tail[4 * k + 1]),
+                                      __float_as_uint(tail[4 * k + 2]), __float_as_uint(tail[4 * k + 3]));
+    }
+    rec[3 * P] = make_uint4(entry[0] | entry[1] << 16, entry[2] | entry[3] << 16, entry[4] | entry[5] << 16,
+                            entry[6] | entry[7] << 16);
+    rec[4 * P] = make_uint4(entry[8] | entry[9] << 16, entry[10] | entry[11] << 16, __float_as_uint(tail_sum), flags);
 }
 
-// Transfer map over the nine pair states ps = a*3 + b: entry ps (0..8) is
-// byte ps of (lo, hi, x), i.e. entries 0-3, 4-7 and 8 (the upper bytes of x
-// are don't-care values in 0..8).
-struct TMap {
-    uint32_t lo, hi, x;
+constexpr int kSolveThreads = 512;
+constexpr int kSolveWaves = kSolveThreads / kWave;
+constexpr int kQueueMax = 65536;  // labels of one frame's queue in LDS
+constexpr int kSolveRows = 1024;  // image rows
+constexpr int kSolveAhead = 4;    // chunks whose records are in registers
+constexpr int kSolveChunks = kSolveRows + kQueueMax / kSolveThreads;  // at most: one per row, and per full chunk
+
+// A difference of weight sums further than this from zero, times the power of
+// two at or above the weights' sum (1 without stale weights), has the sign of
+// the reference's: its two ordered float sums and the difference formed here
+// are each within some 24 * 2^-24 of that sum (4.3e-6 in all).
+constexpr float kSumMargin = 1.0e-5f;
+
+// Parts 0..4 of a record, and the flags of one of the two records before the
+// wavefront's (lane 0 the last, lane 1 the one before).
+struct SlotData {
+    uint4 part[5];
+    uint32_t before;
 };
-constexpr uint32_t kIdLo = 0x03020100u, kIdHi = 0x07060504u, kIdX = 0x08u;
 
-// Entries f[sel_k] for the four selector bytes sel_k (each 0..8) of sel:
-// the byte permute takes entries 0..7 from (hi:lo), and the bytes whose
-// selector is 8 (bit 3 set) are replaced by entry 8 (f8, in every byte).
-// The byte mask is a permute too: selector 12 gives 0x00 and 13 gives 0xff.
-__device__ __forceinline__ uint32_t tmap_pick(const TMap& f, uint32_t f8, uint32_t sel) {
-    const uint32_t v = __builtin_amdgcn_perm(f.hi, f.lo, sel);
-    const uint32_t m = __builtin_amdgcn_perm(0u, 0u, ((sel >> 3) & 0x01010101u) | 0x0c0c0c0cu);
-    return (f8 & m) | (v & ~m);
+// Records of the chunk [first, end), first <= nq.  Lanes past its end read its
+// last record: a wavefront without a pixel reads one line a load.
+__device__ __forceinline__ void load_slots(const uint4* rec, size_t P, int first, int end, SlotData& sd) {
+    const int last = max(end - 1, 0);
+    // 32-bit byte offsets from each part's (uniform) base.
+    const uint32_t o = static_cast<uint32_t>(min(first + static_cast<int>(threadIdx.x), last)) * 16u;
+#pragma unroll
+    for (int k = 0; k < 5; ++k)
+        sd.part[k] = *reinterpret_cast<const uint4*>(reinterpret_cast<const char*>(rec + k * P) + o);
+    const int wave_first = first + (static_cast<int>(threadIdx.x) & ~(kWave - 1));
+    const uint32_t b = static_cast<uint32_t>(min(max(wave_first - 1 - (lane_id() & 1), 0), last)) * 16u;
+    sd.before = *reinterpret_cast<const uint32_t*>(reinterpret_cast<const char*>(rec + 4 * P) + 12 + b);
 }
 
-// f after g.
-__device__ __forceinline__ TMap tmap_compose(const TMap& f, const TMap& g) {
-    const uint32_t f8 = __builtin_amdgcn_perm(0u, f.x, 0u);
-    return TMap{tmap_pick(f, f8, g.lo), tmap_pick(f, f8, g.hi), tmap_pick(f, f8, g.x)};
-}
+// Transfer map of a queue pixel: the pair state 2 * (label of j - 2 is
+// obstacle) + (label of j - 1 is obstacle) to the next one, byte k the image
+// of state k.  Composing f after g is one byte permute.  A pixel left pending
+// counts as ground here; the pixels after it do not weigh it.
+constexpr uint32_t kMapIdentity = 0x03020100u;
+constexpr uint32_t kMapShift = 0x02000200u;  // state k with its older label dropped and a ground appended
 
-__device__ __forceinline__ uint32_t tmap_get(const TMap& m, uint32_t ps) {
-    const uint32_t w = ps < 4 ? m.lo : (ps < 8 ? m.hi : m.x);
-    return (w >> (8 * (ps & 3))) & 0xffu;
-}
+__device__ __forceinline__ uint32_t map_compose(uint32_t f, uint32_t g) { return __builtin_amdgcn_perm(f, f, g); }
 
-// The map of the lane `kCtrl` names (DPP row shift or row broadcast); lanes
-// outside kRowMask or without a source lane read the identity.
 template <int kCtrl, int kRowMask>
-__device__ __forceinline__ TMap tmap_dpp(const TMap& m) {
-    return TMap{static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(kIdLo), static_cast<int>(m.lo),
-                                                                  kCtrl, kRowMask, 0xf, false)),
-                static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(kIdHi), static_cast<int>(m.hi),
-                                                                  kCtrl, kRowMask, 0xf, false)),
-                static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(kIdX), static_cast<int>(m.x),
-                                                                  kCtrl, kRowMask, 0xf, false))};
-}
-
-// Lane `src` (wavefront-uniform) of a map.
-__device__ __forceinline__ TMap tmap_readlane(const TMap& m, int src) {
-    return TMap{static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m.lo), src)),
-                static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m.hi), src)),
-                static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(m.x), src))};
+__device__ __forceinline__ uint32_t map_dpp(uint32_t m) {
+    return static_cast<uint32_t>(__builtin_amdgcn_update_dpp(static_cast<int>(kMapIdentity), static_cast<int>(m), kCtrl,
+                                                             kRowMask, 0xf, false));
 }
 
 // Inclusive scan of the wavefront's maps, m := m_lane o ... o m_0: row
 // shifts by 1, 2, 4 and 8 inside each 16-lane row, then lane 15 of rows 0 / 2
 // into rows 1 / 3 and lane 31 into rows 2 and 3.
-__device__ __forceinline__ TMap tmap_wave_scan(TMap m) {
-    m = tmap_compose(m, tmap_dpp<0x111, 0xf>(m));
-    m = tmap_compose(m, tmap_dpp<0x112, 0xf>(m));
-    m = tmap_compose(m, tmap_dpp<0x114, 0xf>(m));
-    m = tmap_compose(m, tmap_dpp<0x118, 0xf>(m));
-    m = tmap_compose(m, tmap_dpp<0x142, 0xa>(m));
-    m = tmap_compose(m, tmap_dpp<0x143, 0xc>(m));
+__device__ __forceinline__ uint32_t map_wave_scan(uint32_t m) {
+    m = map_compose(m, map_dpp<0x111, 0xf>(m));
+    m = map_compose(m, map_dpp<0x112, 0xf>(m));
+    m = map_compose(m, map_dpp<0x114, 0xf>(m));
+    m = map_compose(m, map_dpp<0x118, 0xf>(m));
+    m = map_compose(m, map_dpp<0x142, 0xa>(m));
+    m = map_compose(m, map_dpp<0x143, 0xc>(m));
     return m;
 }
-constexpr int kSolveThreads = 512;
-constexpr int kSolveWaves = kSolveThreads / kWave;
-constexpr int kFinLds = 65536;
-// LDS label table of the solve: entries 0, 1, 2 are the static labels of
-// sources kSrcObstacle, kSrcGround, kSrcUnknown; queue pixel j is entry j + 3.
-constexpr int kFinBase = 3;
-static_assert(kSrcObstacle + kFinBase == 0 && kSrcGround + kFinBase == 1 && kSrcUnknown + kFinBase == 2,
-              "static sources map to the first three label entries");
 
-// Slot data of one queue pixel, as written by k_jcp_slots: w holds the
-// tail slots' ground addends (entries 0..11) and obstacle addends (12..23),
-// s the head slots' sources (0..11) and weight bit patterns (12..23), ok the
-// sum test.  None of it depends on solved labels, so the solve loads the next
-// chunk's while it solves the current one.
-struct SlotData {
-    float4 w[6];
-    int4 s[6];
-    uint32_t ok;
+// Value of the lane below (lane 0 reads `first`).
+__device__ __forceinline__ uint32_t lane_below(uint32_t v, uint32_t first) {
+    return static_cast<uint32_t>(
+        __builtin_amdgcn_update_dpp(static_cast<int>(first), static_cast<int>(v), 0x138, 0xf, 0xf, false));
+}
+
+// Row-ordered exact solve, one workgroup per frame.  A chunk is up to 512
+// queue pixels of one row; all labels of earlier chunks are final in LDS.
+// Each pixel sums its known slots (at most twelve label reads); open are at
+// most the two queue pixels before it, with weights a1 and a2, so its label as
+// a function of theirs is four signs, and the row is a scan of four-byte maps.
+// Signs within rounding of zero are taken from the reference's ordered sums.
+// The kernel is a chain of rows, bound by latency: each chunk is an LDS read,
+// some 120 instructions and two barriers, and the records are read
+// kSolveAhead - 1 chunks ahead, more than the time of a memory access.  140 ->
+// 63 us for a 64x2048 frame of 16 000 queue pixels (154 -> 68 us for 32): a
+// chunk took nine-entry maps built from nine pairs of ordered sums before.
+// Label entries beyond 16 bits occur in queues of more than 65533 pixels only
+// (kWide): their upper bit costs every slot two instructions.
+struct SolveLds {
+    int8_t lab[kLabelBase + kQueueMax];
+    int chunk_base[kSolveChunks + 2 + kSolveAhead];
+    uint32_t wtot[kSolveWaves];
+    int scan[kSolveWaves + 1];
 };
 
-__device__ __forceinline__ void load_slots(const DevBuf& d, size_t qo, int j, SlotData& sd) {
-    const float4* w4 = reinterpret_cast<const float4*>(d.slot_w + (qo + j) * 24);
-    const int4* s4 = reinterpret_cast<const int4*>(d.slot_src + (qo + j) * 24);
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        sd.w[q] = w4[q];
-        sd.s[q] = s4[q];
-    }
-    sd.ok = d.qsum_ok[qo + j];
-}
-
-// Byte vectors over the nine pair states ps = a*3 + b, laid out like a TMap
-// (bytes 0-3 of lo, 4-7 of hi, byte 0 of x): 3a, 3b and b.
-constexpr uint32_t kA3Lo = 0x03000000u, kA3Hi = 0x06060303u, kA3X = 0x06u;
-constexpr uint32_t kB3Lo = 0x00060300u, kB3Hi = 0x03000603u, kB3X = 0x06u;
-constexpr uint32_t kB1Lo = 0x00020100u, kB1Hi = 0x01000201u, kB1X = 0x02u;
-
-__device__ __forceinline__ uint32_t obstacle_wins(float o, float g) { return o > g ? kSO : kSG; }
-
-// Transfer map of queue pixel j (pair state (state(j-2), state(j-1)) ->
-// (state(j-1), state(j))).  Labels of earlier rows come from `fin`.
-__device__ __forceinline__ TMap pixel_map(const SlotData& sd, int j, int rs, const uint8_t* fin) {
-    float tw[24], hw[12];
-    int32_t hs[12];
-#pragma unroll
-    for (int q = 0; q < 6; ++q) {
-        tw[4 * q] = sd.w[q].x;
-        tw[4 * q + 1] = sd.w[q].y;
-        tw[4 * q + 2] = sd.w[q].z;
-        tw[4 * q + 3] = sd.w[q].w;
-    }
-#pragma unroll
-    for (int q = 0; q < 3; ++q) {
-        hs[4 * q] = sd.s[q].x;
-        hs[4 * q + 1] = sd.s[q].y;
-        hs[4 * q + 2] = sd.s[q].z;
-        hs[4 * q + 3] = sd.s[q].w;
-        hw[4 * q] = __int_as_float(sd.s[q + 3].x);
-        hw[4 * q + 1] = __int_as_float(sd.s[q + 3].y);
-        hw[4 * q + 2] = __int_as_float(sd.s[q + 3].z);
-        hw[4 * q + 3] = __int_as_float(sd.s[q + 3].w);
-    }
-    // Ordered sums of segmenter.cpp:613-626 (wg += w for a GROUND slot, wo +=
-    // w for an OBSTACLE slot), written as selects of w or +0: every weight
-    // is +0 or positive and the sums start at +0, so adding +0 leaves a sum
-    // bit-identical.  Slots 0..9 (rows -2, -1) name
-    // static labels or queue pixels of earlier rows, all final in `fin`
-    // (which holds the three static labels below the queue states, entry
-    // sv + kFinBase).
-    float wg0 = 0.0f, wo0 = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 10; ++i) {
-        const uint32_t l = fin[hs[i] + kFinBase];
-        wg0 += l == kSG ? hw[i] : 0.0f;
-        wo0 += l == kSO ? hw[i] : 0.0f;
-    }
-    // Slots (0,-2), (0,-1) (10, 11): a source in this row is the queue pixel
-    // before (j-1) or two before (j-2) and comes from the pair state; other
-    // sources are static or earlier rows (a stale slot at column 0 or 1 can
-    // name the last queue pixels of the previous row).
-    const int32_t s10 = hs[10], s11 = hs[11];
-    const uint32_t lab10 = s10 < rs ? fin[s10 + kFinBase] : kSU;
-    const uint32_t lab11 = s11 < rs ? fin[s11 + kFinBase] : kSU;
-    const int sel10 = s10 < rs ? 0 : (s10 == j - 2 ? 1 : (s10 == j - 1 ? 2 : 0));  // 1: j-2, 2: j-1
-    const bool sel11 = s11 >= rs && s11 == j - 1;
-    // Each sum with slot 10 / slot 11 counted or not (q bit 0 / bit 1): the
-    // ground sum only sees which of them are GROUND and the obstacle sum which
-    // are OBSTACLE, so four values of each cover all nine pair states.
-    float g0 = wg0, g1 = wg0 + hw[10], g2 = wg0 + hw[11];
-    float g3 = g1 + hw[11];
-    float o0 = wo0, o1 = wo0 + hw[10], o2 = wo0 + hw[11];
-    float o3 = o1 + hw[11];
-    // The tail (slots 12..23) in slot order, its addends precomputed.
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        const float a = tw[k];
-        g0 += a;
-        g1 += a;
-        g2 += a;
-        g3 += a;
-    }
-#pragma unroll
-    for (int k = 0; k < 12; ++k) {
-        const float a = tw[12 + k];
-        o0 += a;
-        o1 += a;
-        o2 += a;
-        o3 += a;
-    }
-    // Decision table over the label pairs (l10, l11), byte l10 * 3 + l11:
-    // ground sum g[(l10 == G) | (l11 == G) << 1] against obstacle sum
-    // o[(l10 == O) | (l11 == O) << 1].  A pixel whose weight sum fails the
-    // test goes to PENDING for every pair state.
-    TMap T{obstacle_wins(o0, g3) | obstacle_wins(o2, g1) << 8 | obstacle_wins(o0, g1) << 16 |
-               obstacle_wins(o1, g2) << 24,
-           obstacle_wins(o3, g0) | obstacle_wins(o1, g0) << 8 | obstacle_wins(o0, g2) << 16 |
-               obstacle_wins(o2, g0) << 24,
-           obstacle_wins(o0, g0)};
-    if (sd.ok == 0) T = TMap{kSU * 0x01010101u, kSU * 0x01010101u, kSU};
-    // Per pair state (a, b): l10 is a, b or static, l11 is b or static; the
-    // entry is (b, t(l10, l11)).
-    const uint32_t r10 = lab10 * 3u * 0x01010101u, r11 = lab11 * 0x01010101u;
-    const uint32_t ilo = (sel10 == 1 ? kA3Lo : (sel10 == 2 ? kB3Lo : r10)) + (sel11 ? kB1Lo : r11);
-    const uint32_t ihi = (sel10 == 1 ? kA3Hi : (sel10 == 2 ? kB3Hi : r10)) + (sel11 ? kB1Hi : r11);
-    const uint32_t ix = (sel10 == 1 ? kA3X : (sel10 == 2 ? kB3X : r10)) + (sel11 ? kB1X : r11);
-    const uint32_t t8 = T.x * 0x01010101u;
-    return TMap{tmap_pick(T, t8, ilo) + kB3Lo, tmap_pick(T, t8, ihi) + kB3Hi, tmap_pick(T, t8, ix) + kB3X};
-}
-
-// Row-ordered exact solve, one workgroup per frame: per row, transfer maps
-// of its queue pixels, a wavefront DPP scan of the maps, one LDS step across
-// the eight wavefronts (two per SIMD, so a row of up to 512 queue pixels is
-// one step and the SIMDs interleave two wavefronts' map evaluation).
-__global__ __launch_bounds__(kSolveThreads) void k_jcp_solve(DevBuf d, Layout L) {
-    __shared__ uint8_t fin[kFinBase + kFinLds];
-    __shared__ int row_start[1025];
-    __shared__ TMap wtot[kSolveWaves];
-    const int f = blockIdx.x;
-    const FrameDesc& fd = d.frames[f];
-    const SegConst& s = fd.sc;
-    const int nq = static_cast<int>(d.fs[f * kFsCount + kFsQueue]);
+template <bool kWide>
+__device__ __forceinline__ void solve_rows(const uint4* rec, size_t P, int nq, int chunks, SolveLds& lds) {
     const int tid = threadIdx.x;
     const int w = tid / kWave;
     const int lane = lane_id();
-    if (nq > kFinLds || s.H > 1024) {
+    int8_t* lab = lds.lab;
+    const int* chunk_base = lds.chunk_base;
+    uint32_t* wtot = lds.wtot;
+    auto chunk = [&](SlotData& sd, int base, int end, int ahead, int ahead_end) {
+        const int j = base + tid;
+        const bool any = base + w * kWave < end;
+        uint32_t m = kMapIdentity;
+        const uint32_t flags = sd.part[4].w;
+        if (any) {
+            float hw[12];
+#pragma unroll
+            for (int k = 0; k < 3; ++k) {
+                hw[4 * k] = __uint_as_float(sd.part[k].x);
+                hw[4 * k + 1] = __uint_as_float(sd.part[k].y);
+                hw[4 * k + 2] = __uint_as_float(sd.part[k].z);
+                hw[4 * k + 3] = __uint_as_float(sd.part[k].w);
+            }
+            const uint32_t ew[6] = {sd.part[3].x, sd.part[3].y, sd.part[3].z, sd.part[3].w, sd.part[4].x, sd.part[4].y};
+            int e[12], l[12];
+#pragma unroll
+            for (int i = 0; i < 12; ++i) e[i] = static_cast<int>((i & 1) ? ew[i / 2] >> 16 : ew[i / 2] & 0xffffu);
+            if (kWide) {
+#pragma unroll
+                for (int i = 0; i < 12; ++i) e[i] |= static_cast<int>(((flags >> i) & 1u) << 16);
+            }
+            // Slots 10 and 11 may name the two queue pixels before this one
+            // in the chunk; a pending one has no label.
+            const int first = base + kLabelBase;
+            const bool in10 = e[10] >= first, in11 = e[11] >= first;
+            const uint32_t ok = flags >> 31;
+            const uint32_t ok1 = lane_below(ok, static_cast<uint32_t>(__builtin_amdgcn_readlane(
+                                                    static_cast<int>(sd.before), 0)) >> 31);
+            const uint32_t ok2 = lane_below(ok1, static_cast<uint32_t>(__builtin_amdgcn_readlane(
+                                                     static_cast<int>(sd.before), 1)) >> 31);
+            const bool one = e[10] == j - 1 + kLabelBase;
+            float a1 = in11 ? hw[11] : 0.0f, a2 = in10 && !one ? hw[10] : 0.0f;
+            if (in10 && one) a1 += hw[10];
+            if (!ok1) a1 = 0.0f;
+            if (!ok2) a2 = 0.0f;
+            if (in10) e[10] = 2;
+            if (in11) e[11] = 2;
+#pragma unroll
+            for (int i = 0; i < 12; ++i) l[i] = lab[e[i]];
+            float d0 = __uint_as_float(sd.part[4].z);
+            int seen = 0;
+#pragma unroll
+            for (int i = 0; i < 12; ++i) {
+                d0 = __builtin_fmaf(hw[i], static_cast<float>(l[i]), d0);
+                seen |= l[i];
+            }
+            // Without any other label the sign of a1, a2 is exact (and 0 is
+            // ground, as in the reference).
+            const bool alone = seen == 0 && !(flags & kRecTail);
+            const float margin =
+                alone ? -1.0f : __uint_as_float(__float_as_uint(kSumMargin) + (((flags >> kRecScale) & 0xffu) << 23));
+            const float p = d0 + a1, q = d0 - a1;
+            const float v0 = q - a2, v1 = p - a2, v2 = q + a2, v3 = p + a2;
+            m = kMapShift | (v0 > 0.0f ? 1u : 0u) | (v1 > 0.0f ? 1u << 8 : 0u) | (v2 > 0.0f ? 1u << 16 : 0u) |
+                (v3 > 0.0f ? 1u << 24 : 0u);
+            const float least = fminf(fminf(fabsf(v0), fabsf(v1)), fminf(fabsf(v2), fabsf(v3)));
+            if (j < end && ok && !(least > margin)) {
+                // The ordered sums of segmenter.cpp:613-626 (wg += w for a
+                // GROUND slot, wo += w for an OBSTACLE slot, as adds of w or
+                // +0: weights are +0 or positive and the sums start at +0, so
+                // adding +0 changes nothing), for each pair of open labels.
+                float tail[12];
+#pragma unroll
+                for (int k = 0; k < 3; ++k) {
+                    const uint4 t = rec[(5 + k) * P + j];
+                    tail[4 * k] = __uint_as_float(t.x);
+                    tail[4 * k + 1] = __uint_as_float(t.y);
+                    tail[4 * k + 2] = __uint_as_float(t.z);
+                    tail[4 * k + 3] = __uint_as_float(t.w);
+                }
+                m = kMapShift;
+                const bool open = a1 > 0.0f || a2 > 0.0f;  // else one pair stands for all
+#pragma nounroll
+                for (int k = 0; k < (open ? 4 : 1); ++k) {
+                    const int s1 = ok1 ? 2 * (k & 1) - 1 : 0, s2 = ok2 ? (k & 2) - 1 : 0;
+                    float g = 0.0f, o = 0.0f;
+#pragma unroll
+                    for (int i = 0; i < 12; ++i) {
+                        int v = l[i];
+                        if (i == 10 && in10) v = one ? s1 : s2;
+                        if (i == 11 && in11) v = s1;
+                        g += v < 0 ? hw[i] : 0.0f;
+                        o += v > 0 ? hw[i] : 0.0f;
+                    }
+#pragma unroll
+                    for (int i = 0; i < 12; ++i) {
+                        g += tail[i] < 0.0f ? -tail[i] : 0.0f;
+                        o += tail[i] > 0.0f ? tail[i] : 0.0f;
+                    }
+                    if (o > g) m |= open ? 1u << (8 * k) : 0x01010101u;
+                }
+            }
+            if (!ok) m = kMapShift;
+            if (j >= end) m = kMapIdentity;
+            m = map_wave_scan(m);
+        }
+        if (lane == kWave - 1) wtot[w] = m;
+        __syncthreads();
+        // State before the wavefront: the totals of the wavefronts before it,
+        // from state 0 (nothing in a chunk hangs on pixels before it).
+        uint32_t t = lane < kSolveWaves ? wtot[lane] : kMapIdentity;
+        load_slots(rec, P, ahead, ahead_end, sd);
+        t = map_compose(t, map_dpp<0x111, 0xf>(t));
+        t = map_compose(t, map_dpp<0x112, 0xf>(t));
+        t = map_compose(t, map_dpp<0x114, 0xf>(t));
+        static_assert(kSolveWaves <= 8, "three row-shift steps scan at most 8 wavefront totals");
+        const uint32_t state = w > 0 ? static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(t), w - 1)) & 3u : 0u;
+        if (j < end) {
+            const uint32_t s = (m >> (8 * state)) & 1u;
+            lab[j + kLabelBase] = static_cast<int8_t>((flags & kRecOk) ? (s ? 1 : -1) : 0);
+        }
+        __syncthreads();
+    };
+    int base[kSolveAhead + 2];
+    SlotData sd[kSolveAhead];
+#pragma unroll
+    for (int k = 0; k <= kSolveAhead + 1; ++k) base[k] = __builtin_amdgcn_readfirstlane(chunk_base[min(k, chunks)]);
+    // Records of the chunk kSolveAhead further replace those just used; the
+    // index is clamped and the order of the loads is kept, so every path has
+    // the same loads in flight and the compiler waits for the oldest only.
+#pragma unroll
+    for (int k = 0; k < kSolveAhead; ++k) {
+        load_slots(rec, P, base[k], base[k + 1], sd[k]);
+        __builtin_amdgcn_sched_barrier(0);
+    }
+    // (The steps are not left early for the same reason: past the last chunk
+    // they have no pixel.)
+    for (int c = 0; c < chunks; c += kSolveAhead) {
+#pragma unroll
+        for (int k = 0; k < kSolveAhead; ++k) {
+            const int after = chunk_base[min(c + k + kSolveAhead + 2, chunks)];
+            chunk(sd[k], base[0], base[1], base[kSolveAhead], base[kSolveAhead + 1]);
+#pragma unroll
+            for (int q = 0; q <= kSolveAhead; ++q) base[q] = base[q + 1];
+            base[kSolveAhead + 1] = __builtin_amdgcn_readfirstlane(after);
+        }
+    }
+}
+
+__global__ __launch_bounds__(kSolveThreads) void k_jcp_solve(DevBuf d, Layout L) {
+    __shared__ SolveLds lds;
+    const int f = blockIdx.x;
+    const FrameDesc& fd = d.frames[f];
+    const int H = fd.sc.H;
+    const int nq = static_cast<int>(d.fs[f * kFsCount + kFsQueue]);
+    const int tid = threadIdx.x;
+    if (nq > kQueueMax || H > kSolveRows) {
         if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrQueueCapacity);
         return;
     }
     if (nq == 0) return;
     const size_t qo = (size_t)f * L.P;
-    for (int r = tid; r <= s.H; r += kSolveThreads) row_start[r] = r < s.H ? d.qrow[(size_t)f * (L.H + 1) + r] : nq;
-    if (tid < kFinBase) fin[tid] = static_cast<uint8_t>(tid == 0 ? kSO : (tid == 1 ? kSG : kSU));
+    const uint4* rec = d.slot_rec + qo * kRecordParts;
+    const size_t P = static_cast<size_t>(L.P);
+    // Chunks in queue order, two rows per thread: a row's chunks start at its
+    // first queue pixel and every kSolveThreads further.  A chunk ends where
+    // the next begins; past the last one every base is nq.
+    const int32_t* qrow = d.qrow + (size_t)f * (L.H + 1);
+    auto row_at = [&](int r) { return r < H ? qrow[r] : nq; };
+    const int r0 = 2 * tid, b0 = row_at(r0), b1 = row_at(r0 + 1), b2 = row_at(r0 + 2);
+    const int n0 = (b1 - b0 + kSolveThreads - 1) / kSolveThreads, n1 = (b2 - b1 + kSolveThreads - 1) / kSolveThreads;
+    int chunks;
+    const int c0 = block_exclusive_sum<kSolveThreads>(n0 + n1, lds.scan, &chunks);
+    for (int k = 0; k < n0; ++k) lds.chunk_base[c0 + k] = b0 + k * kSolveThreads;
+    for (int k = 0; k < n1; ++k) lds.chunk_base[c0 + n0 + k] = b1 + k * kSolveThreads;
+    if (tid < 2 + kSolveAhead) lds.chunk_base[chunks + tid] = nq;
+    if (tid < kLabelBase) lds.lab[tid] = static_cast<int8_t>(tid == 0 ? 1 : (tid == 1 ? -1 : 0));
     __syncthreads();
-    auto row_at = [&](int r) { return __builtin_amdgcn_readfirstlane(row_start[r]); };
-    // Chunks run in queue order: a row's chunks start at rs, rs + T, ... below
-    // its end re, and the next chunk after the row's last starts at re, the
-    // first queue pixel of the next non-empty row (row_start[H] = nq).
-    int r = 0;
-    while (row_at(r + 1) == 0) ++r;
-    int base = 0;
-    uint32_t carry = kSU * 3 + kSU;
-    // One chunk with the slot data `cur`, prefetching the next chunk's into
-    // `nxt` (its index is clamped to the last queue pixel, so every path has
-    // the same loads in flight and the compiler waits for the current chunk's
-    // data only).  Returns false after the last chunk.
-    auto chunk = [&](const SlotData& cur, SlotData& nxt) -> bool {
-        const int rs = row_at(r), re = row_at(r + 1);
-        const int j = base + tid;
-        const int nb = base + kSolveThreads < re ? base + kSolveThreads : re;
-        load_slots(d, qo, min(nb + tid, nq - 1), nxt);
-        TMap m = j < re ? pixel_map(cur, j, rs, fin) : TMap{kIdLo, kIdHi, kIdX};
-        m = tmap_wave_scan(m);  // m := m_j o ... o m_(first of this wavefront)
-        if (lane == kWave - 1) wtot[w] = m;
-        __syncthreads();
-        // Prefixes of the wavefront totals: lane q scans wtot[q] o ... o
-        // wtot[0] with DPP row shifts (the totals sit in lanes 0..7 of row
-        // 0); pre is the prefix of the earlier wavefronts, chain that of all
-        // of them.
-        TMap t = lane < kSolveWaves ? wtot[lane] : TMap{kIdLo, kIdHi, kIdX};
-        t = tmap_compose(t, tmap_dpp<0x111, 0xf>(t));
-        t = tmap_compose(t, tmap_dpp<0x112, 0xf>(t));
-        t = tmap_compose(t, tmap_dpp<0x114, 0xf>(t));
-        static_assert(kSolveWaves <= 8, "three row-shift steps scan at most 8 wavefront totals");
-        const TMap chain = tmap_readlane(t, kSolveWaves - 1);
-        if (w > 0) m = tmap_compose(m, tmap_readlane(t, w - 1));
-        const uint32_t ps = tmap_get(m, carry);
-        if (j < re) fin[kFinBase + j] = static_cast<uint8_t>(ps % 3);
-        carry = tmap_get(chain, carry);
-        __syncthreads();
-        if (nb < re) {
-            base = nb;
-            return true;
-        }
-        if (nb >= nq) return false;
-        ++r;
-        while (row_at(r + 1) == nb) ++r;
-        base = nb;
-        carry = kSU * 3 + kSU;
-        return true;
-    };
-    SlotData sa, sb;
-    load_slots(d, qo, min(tid, nq - 1), sa);
-    while (chunk(sa, sb) && chunk(sb, sa)) {
-    }
+    chunks = __builtin_amdgcn_readfirstlane(chunks);
+    if (nq > (1 << 16) - kLabelBase)
+        solve_rows<true>(rec, P, nq, chunks, lds);
+    else
+        solve_rows<false>(rec, P, nq, chunks, lds);
     for (int j = tid; j < nq; j += kSolveThreads) {
-        const uint32_t v = fin[kFinBase + j];
-        d.fin[qo + j] = v == kSG ? kGround : (v == kSO ? kObstacle : kPending);
+        const int v = lds.lab[j + kLabelBase];
+        d.fin[qo + j] = v < 0 ? kGround : (v > 0 ? kObstacle : kPending);
     }
 }
 
