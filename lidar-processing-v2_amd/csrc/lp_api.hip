@@ -382,7 +382,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.clabel, B * N);
     x.nloc = x.clabel;
     go(x.cell_count, B * C);
-    go(x.cell_start, B * (C + 1));
+    go(x.cell_start, B * C);
     go(x.pt_loc, B * N);
     go(x.cell_items, B * N);
     go(x.cell_zkey, B * N);
@@ -395,7 +395,6 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.big_cells, B * C);
     go(x.cell_list, B * C);
     go(x.cand_count, B * L.cand_stride);
-    go(x.cand_start, B * L.cand_stride);
     go(x.cx, B * N);
     go(x.cy, B * N);
     go(x.cz, B * N);

@@ -130,17 +130,16 @@ struct DevBuf {
     int32_t* clabel;         // cluster label per obstacle point
     // per cell (frame stride cell_stride)
     uint32_t* cell_count;
-    uint32_t* cell_start;    // stride cell_stride + 1 used
+    uint32_t* cell_start;    // first of the cell's entries in cell_items
     int32_t* pt_loc;         // per point (CSR): its place inside its polar cell
     int32_t* cell_items;     // frame stride N
     uint32_t* cell_zkey;     // frame stride N: ord_f32(z) of the cell_items entries, in fill order
     float* zmin;
     float* elev;
     uint32_t* big_cells;     // per frame list of cells needing a workgroup sort
-    uint4* cell_list;        // per frame: the non-empty cells in cell order, {cell, start, count, 0}
+    uint4* cell_list;        // per frame: the non-empty cells, {cell, start, count, 0}: small ones from the front, others from the back
     // RANSAC (per frame)
     uint32_t* cand_count;    // frame stride cand_stride
-    uint32_t* cand_start;
     float *cx, *cy, *cz;     // candidates, frame stride N
     float* hyp;              // [B][60][4]
     uint32_t* hyp_valid;     // [B][60]
@@ -251,7 +250,9 @@ enum FsSlot : int {
     kFsErr,
     kFsBoxes,          // clusters with a box
     kFsHullLarge,      // clusters listed for the workgroup local-rank launch
-    kFsCellsUsed,      // non-empty polar cells
+    kFsCellPoints,     // points in polar cells
+    kFsCellsSmall,     // non-empty polar cells of up to 16 points
+    kFsCellsLarge,     // larger ones
     kFsGround,         // GROUND points (label clouds on)
     kFsVehicles,       // clusters classified as vehicles
     // kept across the per-run clear: written by the noise filter before it

@@ -96,54 +96,57 @@ __global__ __launch_bounds__(256) void k_project_q(DevBuf d, Layout L, int B) {
            [&](int f, int t) { project_tile(d, L, f, t); });
 }
 
-// Exclusive scan of the cell histogram, one 1024-thread workgroup per frame.
-// Cell starts (exclusive scan of the counts), the list of non-empty cells
-// with their starts and counts for k_cell_sort, and the empty marker of every
-// empty cell's minimum.
-__global__ __launch_bounds__(1024) void k_cell_scan(DevBuf d, Layout L) {
-    __shared__ uint64_t lds[1024 / kWave + 1];
-    const int f = blockIdx.x;
+// Cell starts, the lists of non-empty cells for k_cell_sort, and the empty
+// marker of every empty cell's minimum.  Where a cell's points lie does not
+// matter, so each workgroup reserves room for its 2048 cells with one atomic
+// per total instead of a scan over the frame by one workgroup (28 -> 6 us per
+// frame).  Cells of up to kRowCell points are listed from the front of
+// cell_list, larger ones from its back.
+constexpr int kStartThreads = 256;
+constexpr int kStartItems = 8;
+constexpr uint32_t kRowCell = 16;  // points of a cell sorted by one 16-lane row
+
+__global__ __launch_bounds__(kStartThreads) void k_cell_start(DevBuf d, Layout L) {
+    __shared__ uint64_t lds[kStartThreads / kWave + 1];
+    __shared__ uint32_t first[3];
+    const int f = blockIdx.y;
     const int cells = d.frames[f].sc.cells;
+    const int b = (blockIdx.x * kStartThreads + threadIdx.x) * kStartItems;
+    if (static_cast<int>(blockIdx.x) * kStartThreads * kStartItems >= cells) return;
     const size_t co = (size_t)f * L.cell_stride;
-    const uint32_t* cnt = d.cell_count + co;
-    uint32_t* st = d.cell_start + (size_t)f * (L.cell_stride + 1);
-    uint4* list = d.cell_list + co;
-    float* zmin = d.zmin + co;
-    uint32_t carry = 0, used = 0;
-    for (int base = 0; base < cells; base += 1024 * 8) {
-        uint32_t v[8];
-        uint32_t local = 0, nz = 0;
-        const int b = base + threadIdx.x * 8;
+    uint32_t v[kStartItems];
+    uint64_t sum = 0;  // points in the low word, then small and large cells
 #pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            v[k] = (b + k < cells) ? cnt[b + k] : 0u;
-            local += v[k];
-            nz += v[k] ? 1u : 0u;
-        }
-        // Both sums in one block scan: the point count in the high word, the
-        // non-empty cell count in the low one (each frame total < 2^32).
-        uint64_t both_total;
-        const uint64_t both = block_exclusive_sum<1024>((static_cast<uint64_t>(local) << 32) | nz, lds, &both_total);
-        const uint32_t total = static_cast<uint32_t>(both_total >> 32), nz_total = static_cast<uint32_t>(both_total);
-        uint32_t ex = static_cast<uint32_t>(both >> 32) + carry;
-        uint32_t lx = static_cast<uint32_t>(both) + used;
-#pragma unroll
-        for (int k = 0; k < 8; ++k) {
-            if (b + k < cells) {
-                st[b + k] = ex;
-                if (v[k])
-                    list[lx++] = make_uint4(static_cast<uint32_t>(b + k), ex, v[k], 0u);
-                else
-                    zmin[b + k] = u2f(kEmptyZ);
-            }
-            ex += v[k];
-        }
-        carry += total;
-        used += nz_total;
+    for (int k = 0; k < kStartItems; ++k) {
+        v[k] = (b + k < cells) ? d.cell_count[co + b + k] : 0u;
+        sum += v[k] + (v[k] ? (v[k] <= kRowCell ? 1ull << 32 : 1ull << 48) : 0ull);
     }
-    if (threadIdx.x == 0) {
-        st[cells] = carry;
-        d.fs[f * kFsCount + kFsCellsUsed] = used;
+    uint64_t total;
+    const uint64_t ex = block_exclusive_sum<kStartThreads>(sum, lds, &total);
+    if (threadIdx.x < 3) {
+        uint32_t* fs = d.fs + f * kFsCount;
+        uint32_t* ctr = fs + (threadIdx.x == 0 ? kFsCellPoints : (threadIdx.x == 1 ? kFsCellsSmall : kFsCellsLarge));
+        const uint32_t add = threadIdx.x == 0 ? static_cast<uint32_t>(total)
+                                              : static_cast<uint32_t>(total >> (threadIdx.x == 1 ? 32 : 48)) & 0xffffu;
+        first[threadIdx.x] = add ? atomicAdd(ctr, add) : 0u;
+    }
+    __syncthreads();
+    uint32_t start = first[0] + static_cast<uint32_t>(ex);
+    uint32_t small = first[1] + (static_cast<uint32_t>(ex >> 32) & 0xffffu);
+    uint32_t large = first[2] + static_cast<uint32_t>(ex >> 48);
+    uint4* list = d.cell_list + co;
+#pragma unroll
+    for (int k = 0; k < kStartItems; ++k) {
+        if (b + k >= cells) break;
+        d.cell_start[co + b + k] = start;
+        const uint4 e = make_uint4(static_cast<uint32_t>(b + k), start, v[k], 0u);
+        if (v[k] == 0)
+            d.zmin[co + b + k] = u2f(kEmptyZ);
+        else if (v[k] <= kRowCell)
+            list[small++] = e;
+        else
+            list[L.cell_stride - 1 - static_cast<int>(large++)] = e;
+        start += v[k];
     }
 }
 
@@ -158,7 +161,7 @@ __global__ void k_cell_fill(DevBuf d, Layout L) {
     const int gi = fd.pt_off + i;
     const int cell = d.pt_cell[gi];
     if (cell < 0) return;
-    const uint32_t pos = d.cell_start[(size_t)f * (L.cell_stride + 1) + cell] + static_cast<uint32_t>(d.pt_loc[gi]);
+    const uint32_t pos = d.cell_start[(size_t)f * L.cell_stride + cell] + static_cast<uint32_t>(d.pt_loc[gi]);
     d.cell_items[(size_t)f * L.N + pos] = i;
     d.cell_zkey[(size_t)f * L.N + pos] = ord_f32(d.z[gi]);
 }
@@ -300,74 +303,67 @@ __device__ __forceinline__ void sort_cell_row(int32_t* items, const uint32_t* zk
     }
 }
 
-// One wavefront per non-empty cell (a grid-stride loop over the cell list):
-// sorts the cell's point indices ascending (so the cell lists follow the
-// reference's input order) for the RANSAC cells, and sorts z for the robust
-// minimum.  A wavefront takes four consecutive cells of the list (each entry
-// carries the cell's start and count): those of up to 16 points are sorted
-// by one 16-lane row each (DPP bitonic), the others one after the other by
-// the whole wavefront.  Cells up to kSmallCell (512) points sort in
-// registers; larger ones are queued for k_cell_sort_big.
+// Sorts the point indices of every RANSAC cell ascending (so the cell lists
+// follow the reference's input order) and z for the robust minimum.  Cells of
+// up to 16 points are sorted by one 16-lane row each (DPP bitonic), four to a
+// wavefront; larger ones, up to kSmallCell (512) points, by a wavefront each in
+// registers; beyond that they are queued for k_cell_sort_big.  The cells near
+// the sensor are both the largest and neighbours in cell order, so taken in
+// that order a wavefront got four of them in a row and was the launch's tail:
+// 22 -> 14 us per frame with the large cells on a list of their own.
 __global__ __launch_bounds__(256) void k_cell_sort(DevBuf d, Layout L) {
     static_assert(kSmallCell == 8 * kWave, "the register sorts cover cells up to kSmallCell points");
     int tile, f;
     xcd_tile_frame(tile, f);
     const FrameDesc& fd = d.frames[f];
     const SegConst& s = fd.sc;
-    const int w = threadIdx.x / kWave;
     const int lane = lane_id();
     const size_t co = (size_t)f * L.cell_stride;
-    const int used = static_cast<int>(d.fs[f * kFsCount + kFsCellsUsed]);
+    const int small = static_cast<int>(d.fs[f * kFsCount + kFsCellsSmall]);
+    const int large = static_cast<int>(d.fs[f * kFsCount + kFsCellsLarge]);
     const int waves = gridDim.x * 4;
+    const int wave = tile * 4 + static_cast<int>(threadIdx.x) / kWave;
     float* zmin = d.zmin + co;
-    // Row g of the wavefront takes list entry q4 + g; the entry of its next
-    // iteration is loaded one iteration ahead.
+    const uint4* list = d.cell_list + co;
+    for (int q = wave; q < large; q += waves) {
+        const uint4 e = list[L.cell_stride - 1 - q];
+        const int cell = __builtin_amdgcn_readfirstlane(static_cast<int>(e.x));
+        const int n = __builtin_amdgcn_readfirstlane(static_cast<int>(e.z));
+        const uint32_t start = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(e.y)));
+        if (n > kSmallCell) {
+            if (lane == 0) {
+                const uint32_t k = atomicAdd(&d.fs[f * kFsCount + kFsNumBig], 1u);
+                if (k < static_cast<uint32_t>(L.cell_stride)) d.big_cells[co + k] = cell;
+            }
+            continue;
+        }
+        int32_t* items = d.cell_items + (size_t)f * L.N + start;
+        const uint32_t* zk = d.cell_zkey + (size_t)f * L.N + start;
+        const int radial = cell % s.rings;
+        if (n <= kWave)
+            sort_cell_regs<1>(items, zk, n, radial, zmin + cell);
+        else if (n <= 2 * kWave)
+            sort_cell_regs<2>(items, zk, n, radial, zmin + cell);
+        else if (n <= 4 * kWave)
+            sort_cell_regs<4>(items, zk, n, radial, zmin + cell);
+        else
+            sort_cell_regs<8>(items, zk, n, radial, zmin + cell);
+    }
+    // Row g of the wavefront takes list entry q + g.  The wavefronts after
+    // those with a large cell come first; an entry is loaded one iteration
+    // ahead.
     const int g = lane >> 4;
-    const int step = waves * 4;
-    int q4 = (tile * 4 + w) * 4;
-    const uint4 none = make_uint4(0xffffffffu, 0u, 0u, 0u);
-    uint4 next = q4 + g < used ? d.cell_list[co + q4 + g] : none;
-    for (; q4 < used; q4 += step) {
+    const int turn = (wave - large % waves + waves) % waves;
+    const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+    uint4 next = turn * 4 + g < small ? list[turn * 4 + g] : none;
+    for (int q = turn * 4; q < small; q += waves * 4) {
         const uint4 e = next;
-        next = q4 + step + g < used ? d.cell_list[co + q4 + step + g] : none;
-        const int cell_g = static_cast<int>(e.x);  // -1: no entry
-        const uint32_t start_g = e.y;
-        const uint32_t n_g = e.z;
-        if (cell_g >= 0 && n_g <= 16u) {
-            sort_cell_row(d.cell_items + (size_t)f * L.N + start_g, d.cell_zkey + (size_t)f * L.N + start_g,
-                          static_cast<int>(n_g), cell_g % s.rings, zmin + cell_g);
-        }
-        // Rows whose cell is larger: the whole wavefront, one cell at a time.
-        const uint64_t large = __ballot(cell_g >= 0 && n_g > 16u && (lane & 15) == 0);
-        for (int gg = 0; gg < 4; ++gg) {
-            if (!((large >> (gg * 16)) & 1ull)) continue;
-            const int cell = __shfl(cell_g, gg * 16, kWave);
-            const uint32_t n = static_cast<uint32_t>(__shfl(static_cast<int>(n_g), gg * 16, kWave));
-            if (n > static_cast<uint32_t>(kSmallCell)) {
-                if (lane == 0) {
-                    const uint32_t k = atomicAdd(&d.fs[f * kFsCount + kFsNumBig], 1u);
-                    if (k < static_cast<uint32_t>(L.cell_stride)) d.big_cells[co + k] = cell;
-                }
-                continue;
-            }
-            const uint32_t start = static_cast<uint32_t>(__shfl(static_cast<int>(start_g), gg * 16, kWave));
-            int32_t* items = d.cell_items + (size_t)f * L.N + start;
-            const uint32_t* zk = d.cell_zkey + (size_t)f * L.N + start;
-            const int radial = cell % s.rings;
-            if (n <= static_cast<uint32_t>(kWave)) {
-                sort_cell_regs<1>(items, zk, static_cast<int>(n), radial, zmin + cell);
-                continue;
-            }
-            if (n <= static_cast<uint32_t>(2 * kWave)) {
-                sort_cell_regs<2>(items, zk, static_cast<int>(n), radial, zmin + cell);
-                continue;
-            }
-            if (n <= static_cast<uint32_t>(4 * kWave)) {
-                sort_cell_regs<4>(items, zk, static_cast<int>(n), radial, zmin + cell);
-                continue;
-            }
-            sort_cell_regs<8>(items, zk, static_cast<int>(n), radial, zmin + cell);  // n <= kSmallCell
-        }
+        const int ahead = q + waves * 4 + g;
+        next = ahead < small ? list[ahead] : none;
+        const int cell = static_cast<int>(e.x);
+        if (e.z)
+            sort_cell_row(d.cell_items + (size_t)f * L.N + e.y, d.cell_zkey + (size_t)f * L.N + e.y,
+                          static_cast<int>(e.z), cell % s.rings, zmin + cell);
     }
 }
 
@@ -389,7 +385,7 @@ __global__ __launch_bounds__(1024) void k_cell_sort_big(DevBuf d, Layout L) {
             if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrCellCapacity);
             continue;
         }
-        const uint32_t start = d.cell_start[(size_t)f * (L.cell_stride + 1) + cell];
+        const uint32_t start = d.cell_start[(size_t)f * L.cell_stride + cell];
         int32_t* items = d.cell_items + (size_t)f * L.N + start;
         int m = 1;
         while (m < static_cast<int>(n)) m <<= 1;
@@ -425,52 +421,79 @@ __global__ __launch_bounds__(1024) void k_cell_sort_big(DevBuf d, Layout L) {
 // RECM recurrence along each azimuth slice (segmenter.cpp:215-267).  The
 // 49 float additions must happen in order (a log-step min-plus scan would
 // re-associate them), so each slice is one sequential lane.
-// One wavefront per 64 slices.  A slice's cells are contiguous (cell =
-// slice * rings + r), so the wavefront's 64 x rings minima are one
-// contiguous block: it is loaded into LDS with coalesced reads, each lane runs
-// its slice's recurrence there, and the elevations go back the same way.
-// Grids with more than kRecmRings rings read and write global memory
-// directly (eight rings' minima loaded ahead of their eight steps).
+// One workgroup per 64 slices.  A slice's cells are contiguous (cell =
+// slice * rings + r), so its 64 x rings minima are one contiguous block: four
+// wavefronts load it into LDS with coalesced reads in flight together (one
+// wavefront waited for them in 49 turns: 17 -> 8 us per frame), each lane
+// of the first runs its slice's recurrence there, and the elevations go back
+// the same way.  Grids with more than kRecmRings rings read and write global
+// memory directly (eight rings' minima loaded ahead of their eight steps).
 constexpr int kRecmRings = 64;
+constexpr int kRecmThreads = 256;
 
-__global__ __launch_bounds__(kWave) void k_recm(DevBuf d, Layout L) {
-    __shared__ float blk[kWave * kRecmRings];
+__global__ __launch_bounds__(kRecmThreads) void k_recm(DevBuf d, Layout L) {
+    __shared__ float blk[kWave * (kRecmRings + 1)];
     const int f = blockIdx.y;
     const SegConst& s = d.frames[f].sc;
     const int s0 = blockIdx.x * kWave;
     if (s0 >= s.slices) return;
-    const int lane = lane_id();
-    const int sl = s0 + lane;
+    const int tid = threadIdx.x;
     const int R = s.rings;
     const size_t co = (size_t)f * L.cell_stride;
     float* E = d.elev + co;
     const float* zm = d.zmin + co;
     auto step = [&](float prev, float z) {
-        if (f2u(z) == kEmptyZ) return prev + s.dz;
         const float b = prev + s.dz;
+        if (f2u(z) == kEmptyZ) return b;
         return (b < z) ? b : z;  // std::min(curr_z_min, prev + dz)
     };
     if (R <= kRecmRings) {
         const int ns = min(kWave, s.slices - s0);
         const int total = ns * R;
         const float* src = zm + (size_t)s0 * R;
-        for (int i = lane; i < total; i += kWave) blk[i] = src[i];
+        // An odd row length keeps the lanes of the recurrence on different
+        // banks.
+        const int pitch = R | 1;
+        constexpr int kTurns = kWave * kRecmRings / kRecmThreads;
+        float v[kTurns];
+#pragma unroll
+        for (int k = 0; k < kTurns; ++k) {
+            const int i = tid + k * kRecmThreads;
+            v[k] = i < total ? src[i] : 0.0f;
+        }
+#pragma unroll
+        for (int k = 0; k < kTurns; ++k) {
+            const int i = tid + k * kRecmThreads;
+            if (i < total) blk[(i / R) * pitch + i % R] = v[k];
+        }
         __syncthreads();
-        if (lane < ns) {
-            float* row = blk + lane * R;
+        if (tid < ns) {
+            float* row = blk + tid * pitch;
             float prev = s.e0;
             row[0] = prev;
-            for (int r = 1; r < R; ++r) {
-                prev = step(prev, row[r]);
-                row[r] = prev;
+            for (int r0 = 1; r0 < R; r0 += 8) {
+                float z[8];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) z[k] = row[min(r0 + k, R - 1)];
+#pragma unroll
+                for (int k = 0; k < 8; ++k) {
+                    if (r0 + k >= R) break;
+                    prev = step(prev, z[k]);
+                    row[r0 + k] = prev;
+                }
             }
         }
         __syncthreads();
         float* dst = E + (size_t)s0 * R;
-        for (int i = lane; i < total; i += kWave) dst[i] = blk[i];
+#pragma unroll
+        for (int k = 0; k < kTurns; ++k) {
+            const int i = tid + k * kRecmThreads;
+            if (i < total) dst[i] = blk[(i / R) * pitch + i % R];
+        }
         return;
     }
-    if (sl >= s.slices) return;
+    const int sl = s0 + tid;
+    if (tid >= kWave || sl >= s.slices) return;
     const int off = sl * R;
     E[off] = s.e0;
     float prev = s.e0;
@@ -500,7 +523,7 @@ __global__ __launch_bounds__(256) void k_cand_count(DevBuf d, Layout L) {
     const int cell = (k / kRansacRadialBins) * s.rings + (k % kRansacRadialBins);
     const size_t co = (size_t)f * L.cell_stride;
     const uint32_t n = d.cell_count[co + cell];
-    const uint32_t start = d.cell_start[(size_t)f * (L.cell_stride + 1) + cell];
+    const uint32_t start = d.cell_start[(size_t)f * L.cell_stride + cell];
     const uint32_t* zk = d.cell_zkey + (size_t)f * L.N + start;  // the cell's z in any order
     const float e = d.elev[co + cell];
     uint32_t c = 0;
@@ -513,72 +536,62 @@ __global__ __launch_bounds__(256) void k_cand_count(DevBuf d, Layout L) {
     }
 }
 
-__global__ __launch_bounds__(1024) void k_cand_scan(DevBuf d, Layout L) {
-    __shared__ uint32_t lds[1024 / kWave + 1];
-    const int f = blockIdx.x;
-    const SegConst& s = d.frames[f].sc;
-    const int cnt = s.slices * kRansacRadialBins;
-    const uint32_t* in = d.cand_count + (size_t)f * L.cand_stride;
-    uint32_t* out = d.cand_start + (size_t)f * L.cand_stride;
-    uint32_t carry = 0;
-    for (int base = 0; base < cnt; base += 1024 * 4) {
-        uint32_t v[4];
-        uint32_t local = 0;
-        const int b = base + threadIdx.x * 4;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            v[q] = (b + q < cnt) ? in[b + q] : 0u;
-            local += v[q];
-        }
-        uint32_t total;
-        uint32_t ex = block_exclusive_sum<1024>(local, lds, &total) + carry;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-            if (b + q < cnt) out[b + q] = ex;
-            ex += v[q];
-        }
-        carry += total;
-    }
-    if (threadIdx.x == 0) d.fs[f * kFsCount + kFsCands] = carry;
-}
-
-// Candidate compaction: each wave writes its cell's candidates in input
-// order at the cell's scanned offset (grid-stride over the near cells).
+// Candidate compaction in the reference's order, a wavefront per near cell and
+// four cells in a row per workgroup and turn.  A workgroup sums the counts of
+// the cells before its own itself (a few reads per thread; a launch for their
+// scan cost more than that); the one with the last cells writes the total.
 __global__ __launch_bounds__(256) void k_cand_fill(DevBuf d, Layout L) {
+    __shared__ uint32_t part[256 / kWave];
     const int f = blockIdx.y;
     const FrameDesc& fd = d.frames[f];
     const SegConst& s = fd.sc;
     const int w = threadIdx.x / kWave;
     const int lane = lane_id();
-    for (int k = blockIdx.x * 4 + w; k < s.slices * kRansacRadialBins; k += gridDim.x * 4) {
-    const int cell = (k / kRansacRadialBins) * s.rings + (k % kRansacRadialBins);
+    const int cells = s.slices * kRansacRadialBins;
+    const uint32_t* count = d.cand_count + (size_t)f * L.cand_stride;
     const size_t co = (size_t)f * L.cell_stride;
-    const uint32_t n = d.cell_count[co + cell];
-    const uint32_t start = d.cell_start[(size_t)f * (L.cell_stride + 1) + cell];
-    const int32_t* items = d.cell_items + (size_t)f * L.N + start;
-    const float e = d.elev[co + cell];
-    uint32_t pos = d.cand_start[(size_t)f * L.cand_stride + k];
     const size_t ob = (size_t)f * L.N;
-    for (uint32_t t0 = 0; t0 < n; t0 += kWave) {
-        const uint32_t t = t0 + lane;
-        bool pred = false;
-        float x = 0, y = 0, z = 0;
-        if (t < n) {
-            const float4 pc = d.pt_xyzc[fd.pt_off + items[t]];  // one gather per point
-            x = pc.x;
-            y = pc.y;
-            z = pc.z;
-            pred = fabsf(e - z) < s.two_thr;
+    uint32_t before = 0;  // candidates of the cells before k0
+    int summed = 0;
+    for (int k0 = blockIdx.x * 4; k0 < cells; k0 += gridDim.x * 4) {
+        uint32_t sum = 0;
+        for (int i = summed + threadIdx.x; i < k0; i += 256) sum += count[i];
+        sum = wave_sum(sum);
+        if (lane == 0) part[w] = sum;
+        __syncthreads();
+        before += part[0] + part[1] + part[2] + part[3];
+        __syncthreads();
+        summed = k0;
+        uint32_t pos = before;
+        for (int q = 0; q < w; ++q) pos += k0 + q < cells ? count[k0 + q] : 0u;
+        const int k = k0 + w;
+        if (k + 1 == cells && lane == 0) d.fs[f * kFsCount + kFsCands] = pos + count[k];
+        if (k >= cells) continue;
+        const int cell = (k / kRansacRadialBins) * s.rings + (k % kRansacRadialBins);
+        const uint32_t n = d.cell_count[co + cell];
+        const uint32_t start = d.cell_start[co + cell];
+        const int32_t* items = d.cell_items + ob + start;
+        const float e = d.elev[co + cell];
+        for (uint32_t t0 = 0; t0 < n; t0 += kWave) {
+            const uint32_t t = t0 + lane;
+            bool pred = false;
+            float x = 0, y = 0, z = 0;
+            if (t < n) {
+                const float4 pc = d.pt_xyzc[fd.pt_off + items[t]];  // one gather per point
+                x = pc.x;
+                y = pc.y;
+                z = pc.z;
+                pred = fabsf(e - z) < s.two_thr;
+            }
+            const uint64_t mask = __ballot(pred);
+            if (pred) {
+                const uint32_t o = pos + lanes_below(mask);
+                d.cx[ob + o] = x;
+                d.cy[ob + o] = y;
+                d.cz[ob + o] = z;
+            }
+            pos += static_cast<uint32_t>(__popcll(mask));
         }
-        const uint64_t mask = __ballot(pred);
-        if (pred) {
-            const uint32_t o = pos + lanes_below(mask);
-            d.cx[ob + o] = x;
-            d.cy[ob + o] = y;
-            d.cz[ob + o] = z;
-        }
-        pos += static_cast<uint32_t>(__popcll(mask));
-    }
     }
 }
 
@@ -609,197 +622,199 @@ __global__ void k_mt19937(uint32_t* out, int count) {
     }
 }
 
-// Hypotheses: lane 0 maps the raw stream to indices with libstdc++'s
+// The index pairs of the 60 hypotheses by one lane: libstdc++'s
 // uniform_int_distribution<uint32_t> for a 32-bit engine (Lemire's
-// nearly-divisionless method, bits/uniform_int_dist.h), redrawing p3 while
-// it equals p2 (segmenter.cpp:379-386); lanes 0..59 then build the planes
-// (segmenter.cpp:389-418).
-__global__ __launch_bounds__(64) void k_ransac_hyp(DevBuf d, Layout L) {
-    __shared__ uint32_t idx2[kRansacIters], idx3[kRansacIters];
-    // 60 hypotheses draw about 120 values (a few more after rejections or
-    // repeated indices): the first 256 are staged in LDS, later ones are read
-    // from global memory.
-    constexpr int kStaged = 256;
-    __shared__ uint32_t raw[kStaged];
-    __shared__ uint32_t ok;
-    const int f = blockIdx.x;
-    const FrameDesc& fd = d.frames[f];
-    const SegConst& s = fd.sc;
-    const uint32_t n = d.fs[f * kFsCount + kFsCands];
-    const int lane = threadIdx.x;
-    if (n == 0) return;  // no candidates: the reference returns (segmenter.cpp:353-356)
-    if (n == 1) {
-        if (lane == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrRansacSingle);
-        return;
-    }
-#pragma unroll
-    for (int i = lane; i < kStaged; i += 64) raw[i] = d.mt_raw[i];
-    __syncthreads();
-    if (lane == 0) {
-        int pos = 0;
-        bool good = true;
-        auto draw = [&]() -> uint32_t {
-            if (pos >= kMtRawCount) {
-                good = false;
-                return 0;
-            }
-            uint64_t prod = static_cast<uint64_t>(pos < kStaged ? raw[pos] : d.mt_raw[pos]) * n;
-            ++pos;
-            uint32_t low = static_cast<uint32_t>(prod);
-            if (low < n) {
-                const uint32_t thresh = (0u - n) % n;
-                while (low < thresh && good) {
-                    if (pos >= kMtRawCount) {
-                        good = false;
-                        break;
-                    }
-                    prod = static_cast<uint64_t>(pos < kStaged ? raw[pos] : d.mt_raw[pos]) * n;
-                    ++pos;
-                    low = static_cast<uint32_t>(prod);
+// nearly-divisionless method, bits/uniform_int_dist.h) over the raw stream,
+// redrawing p3 while it equals p2 (segmenter.cpp:379-386).  False when the
+// stored stream ends.
+__device__ bool draw_pairs(const uint32_t* raw, uint32_t n, uint2* pairs) {
+    int pos = 0;
+    bool good = true;
+    auto draw = [&]() -> uint32_t {
+        if (pos >= kMtRawCount) {
+            good = false;
+            return 0;
+        }
+        uint64_t prod = static_cast<uint64_t>(raw[pos]) * n;
+        ++pos;
+        uint32_t low = static_cast<uint32_t>(prod);
+        if (low < n) {
+            const uint32_t thresh = (0u - n) % n;
+            while (low < thresh && good) {
+                if (pos >= kMtRawCount) {
+                    good = false;
+                    break;
                 }
+                prod = static_cast<uint64_t>(raw[pos]) * n;
+                ++pos;
+                low = static_cast<uint32_t>(prod);
             }
-            return static_cast<uint32_t>(prod >> 32);
-        };
-        for (int it = 0; it < kRansacIters && good; ++it) {
-            const uint32_t a = draw();
-            uint32_t b = draw();
-            while (b == a && good) b = draw();
-            idx2[it] = a;
-            idx3[it] = b;
         }
-        ok = good ? 1u : 0u;
-        if (!good) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrRngExhausted);
+        return static_cast<uint32_t>(prod >> 32);
+    };
+    for (int it = 0; it < kRansacIters && good; ++it) {
+        const uint32_t a = draw();
+        uint32_t b = draw();
+        while (b == a && good) b = draw();
+        pairs[it] = make_uint2(a, b);
     }
-    __syncthreads();
-    if (!ok || lane >= kRansacIters) return;
-    const size_t ob = (size_t)f * L.N;
-    const float p1x = 0.0f, p1y = 0.0f, p1z = s.neg_h;
-    const uint32_t i2 = idx2[lane], i3 = idx3[lane];
-    const float p2x = d.cx[ob + i2], p2y = d.cy[ob + i2], p2z = d.cz[ob + i2];
-    const float p3x = d.cx[ob + i3], p3y = d.cy[ob + i3], p3z = d.cz[ob + i3];
-    float nx = ((p2y - p1y) * (p3z - p1z)) - ((p2z - p1z) * (p3y - p1y));
-    float ny = ((p2z - p1z) * (p3x - p1x)) - ((p2x - p1x) * (p3z - p1z));
-    float nz = ((p2x - p1x) * (p3y - p1y)) - ((p2y - p1y) * (p3x - p1x));
-    const float den2 = (nx * nx) + (ny * ny) + (nz * nz);
-    uint32_t valid = 0;
-    float pd = 0.0f;
-    if (!(den2 < 1.0e-5F)) {
-        const float norm = 1.0F / sqrtf(den2);
-        nz *= norm;
-        if (!(fabsf(nz) < s.cos_max)) {
-            nx *= norm;
-            ny *= norm;
-            pd = (nx * p1x) + (ny * p1y) + (nz * p1z);
-            valid = 1;
-        }
-    }
-    float* h = d.hyp + ((size_t)f * kRansacIters + lane) * 4;
-    h[0] = nx;
-    h[1] = ny;
-    h[2] = nz;
-    h[3] = pd;
-    d.hyp_valid[f * kRansacIters + lane] = valid;
+    return good;
 }
 
-// Inlier counts of all 60 hypotheses at once: one candidate per thread,
-// ballot + popcount per hypothesis, LDS totals, one atomic per block and
-// hypothesis (segmenter.cpp:420-431).
-constexpr int kScoreRows = 4;  // candidates per thread: rows of 256, each plane read once for all of them
-
-// Every candidate scores all hypotheses (segmenter.cpp:410-430: |a x + b y +
-// c z - d| < thr, the same float expression).  The planes are read as
-// wavefront-uniform values (scalar loads, no LDS); each wavefront counts a
-// plane's hits with ballots over its rows, lane `it` keeps plane it's count,
-// and the block's counts meet in LDS before one atomic per plane.
+// Hypotheses and their inlier counts (segmenter.cpp:376-431).  Every workgroup
+// draws the index pairs and builds the 60 planes itself, one per lane of its
+// first wavefront, while the others' candidates are on their way: unless a
+// draw is rejected or repeats (about one frame in a hundred; then one lane
+// draws them all in order), pair `it` comes from values 2 it and 2 it + 1 of
+// the stream.  Every candidate scores all planes with the reference's float
+// expression; a wavefront counts a plane's hits with ballots over its rows,
+// lane `it` keeps plane it's count, and the workgroup's counts meet in LDS
+// before one atomic per plane.  With R = 1 candidate per thread more
+// workgroups share a frame (few frames), with 4 each plane is read once for
+// four rows.  Per frame with the serial draw in a launch of its own: 38 us,
+// now 9.
+template <int R>
 __global__ __launch_bounds__(256) void k_ransac_count(DevBuf d, Layout L) {
     __shared__ uint32_t acc[kRansacIters];
-    static_assert(kRansacIters <= kWave, "one lane per hypothesis holds its count");
+    __shared__ float4 plane[kRansacIters];
+    __shared__ uint2 pairs[kRansacIters];
+    __shared__ uint32_t usable;
+    static_assert(kRansacIters <= kWave, "one lane per hypothesis");
     const int f = blockIdx.y;
     const SegConst& s = d.frames[f].sc;
     const uint32_t n = d.fs[f * kFsCount + kFsCands];
-    const uint32_t base = blockIdx.x * (256u * kScoreRows);
-    if (n < 2 || base >= n) return;
-    if ((d.fs[f * kFsCount + kFsErr] & (kErrRansacSingle | kErrRngExhausted)) != 0) return;
+    const uint32_t base = blockIdx.x * (256u * R);
     const int tid = threadIdx.x;
     const int lane = lane_id();
-    if (tid < kRansacIters) acc[tid] = 0;
+    if (n < 2) {  // without candidates the reference returns (segmenter.cpp:353-356); with one it never ends
+        if (n == 1 && blockIdx.x == 0 && tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrRansacSingle);
+        return;
+    }
+    if (base >= n) return;
     const size_t ob = (size_t)f * L.N;
-    float x[kScoreRows], y[kScoreRows], z[kScoreRows];
-    bool act[kScoreRows];
+    float x[R], y[R], z[R];
+    bool act[R];
 #pragma unroll
-    for (int r = 0; r < kScoreRows; ++r) {
+    for (int r = 0; r < R; ++r) {
         const uint32_t t = base + r * 256u + tid;
         act[r] = t < n;
         x[r] = act[r] ? d.cx[ob + t] : 0.0f;
         y[r] = act[r] ? d.cy[ob + t] : 0.0f;
         z[r] = act[r] ? d.cz[ob + t] : 0.0f;
     }
-    const float4* hyp = reinterpret_cast<const float4*>(d.hyp) + (size_t)f * kRansacIters;
-    const uint32_t* valid = d.hyp_valid + f * kRansacIters;
+    if (tid < kRansacIters) acc[tid] = 0;
+    if (tid < kWave) {
+        const int it = min(lane, kRansacIters - 1);
+        const uint64_t pa = static_cast<uint64_t>(d.mt_raw[2 * it]) * n, pb = static_cast<uint64_t>(d.mt_raw[2 * it + 1]) * n;
+        uint2 pr = make_uint2(static_cast<uint32_t>(pa >> 32), static_cast<uint32_t>(pb >> 32));
+        bool ok = true;
+        // A product whose low word is below n may be rejected.
+        if (__ballot(static_cast<uint32_t>(pa) < n || static_cast<uint32_t>(pb) < n || pr.x == pr.y)) {
+            if (lane == 0) usable = draw_pairs(d.mt_raw, n, pairs) ? 1u : 0u;
+            wave_sync();
+            ok = usable != 0;
+            if (ok) pr = pairs[it];
+            if (!ok && lane == 0 && blockIdx.x == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrRngExhausted);
+        }
+        wave_sync();
+        if (lane == 0) usable = ok ? 1u : 0u;
+        if (ok && lane < kRansacIters) {
+            // Plane through the sensor's foot point and two candidates
+            // (segmenter.cpp:389-418).
+            const float p1x = 0.0f, p1y = 0.0f, p1z = s.neg_h;
+            const float p2x = d.cx[ob + pr.x], p2y = d.cy[ob + pr.x], p2z = d.cz[ob + pr.x];
+            const float p3x = d.cx[ob + pr.y], p3y = d.cy[ob + pr.y], p3z = d.cz[ob + pr.y];
+            float nx = ((p2y - p1y) * (p3z - p1z)) - ((p2z - p1z) * (p3y - p1y));
+            float ny = ((p2z - p1z) * (p3x - p1x)) - ((p2x - p1x) * (p3z - p1z));
+            float nz = ((p2x - p1x) * (p3y - p1y)) - ((p2y - p1y) * (p3x - p1x));
+            const float den2 = (nx * nx) + (ny * ny) + (nz * nz);
+            uint32_t valid = 0;
+            float pd = 0.0f;
+            if (!(den2 < 1.0e-5F)) {
+                const float norm = 1.0F / sqrtf(den2);
+                nz *= norm;
+                if (!(fabsf(nz) < s.cos_max)) {
+                    nx *= norm;
+                    ny *= norm;
+                    pd = (nx * p1x) + (ny * p1y) + (nz * p1z);
+                    valid = 1;
+                }
+            }
+            // A plane that is not valid scores nothing: NaN compares false.
+            plane[lane] = valid ? make_float4(nx, ny, nz, pd) : make_float4(0.0f, 0.0f, 0.0f, __builtin_nanf(""));
+            if (blockIdx.x == 0) {
+                reinterpret_cast<float4*>(d.hyp)[(size_t)f * kRansacIters + lane] = make_float4(nx, ny, nz, pd);
+                d.hyp_valid[f * kRansacIters + lane] = valid;
+            }
+        }
+    }
+    __syncthreads();
+    if (!usable) return;
     const float thr = s.thr;
     uint32_t mine = 0;
+#pragma unroll 4
     for (int it = 0; it < kRansacIters; ++it) {
-        if (!valid[it]) continue;
-        const float4 p = hyp[it];
+        const float4 p = plane[it];
         uint32_t c = 0;
 #pragma unroll
-        for (int r = 0; r < kScoreRows; ++r) {
+        for (int r = 0; r < R; ++r) {
             const float od = fabsf((p.x * x[r]) + (p.y * y[r]) + (p.z * z[r]) - p.w);
             c += static_cast<uint32_t>(__popcll(__ballot(act[r] && od < thr)));
         }
         mine += lane == it ? c : 0u;
     }
-    __syncthreads();
     if (lane < kRansacIters && mine) atomicAdd(&acc[lane], mine);
     __syncthreads();
-    if (tid < kRansacIters && valid[tid] && acc[tid]) atomicAdd(&d.hyp_count[f * kRansacIters + tid], acc[tid]);
+    if (tid < kRansacIters && acc[tid]) atomicAdd(&d.hyp_count[f * kRansacIters + tid], acc[tid]);
 }
 
-// Best hypothesis: strict `>` in iteration order, then the sign flip
-// (segmenter.cpp:433-453).
-__global__ void k_ransac_best(DevBuf d, Layout L) {
-    const int f = blockIdx.x * blockDim.x + threadIdx.x;
-    if (f >= L.B_active) return;
-    uint32_t* fs = d.fs + f * kFsCount;
-    if (fs[kFsCands] < 2 || (fs[kFsErr] & (kErrRansacSingle | kErrRngExhausted))) return;
-    uint32_t best = 0;
-    float a = 0.0f, b = 0.0f, c = 1.0f, dd = 0.0f;
-    for (int it = 0; it < kRansacIters; ++it) {
-        if (!d.hyp_valid[f * kRansacIters + it]) continue;
-        const uint32_t cnt = d.hyp_count[f * kRansacIters + it];
-        if (cnt > best) {
-            best = cnt;
-            const float* h = d.hyp + ((size_t)f * kRansacIters + it) * 4;
-            a = h[0];
-            b = h[1];
-            c = h[2];
-            dd = h[3];
-        }
+// The best hypothesis, by every wavefront that needs it: the largest count,
+// the first of equal ones (strict `>` in iteration order), then the sign flip
+// (segmenter.cpp:433-453).  Returns its count, 0 when none applies.
+__device__ __forceinline__ uint32_t best_plane(const DevBuf& d, int f, float4& plane) {
+    const uint32_t* fs = d.fs + f * kFsCount;
+    plane = make_float4(0.0f, 0.0f, 1.0f, 0.0f);
+    if (fs[kFsCands] < 2 || (fs[kFsErr] & (kErrRansacSingle | kErrRngExhausted))) return 0;
+    const int it = lane_id();
+    uint64_t key = 0;
+    if (it < kRansacIters && d.hyp_valid[f * kRansacIters + it])
+        key = static_cast<uint64_t>(d.hyp_count[f * kRansacIters + it]) << 6 | static_cast<uint64_t>(kWave - 1 - it);
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        const uint64_t k = __shfl_xor(key, o, kWave);
+        key = k > key ? k : key;
     }
-    if (best > 0 && c < 0) {
-        a = -a;
-        b = -b;
-        c = -c;
-        dd = -dd;
-    }
-    fs[kFsBest] = best;
-    fs[kFsApplied] = best > 0 ? 1u : 0u;
-    fs[kFsPlaneA] = f2u(a);
-    fs[kFsPlaneB] = f2u(b);
-    fs[kFsPlaneC] = f2u(c);
-    fs[kFsPlaneD] = f2u(dd);
+    const uint32_t best = static_cast<uint32_t>(key >> 6);
+    if (best == 0) return 0;
+    const int at = kWave - 1 - static_cast<int>(key & (kWave - 1));
+    plane = reinterpret_cast<const float4*>(d.hyp)[(size_t)f * kRansacIters + at];
+    if (plane.z < 0) plane = make_float4(-plane.x, -plane.y, -plane.z, -plane.w);
+    return best;
 }
 
 // Pixel states after RECM + RANSAC: the winner's label (segmenter.cpp:
 // 278-281 and 466-475), its index (cloud_mapping_indices_) and xyz.
-__global__ void k_pixel_label(DevBuf d, Layout L) {
+__global__ __launch_bounds__(256) void k_pixel_label(DevBuf d, Layout L) {
     const int f = blockIdx.y;
     const FrameDesc& fd = d.frames[f];
     const SegConst& s = fd.sc;
     const int p = blockIdx.x * blockDim.x + threadIdx.x;
-    if (p >= s.H * s.W) return;
-    const unsigned long long key = d.pix_key[fd.pix_off + p];
+    if (static_cast<int>(blockIdx.x * blockDim.x) >= s.H * s.W) return;
     const size_t po = fd.pix_off + p;
+    const unsigned long long key = p < s.H * s.W ? d.pix_key[po] : ~0ull;
+    float4 plane;
+    const uint32_t best = best_plane(d, f, plane);
+    if (p == 0 && d.fs[f * kFsCount + kFsCands] >= 2 &&
+        !(d.fs[f * kFsCount + kFsErr] & (kErrRansacSingle | kErrRngExhausted))) {
+        uint32_t* fs = d.fs + f * kFsCount;
+        fs[kFsBest] = best;
+        fs[kFsApplied] = best > 0 ? 1u : 0u;
+        fs[kFsPlaneA] = f2u(plane.x);
+        fs[kFsPlaneB] = f2u(plane.y);
+        fs[kFsPlaneC] = f2u(plane.z);
+        fs[kFsPlaneD] = f2u(plane.w);
+    }
+    if (p >= s.H * s.W) return;
     if (key == ~0ull) {
         d.state[po] = kEmpty;
         d.mapping[po] = -1;
@@ -812,10 +827,8 @@ __global__ void k_pixel_label(DevBuf d, Layout L) {
     const int cell = __float_as_int(pc.w);
     const float e = d.elev[(size_t)f * L.cell_stride + cell];
     uint8_t lab = (z >= e + s.thr) ? kObstacle : kGround;
-    const uint32_t* fs = d.fs + f * kFsCount;
-    if (fs[kFsApplied] && (cell % s.rings) < kRansacRadialBins) {
-        const float a = u2f(fs[kFsPlaneA]), b = u2f(fs[kFsPlaneB]), c = u2f(fs[kFsPlaneC]), dd = u2f(fs[kFsPlaneD]);
-        const float sd = (a * x) + (b * y) + (c * z) - dd;
+    if (best > 0 && (cell % s.rings) < kRansacRadialBins) {
+        const float sd = (plane.x * x) + (plane.y * y) + (plane.z * z) - plane.w;
         if (sd < s.thr) lab = kGround;
     }
     d.state[po] = lab;
@@ -837,24 +850,27 @@ void launch_segment_front(lp_context* c, int B) {
     else
         hipLaunchKernelGGL(k_project, dim3((L.N + wg - 1) / wg, B), dim3(wg), 0, st, d, L);
     stage_mark(c, "cells");
-    hipLaunchKernelGGL(k_cell_scan, dim3(B), dim3(1024), 0, st, d, L);
+    constexpr int kStartTile = kStartThreads * kStartItems;
+    hipLaunchKernelGGL(k_cell_start, dim3((L.cell_stride + kStartTile - 1) / kStartTile, B), dim3(kStartThreads), 0, st, d, L);
     hipLaunchKernelGGL(k_cell_fill, dim3(nb, B), dim3(256), 0, st, d, L);
     // About 8192 wavefronts in all, at least 64 and at most 4096 per frame.
     hipLaunchKernelGGL(k_cell_sort, dim3(std::min(1024, std::max(16, 2048 / B)), B), dim3(256), 0, st, d, L);
     // Cells beyond kSmallCell points are rare: about 1024 workgroups in all.
     hipLaunchKernelGGL(k_cell_sort_big, dim3(std::min(64, std::max(4, 1024 / B)), B), dim3(1024), 0, st, d, L);
     stage_mark(c, "recm");
-    hipLaunchKernelGGL(k_recm, dim3((L.cand_stride / kRansacRadialBins + kWave - 1) / kWave, B), dim3(kWave), 0, st, d,
-                       L);
+    hipLaunchKernelGGL(k_recm, dim3((L.cand_stride / kRansacRadialBins + kWave - 1) / kWave, B), dim3(kRecmThreads), 0,
+                       st, d, L);
     stage_mark(c, "ransac");
-    // 128 workgroups (512 wavefronts) per frame walk the slices x 4 near cells.
-    hipLaunchKernelGGL(k_cand_count, dim3(128, B), dim3(256), 0, st, d, L);
-    hipLaunchKernelGGL(k_cand_scan, dim3(B), dim3(1024), 0, st, d, L);
-    hipLaunchKernelGGL(k_cand_fill, dim3(128, B), dim3(256), 0, st, d, L);
-    hipLaunchKernelGGL(k_ransac_hyp, dim3(B), dim3(64), 0, st, d, L);
-    hipLaunchKernelGGL(k_ransac_count, dim3((L.N + 256 * kScoreRows - 1) / (256 * kScoreRows), B), dim3(256), 0, st,
-                       d, L);
-    hipLaunchKernelGGL(k_ransac_best, dim3((B + 63) / 64), dim3(64), 0, st, d, L);
+    // A wavefront per near cell (slices x 4, 1440 by default) for few frames,
+    // 512 wavefronts a frame on larger batches.
+    const int cand_grid = std::min(384, std::max(128, 1536 / B));
+    hipLaunchKernelGGL(k_cand_count, dim3(cand_grid, B), dim3(256), 0, st, d, L);
+    hipLaunchKernelGGL(k_cand_fill, dim3(cand_grid, B), dim3(256), 0, st, d, L);
+    // Up to eight frames leave room for a candidate per thread.
+    if (B <= 8)
+        hipLaunchKernelGGL(k_ransac_count<1>, dim3((L.N + 255) / 256, B), dim3(256), 0, st, d, L);
+    else
+        hipLaunchKernelGGL(k_ransac_count<4>, dim3((L.N + 1023) / 1024, B), dim3(256), 0, st, d, L);
     stage_mark(c, "pixels");
     hipLaunchKernelGGL(k_pixel_label, dim3((L.P + 255) / 256, B), dim3(256), 0, st, d, L);
 }
