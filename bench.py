@@ -79,7 +79,7 @@ def kernel_bytes_8d(kernel, n, p, n_obs, voxels, hull_vertices):
     their cluster labels, the voxel insert writes the hash, and the hull
     rounds read the hull inputs and produce the vertices."""
     return {"k_project": 14 * n, "k_pixel_label": 5 * p, "k_jcp_solve": 5 * p, "k_seg_labels": 4 * n,
-            "k_spherical": 12 * n_obs, "k_component_label": 4 * n_obs, "k_voxel_insert": 8 * voxels,
+            "k_obs_gather": 12 * n_obs, "k_cluster_label": 4 * n_obs, "k_voxel_insert": 8 * voxels,
             "k_hull_round": 8 * n_obs + 16 * hull_vertices}.get(kernel, 0)
 
 

@@ -371,6 +371,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.labels, B * N);
     go(x.obs_flag, B * N);
     go(x.obs_src, B * N);
+    go(x.obs_rows, B * static_cast<size_t>(L.obs_rows));
     go(x.ox, B * N);
     go(x.oy, B * N);
     go(x.oz, B * N);
@@ -415,11 +416,10 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.hslot, B * HC);
     go(x.vlist, B * N);
     go(x.vpar, B * N);
-    go(x.vnb, B * N * 13);
+    go(x.vnb, B * N * 8);
     go(x.vmin, B * N);
     go(x.vcnt, B * N);
     go(x.vlab, B * N);
-    go(x.cl_root, B * N);
     go(x.cl_size, B * N);
     go(x.cl_off, B * N);
     go(x.cl_cursor, B * N);
@@ -435,6 +435,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.hull_count, B * N);
     go(x.hull_off, B * N);
     go(x.hull_local, B * N);
+    x.vroots = x.hull_local;
     go(x.blk, B * L.blk_stride);
     go(x.fs, B * kFsCount);
     go(x.wq, kWqCounters);
@@ -777,6 +778,7 @@ int create_lane(const lp_capacity* cap, lp_context** out) {
     L.hash_cap = 1 << ceil_log2(static_cast<int64_t>(std::ceil(L.N / static_cast<double>(cap->hash_load_factor))));
     L.blk_stride = (std::max({L.N, L.P, L.hash_cap}) + 2047) / 2048 + 1;
     L.box_stride = L.N / 3 + 1024;
+    L.obs_rows = (L.N + 63) / 64;
     const size_t bytes = layout_bytes(L, nullptr, nullptr);
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&c->arena, bytes);

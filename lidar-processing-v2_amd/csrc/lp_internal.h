@@ -123,6 +123,7 @@ struct DevBuf {
     uint32_t* labels;
     uint32_t* obs_flag;      // scan scratch over points
     int32_t* obs_src;        // [frame stride N] input index of obstacle k
+    uint32_t* obs_rows;      // [frame][obs_rows] obstacles among every 64 points
     float *ox, *oy, *oz;     // obstacle xyz (frame stride N)
     float *sr, *sa, *se;     // spherical coords of obstacle points
     int32_t* vslot;          // hash slot of each obstacle point
@@ -162,12 +163,12 @@ struct DevBuf {
     // dense voxels (frame stride N)
     int32_t* vlist;          // dense id -> hash slot (insertion order)
     int32_t* vpar;           // union-find parent / component root (dense ids)
-    int32_t* vnb;            // [13][N] per frame: dense id of each forward neighbour voxel, -1 none
+    int32_t* vnb;            // [8][N] per frame: dense ids of the voxels to join with, ended by -1
     int32_t* vmin;           // per root: minimum obstacle index of the component
     uint32_t* vcnt;          // per root: points in the component
+    int32_t* vroots;         // = hull_local (free until the local ranks): the components' roots, in any order
     int32_t* vlab;           // per root: cluster label (components of at least min_size points)
     // clusters (frame stride N)
-    int32_t* cl_root;
     uint32_t* cl_size;
     uint32_t* cl_off;
     uint32_t* cl_cursor;
@@ -223,7 +224,7 @@ struct DevBuf {
 };
 
 // Work-queue counters of the persistent launches (lp_queue.h): 8 per site.
-constexpr int kWqCounters = 4 * 8;
+constexpr int kWqCounters = 3 * 8;
 
 constexpr bool kKdSearchDisabled = true;  // LP_NOISE_KDTREE rejected by lp_set_noise_search
 constexpr int kKdEntriesPerPoint = 8;
@@ -241,12 +242,12 @@ enum FsSlot : int {
     kFsObstacles,
     kFsMaxR, kFsMaxA, kFsMaxE,
     kFsVoxels,
+    kFsRoots,          // components
     kFsClusters,
     kFsHullTotal,
     kFsHullChunks,
     kFsHullInexact,    // predicates whose double evaluation had the wrong sign
     kFsHullRounded,    // clusters whose hull was redone with the reference's rounded predicate
-    kFsCcGlobal,       // 1: too many voxels for the LDS union-find
     kFsErr,
     kFsBoxes,          // clusters with a box
     kFsHullLarge,      // clusters listed for the workgroup local-rank launch
@@ -274,6 +275,7 @@ struct Layout {
     int32_t hash_cap;       // power of two
     int32_t blk_stride;     // scan block sums per frame
     int32_t box_stride;     // oriented boxes per frame (capacity)
+    int32_t obs_rows;       // runs of 64 points per frame
 };
 
 }  // namespace lp

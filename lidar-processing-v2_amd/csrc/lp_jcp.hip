@@ -601,6 +601,9 @@ __device__ __forceinline__ void seg_labels_tile(const DevBuf& d, const Layout& L
         }
     }
     d.labels[gi] = lab;
+    // Obstacles of every 64 points, for the split that follows.
+    const uint64_t obs = __ballot(lab == LP_LABEL_OBSTACLE);
+    if (lane_id() == 0) d.obs_rows[(size_t)f * L.obs_rows + i / kWave] = static_cast<uint32_t>(__popcll(obs));
     if (d.gnd_flag) d.gnd_flag[(size_t)f * L.N + i] = lab == LP_LABEL_GROUND ? 1u : 0u;
 }
 

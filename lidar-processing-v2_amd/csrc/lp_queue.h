@@ -18,7 +18,7 @@
 namespace lp {
 
 // Queues of one persistent launch site (8 counters each).
-enum WqSite : int { kWqProject = 0, kWqSegLabels, kWqSpherical, kWqVoxelInsert, kWqSites };
+enum WqSite : int { kWqProject = 0, kWqSegLabels, kWqVoxelInsert, kWqSites };
 static_assert(kWqCounters == kWqSites * 8, "one counter per XCD queue and site");
 constexpr int kPersistentWorkgroups = 1024;  // 256 CUs x 4
 

@@ -9,7 +9,7 @@ The knobs are the ones the library exposes at run time:
 * ``hash_load_factor``: worst-case load of the voxel and noise-cell hash
   tables; a smaller table is cleared and probed with fewer cache misses;
 * ``point_workgroup``: workgroup size (64, 128 or 256) of the per-point
-  kernels (projection, labels, spherical coordinates, voxel insert);
+  kernels (projection, labels, voxel insert);
 * ``mark_tile``: columns per workgroup (64, 128 or 256) of the JCP queue
   marking, whose workgroup stages a 5-row LDS tile of that width plus a
   two-pixel halo on each side;
