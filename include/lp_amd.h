@@ -315,16 +315,18 @@ int lp_set_label_clouds(lp_context* ctx, int32_t enable);
 int lp_set_vehicle_boxes(lp_context* ctx, int32_t enable);
 
 /* Launch form of the widest per-point kernels (projection, labels, voxel
- * insert): 0 = one workgroup per (tile, frame) of the capacity grid (the default); 1 = a persistent launch of a fixed
- * number of workgroups taking (frame, tile) items from per-XCD work queues
- * (a frame's items stay on one XCD), so frames of uneven sizes leave no idle
- * workgroups.  Outputs are identical in both forms.  No reference
- * counterpart (the reference processes one frame on the CPU). */
+ * insert): 0 = one workgroup per (tile, frame) of the capacity grid (the
+ * default); 1 = a persistent launch of a fixed number of workgroups taking
+ * (frame, tile) items from per-XCD work queues (a frame's items stay on one
+ * XCD), so frames of uneven sizes leave no idle workgroups.  Outputs are
+ * identical in both forms.  No reference counterpart (the reference processes
+ * one frame on the CPU). */
 int lp_set_persistent(lp_context* ctx, int32_t enable);
 /* Launch shape, tuned per device and workload (lidar_amd.autotune): the
- * workgroup size of the per-point kernels (projection, labels, voxel
- * insert) and the tile width in columns of the JCP queue marking (a 5-row LDS tile per
- * workgroup); each 64, 128 or 256 (default 256 and 256).  Outputs are identical under every shape. */
+ * workgroup size of the per-point kernels (projection, labels, voxel insert)
+ * and the tile width in columns of the JCP queue marking (a 5-row LDS tile per
+ * workgroup); each 64, 128 or 256 (default 256 and 256).  Outputs are identical
+ * under every shape. */
 int lp_set_launch_shape(lp_context* ctx, int32_t point_workgroup, int32_t mark_tile_width);
 
 /* Processes num_frames frames as one batch (CSR-packed on the device, one

@@ -13,6 +13,10 @@ int set_last_error(int code, const char* msg);
 // record layout) without staging: LP_OK or the error lp_batch_stage would give.
 int validate_frame(const lp_context* c, const lp_segmenter_config& cfg, const lp_cloud& cl);
 
+// Gives the idle contexts, up to four of them, streams on hardware queues of
+// their own, as far as the runtime's choice of queues allows.
+int spread_streams(const std::vector<lp_context*>& contexts);
+
 // Records a named stage boundary on the context stream when profiling.
 void stage_mark(lp_context* c, const char* name);
 
