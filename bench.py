@@ -23,10 +23,10 @@ import numpy as np  # noqa: E402
 
 METRIC = "frames/s + points/s at 64x2048 (batched vs plain GPU vs CPU); p50/p99 ms"
 # Profiled stages that consist of exactly one kernel launch (a name that
-# recurs, like the three hull rounds, is summed over its launches).
+# recurs is summed over its launches).
 SINGLE_KERNEL_STAGES = {"project": "k_project", "recm": "k_recm", "pixels": "k_pixel_label",
                         "jcp_slots": "k_jcp_slots", "jcp_solve": "k_jcp_solve", "labels": "k_seg_labels",
-                        "hull_round": "k_hull_round", "hull_big": "k_hull_big", "hull_ref": "k_hull_ref",
+                        "hull_round": "k_hull_round", "hull_merge": "k_hull_merge", "hull_big": "k_hull_big",
                         "hull_local": "k_hull_local"}
 # The noise filter's stages that are single kernels (radius rule search).
 NOISE_STAGES = {"noise_count": "k_noise_count", "noise_search": "k_noise_search"}

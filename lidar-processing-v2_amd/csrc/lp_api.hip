@@ -388,8 +388,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.cell_items, B * N);
     go(x.cell_zkey, B * N);
     x.hc_chunk_c = x.cell_items;
-    go(x.hull_large, B * N);
-    x.hc_chunk_b = reinterpret_cast<uint32_t*>(x.hull_large);
+    go(x.hc_chunk_b, B * N);
     x.hc_chunk_i = x.cell_zkey;
     go(x.zmin, B * C);
     go(x.elev, B * C);
@@ -430,7 +429,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.hcy, 2 * B * N);
     go(x.hci, 2 * B * N);
     go(x.hc_count, 2 * B * N);
-    go(x.hc_choff, B * N);
+    go(x.hc_open, B * N);
     go(x.hull_idx, B * N);
     go(x.hull_count, B * N);
     go(x.hull_off, B * N);
@@ -1587,7 +1586,7 @@ int lp_convex_hulls(lp_context* c, const double* x, const double* y, const int32
     if (total > 0 && (!x || !y)) return fail(LP_ERR_INVALID_ARGUMENT, "null coordinates");
     LP_HIP(hipSetDevice(c->device));
     c->L.B_active = 1;
-    LP_HIP(hipMemcpyAsync(c->d.hc_choff, offsets, (num_lists + 1) * sizeof(int32_t), hipMemcpyHostToDevice,
+    LP_HIP(hipMemcpyAsync(c->d.hc_open, offsets, (num_lists + 1) * sizeof(int32_t), hipMemcpyHostToDevice,
                           c->stream));
     if (total) {
         LP_HIP(hipMemcpyAsync(c->d.hcx, x, total * sizeof(double), hipMemcpyHostToDevice, c->stream));

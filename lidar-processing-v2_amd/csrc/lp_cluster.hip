@@ -734,7 +734,8 @@ void launch_cluster(lp_context* c, int B, bool from_split) {
     } else {
         hipLaunchKernelGGL(k_cluster_label<false>, dim3(nb, B), dim3(256), 0, st, d, L);
     }
-    launch_hash_reset(c, B, d.vlist, kFsVoxels);
+    // The hull stage clears the voxel table; here nothing follows.
+    if (!from_split) launch_hash_reset(c, B, d.vlist, kFsVoxels);
 }
 
 }  // namespace lp

@@ -20,6 +20,7 @@
 #include <algorithm>
 #include <cfloat>
 
+#include "lp_hash.h"
 #include "lp_kernels.h"
 
 namespace lp {
@@ -663,17 +664,17 @@ __device__ int sort_dedupe_chunk(double* X, double* Y, int32_t* I, uint16_t* P, 
     return nd;
 }
 
-// Chunk plan for round r, one 1024-thread workgroup per frame walking the
-// clusters in tiles with a running carry: a cluster that is not final yet
-// needs ceil(cnt / 256) chunks (one if it fits: that chunk's hull is final);
-// hc_choff receives the exclusive scan of the chunk counts, hc_chunk_c /
-// hc_chunk_i / hc_chunk_b each chunk's cluster, index, size and the cluster's
-// first candidate, and the frame's total goes to kFsHullChunks.  Round 0 also clears the hull count and flag,
-// and every round clears the next round's candidate counts.
+// Chunk plan, one 1024-thread workgroup per frame walking the clusters in
+// tiles with a running carry: a cluster needs ceil(cnt / 256) chunks (one if
+// it fits: that chunk's hull is final).  hc_chunk_c / hc_chunk_i / hc_chunk_b
+// receive each chunk's cluster, index and size, and the cluster's first
+// candidate, the frame's total goes to kFsHullChunks, and the clusters of more
+// than one chunk are listed in hc_open for the rounds after the first.  It also
+// clears the hull counts and flags and the second buffer's candidate counts.
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanItems = 4;
 
-__global__ __launch_bounds__(kPlanThreads) void k_hull_plan(DevBuf d, Layout L, int r) {
+__global__ __launch_bounds__(kPlanThreads) void k_hull_plan(DevBuf d, Layout L) {
     __shared__ uint32_t lds[kPlanThreads / kWave + 1];
     const int f = blockIdx.x;
     const int K = static_cast<int>(d.fs[f * kFsCount + kFsClusters]);
@@ -691,16 +692,12 @@ __global__ __launch_bounds__(kPlanThreads) void k_hull_plan(DevBuf d, Layout L, 
             v[q] = 0;
             cn[q] = 0;
             if (c < K) {
-                if (r == 0) {
-                    d.hull_count[ob + c] = 0;
-                    d.hull_flag[ob + c] = 0;
-                }
-                if (r == 0 || d.hull_count[ob + c] == 0) {
-                    const uint32_t cnt = d.hc_count[(r & 1) * BN + ob + c];
-                    v[q] = cnt <= static_cast<uint32_t>(kHullChunk) ? 1u : (cnt + kHullChunk - 1) / kHullChunk;
-                    cn[q] = cnt;
-                }
-                d.hc_count[((r + 1) & 1) * BN + ob + c] = 0;
+                d.hull_count[ob + c] = 0;
+                d.hull_flag[ob + c] = 0;
+                d.hc_count[BN + ob + c] = 0;
+                cn[q] = d.hc_count[ob + c];
+                v[q] = cn[q] <= static_cast<uint32_t>(kHullChunk) ? 1u : (cn[q] + kHullChunk - 1) / kHullChunk;
+                if (v[q] > 1) d.hc_open[ob + atomicAdd(&d.fs[f * kFsCount + kFsHullOpen], 1u)] = static_cast<uint32_t>(c);
                 local += v[q];
             }
         }
@@ -708,21 +705,18 @@ __global__ __launch_bounds__(kPlanThreads) void k_hull_plan(DevBuf d, Layout L, 
         uint32_t ex = block_exclusive_sum<kPlanThreads>(local, lds, &total) + carry;
 #pragma unroll
         for (int q = 0; q < kPlanItems; ++q) {
-            if (b + q < K) {
-                d.hc_choff[ob + b + q] = ex;
-                // The chunk map of each of the cluster's chunks, so a round's
-                // wavefront has its chunk's cluster, place and size with one
-                // round of loads.  A round has at most N chunks (a cluster's
-                // chunk count never exceeds its candidate count).
-                if (v[q]) {
-                    const uint32_t base = d.cl_off[ob + b + q];
-                    const uint32_t fin = cn[q] <= static_cast<uint32_t>(kHullChunk) ? 0x80000000u : 0u;
-                    for (uint32_t k = 0; k < v[q] && ex + k < static_cast<uint32_t>(L.N); ++k) {
-                        const uint32_t nk = min(cn[q] - k * kHullChunk, static_cast<uint32_t>(kHullChunk));
-                        d.hc_chunk_c[ob + ex + k] = static_cast<int32_t>(static_cast<uint32_t>(b + q) | fin);
-                        d.hc_chunk_i[ob + ex + k] = k | nk << 16;
-                        d.hc_chunk_b[ob + ex + k] = base;
-                    }
+            // The chunk map of each of the cluster's chunks, so a wavefront
+            // has its chunk's cluster, place and size with one round of
+            // loads.  There are at most N chunks (a cluster's chunk count
+            // never exceeds its candidate count).
+            if (v[q]) {
+                const uint32_t first = d.cl_off[ob + b + q];
+                const uint32_t fin = cn[q] <= static_cast<uint32_t>(kHullChunk) ? 0x80000000u : 0u;
+                for (uint32_t k = 0; k < v[q] && ex + k < static_cast<uint32_t>(L.N); ++k) {
+                    const uint32_t nk = min(cn[q] - k * kHullChunk, static_cast<uint32_t>(kHullChunk));
+                    d.hc_chunk_c[ob + ex + k] = static_cast<int32_t>(static_cast<uint32_t>(b + q) | fin);
+                    d.hc_chunk_i[ob + ex + k] = k | nk << 16;
+                    d.hc_chunk_b[ob + ex + k] = first;
                 }
             }
             ex += v[q];
@@ -732,253 +726,455 @@ __global__ __launch_bounds__(kPlanThreads) void k_hull_plan(DevBuf d, Layout L, 
     if (threadIdx.x == 0) d.fs[f * kFsCount + kFsHullChunks] = carry;
 }
 
-// Register budget for three wavefronts per SIMD (168 VGPRs, a few spills in
-// the cold paths): the chunks' sort and prune phases are VALU- and
+// One wavefront's chunk: its points, sorted order, lists and chains.
+struct ChunkLds {
+    double x[kHullChunk];
+    double y[kHullChunk];
+    int32_t i[kHullChunk];
+    uint16_t perm[kHullChunk];
+    uint16_t stk[2 * kHullChunk];
+    uint16_t lol[kHullChunk];
+    uint16_t upl[kHullChunk];
+    int nlo;
+    int nup;
+
+    // Vertex v of the hull: the lower chain, then the upper one without its ends.
+    __device__ __forceinline__ int vertex(int v) const { return v < nlo ? stk[v] : stk[kHullChunk + v - nlo + 1]; }
+};
+
+// The hull of the n <= 256 points at src of the candidate buffers, by one
+// wavefront, as two chains in LDS; returns its vertex count.
+__device__ __forceinline__ int chunk_hull(ChunkLds& s, const DevBuf& d, const Layout& L, int f, int c, size_t src, int n) {
+    const int lane = lane_id();
+    double* X = s.x;
+    double* Y = s.y;
+    int32_t* I = s.i;
+    uint16_t* P = s.perm;
+    uint16_t* S = s.stk;
+    for (int i = lane; i < n; i += kWave) {
+        X[i] = d.hcx[src + i];
+        Y[i] = d.hcy[src + i];
+        I[i] = d.hci[src + i];
+    }
+    wave_sync();
+    // Coordinates that are all floats (every obstacle point) take the
+    // register path: keys, cull, sort and duplicate drop in one pass.
+    // Other lists use the LDS forms below.
+    bool as_float = true;
+    for (int i = lane; i < n; i += kWave) {
+        const double x = X[i], y = Y[i];
+        as_float = as_float && static_cast<double>(static_cast<float>(x)) == x &&
+                   static_cast<double>(static_cast<float>(y)) == y;
+    }
+    as_float = __ballot(!as_float) == 0;
+    int ns = 0;
+    int ns_in = 0;
+    // Exact duplicates (same x and y) are adjacent after the sort.  A
+    // second copy of a point is never a hull vertex of a set with two or
+    // more distinct points (the reference's chain pops it: its turn is
+    // zero), so only the first copy stays; a list of one repeated point
+    // keeps two copies, the reference's result for it.  Vertical surfaces
+    // repeat one (x, y) once per beam, so this often shrinks a chunk
+    // several times over.  Fewer than three points are kept as they are.
+    if (as_float) {
+        if (n <= kWave)
+            ns = cull_sort_float_chunk<1>(X, Y, I, P, n, &ns_in);
+        else if (n <= 2 * kWave)
+            ns = cull_sort_float_chunk<2>(X, Y, I, P, n, &ns_in);
+        else
+            ns = cull_sort_float_chunk<4>(X, Y, I, P, n, &ns_in);
+    } else {
+    // Akl-Toussaint cull: points strictly inside the quadrilateral of the
+    // leftmost, lowest, rightmost and highest points (counter-clockwise
+    // along the hull boundary) are no hull vertices; exact tests only.
+    int ex[4] = {0, 0, 0, 0};
+    for (int i = lane; i < n; i += kWave) {
+        if (X[i] < X[ex[0]] || (X[i] == X[ex[0]] && i < ex[0])) ex[0] = i;
+        if (Y[i] < Y[ex[1]] || (Y[i] == Y[ex[1]] && i < ex[1])) ex[1] = i;
+        if (X[i] > X[ex[2]] || (X[i] == X[ex[2]] && i < ex[2])) ex[2] = i;
+        if (Y[i] > Y[ex[3]] || (Y[i] == Y[ex[3]] && i < ex[3])) ex[3] = i;
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        int c0 = __shfl_xor(ex[0], o, kWave), c1 = __shfl_xor(ex[1], o, kWave);
+        int c2 = __shfl_xor(ex[2], o, kWave), c3 = __shfl_xor(ex[3], o, kWave);
+        if (X[c0] < X[ex[0]] || (X[c0] == X[ex[0]] && c0 < ex[0])) ex[0] = c0;
+        if (Y[c1] < Y[ex[1]] || (Y[c1] == Y[ex[1]] && c1 < ex[1])) ex[1] = c1;
+        if (X[c2] > X[ex[2]] || (X[c2] == X[ex[2]] && c2 < ex[2])) ex[2] = c2;
+        if (Y[c3] > Y[ex[3]] || (Y[c3] == Y[ex[3]] && c3 < ex[3])) ex[3] = c3;
+    }
+    // The distinct extremes, in counter-clockwise order; repeated ones
+    // (e.g. the leftmost point is also the lowest) are dropped so no edge
+    // has zero length.  With fewer than three there is no interior.
+    int poly[4];
+    int npoly = 0;
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+        const int v = ex[e];
+        if (npoly == 0 || X[v] != X[poly[npoly - 1]] || Y[v] != Y[poly[npoly - 1]]) poly[npoly++] = v;
+    }
+    if (npoly > 1 && X[poly[npoly - 1]] == X[poly[0]] && Y[poly[npoly - 1]] == Y[poly[0]]) --npoly;
+    for (int i0 = 0; i0 < n; i0 += kWave) {
+        const int i = i0 + lane;
+        bool keep = false;
+        if (i < n) {
+            int dummy;
+            keep = true;
+            if (npoly >= 3) {
+                bool inside = true;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    if (e < npoly && inside) {
+                        const int a = poly[e], b = poly[e + 1 < npoly ? e + 1 : 0];
+                        inside = orient_exact(X[a], Y[a], X[b], Y[b], X[i], Y[i], &dummy) > 0;
+                    }
+                }
+                keep = !inside;
+            }
+        }
+        const uint64_t mask = __ballot(keep);
+        if (keep) P[ns + lanes_below(mask)] = static_cast<uint16_t>(i);
+        ns += static_cast<int>(__popcll(mask));
+    }
+    ns_in = ns;
+    int m = 1;
+    while (m < ns) m <<= 1;
+    for (int i = ns + lane; i < m; i += kWave) P[i] = static_cast<uint16_t>(n + i);  // padding sorts last
+    wave_sync();
+    // Bitonic sort of the permutation; padding entries (>= n) sort last.
+    for (int k = 2; k <= m; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int q = lane; q < (m >> 1); q += kWave) {
+                const int a = ((q & ~(j - 1)) << 1) | (q & (j - 1));
+                const int b = a + j;
+                const int pa = P[a], pb = P[b];
+                const bool gt = (pa >= n) ? (pb < n || pa > pb) : (pb < n && pt_less(X, Y, I, pb, pa));
+                const bool up = (a & k) == 0;
+                if (gt == up) {
+                    P[a] = static_cast<uint16_t>(pb);
+                    P[b] = static_cast<uint16_t>(pa);
+                }
+            }
+            wave_sync();
+        }
+    }
+    if (ns >= 3) {
+        int nd = 0;
+        for (int i0 = 0; i0 < ns; i0 += kWave) {
+            const int i = i0 + lane;
+            bool keep = false;
+            int p = 0;
+            if (i < ns) {
+                p = P[i];
+                const int q = P[i > 0 ? i - 1 : 0];
+                keep = i == 0 || X[p] != X[q] || Y[p] != Y[q];
+            }
+            const uint64_t mk = __ballot(keep);
+            if (keep) S[nd + lanes_below(mk)] = static_cast<uint16_t>(p);
+            nd += static_cast<int>(__popcll(mk));
+        }
+        if (nd == 1) {
+            if (lane == 0) S[1] = P[1];
+            nd = 2;
+        }
+        wave_sync();
+        for (int i = lane; i < nd; i += kWave) P[i] = S[i];
+        wave_sync();
+        ns = nd;
+    }
+    }
+    // Lane 0 the lower chain, lane 1 the upper one (in S + kHullChunk);
+    // vertex i of the hull is lower[i] for i < kl, then upper[i - kl + 1].
+    // Fewer than three input points take the reference's short path; two
+    // distinct points left after the duplicates go through the chain,
+    // which returns them in (x, y) order.
+    if (ns_in < 3) {
+        if (lane == 0) {
+            uint32_t inexact = 0;
+            s.nlo = chain_hull(X, Y, I, P, ns, S, &inexact);
+            s.nup = 2;
+        }
+    } else {
+        int cl, cu;
+        split_by_chord(X, Y, P, ns, s.lol, s.upl, &cl, &cu);
+        wave_sync();
+        bool dl, du;
+        uint32_t inexact = 0;
+        cl = prune_chain(X, Y, s.lol, S, cl, 1, kPrunePasses, &dl, &inexact);
+        cu = prune_chain(X, Y, s.upl, S + kHullChunk, cu, -1, kPrunePasses, &du, &inexact);
+        if (dl && du) {
+            // Both halves are already chains: lower as listed, upper
+            // from the right end back.
+            for (int i = lane; i < cl; i += kWave) S[i] = s.lol[i];
+            for (int i = lane; i < cu; i += kWave) S[kHullChunk + i] = s.upl[cu - 1 - i];
+            if (lane == 0) {
+                s.nlo = cl;
+                s.nup = cu;
+            }
+        } else if (max(cl, cu) > kMergeChain) {
+            // Long halves: the wavefront's divide-and-conquer chain.
+            const int kl2 = merge_half_chain(X, Y, s.lol, cl, false, S, &inexact);
+            const int ku2 = merge_half_chain(X, Y, s.upl, cu, true, S + kHullChunk, &inexact);
+            if (lane == 0) {
+                s.nlo = kl2;
+                s.nup = ku2;
+            }
+        } else if (lane < 2) {
+            // One call with per-lane arguments, so the two chains run in
+            // lock-step instead of one after the other.
+            const int len = half_chain(X, Y, lane == 0 ? s.lol : s.upl, lane == 0 ? cl : cu, lane == 1,
+                                       lane == 1 ? S + kHullChunk : S, &inexact);
+            if (lane == 0)
+                s.nlo = len;
+            else
+                s.nup = len;
+        }
+        inexact = wave_sum(inexact);
+        if (lane == 0 && inexact) {
+            atomicAdd(&d.fs[f * kFsCount + kFsHullInexact], inexact);
+            atomicOr(&d.hull_flag[(size_t)f * L.N + c], 1u);
+        }
+    }
+    wave_sync();
+    return s.nlo + s.nup - 2;
+}
+
+// A chunk's hull as the cluster's result, or added to the cluster's candidates
+// in the buffer at dst, of which `count` says how many there are.
+__device__ __forceinline__ void put_hull(const ChunkLds& s, const DevBuf& d, size_t ob, int c, uint32_t base, int kk) {
+    const int lane = lane_id();
+    for (int i = lane; i < kk; i += kWave) d.hull_idx[ob + base + i] = s.i[s.vertex(i)];
+    if (lane == 0) d.hull_count[ob + c] = static_cast<uint32_t>(kk);
+}
+
+__device__ __forceinline__ void put_candidates(const ChunkLds& s, const DevBuf& d, size_t dst, uint32_t* count, int kk) {
+    const int lane = lane_id();
+    uint32_t pos = 0;
+    if (lane == 0) pos = atomicAdd(count, static_cast<uint32_t>(kk));
+    pos = __shfl(pos, 0, kWave);
+    for (int i = lane; i < kk; i += kWave) {
+        const int v = s.vertex(i);
+        d.hcx[dst + pos + i] = s.x[v];
+        d.hcy[dst + pos + i] = s.y[v];
+        d.hci[dst + pos + i] = s.i[v];
+    }
+}
+
+// The first round: all chunks of all clusters, a wavefront each.
+// Register budget for three wavefronts per SIMD (168 VGPRs): the chunks' sort and prune phases are VALU- and
 // LDS-latency-bound, and a third wavefront hides more of it than two.
-__global__ __launch_bounds__(256, 3) void k_hull_round(DevBuf d, Layout L, int r) {
-    __shared__ double sx[kWavesPerBlock][kHullChunk];
-    __shared__ double sy[kWavesPerBlock][kHullChunk];
-    __shared__ int32_t si[kWavesPerBlock][kHullChunk];
-    __shared__ uint16_t perm[kWavesPerBlock][kHullChunk];
-    __shared__ uint16_t stk[kWavesPerBlock][2 * kHullChunk];
-    __shared__ uint16_t lol[kWavesPerBlock][kHullChunk];
-    __shared__ uint16_t upl[kWavesPerBlock][kHullChunk];
-    __shared__ int nlo[kWavesPerBlock];
-    __shared__ int nup[kWavesPerBlock];
+__global__ __launch_bounds__(256, 3) void k_hull_round(DevBuf d, Layout L) {
+    __shared__ ChunkLds lds[kWavesPerBlock];
     int tile, f;
     xcd_tile_frame(tile, f);
     const uint32_t total = min(d.fs[f * kFsCount + kFsHullChunks], static_cast<uint32_t>(L.N));
     const int w = threadIdx.x / kWave;
-    const int lane = lane_id();
     const size_t ob = (size_t)f * L.N;
     const size_t BN = (size_t)L.B * L.N;
-    double* X = sx[w];
-    double* Y = sy[w];
-    int32_t* I = si[w];
-    uint16_t* P = perm[w];
-    uint16_t* S = stk[w];
-    const size_t in_b = (size_t)(r & 1) * BN;
-    const size_t out_b = (size_t)((r + 1) & 1) * BN;
     for (uint32_t t = tile * kWavesPerBlock + w; t < total; t += gridDim.x * kWavesPerBlock) {
         const uint32_t cw = static_cast<uint32_t>(d.hc_chunk_c[ob + t]);
         const uint32_t iw = d.hc_chunk_i[ob + t];
         const uint32_t base = d.hc_chunk_b[ob + t];
         const int c = static_cast<int>(cw & 0x7fffffffu);
-        const bool final_chunk = (cw >> 31) != 0;
         const uint32_t lo = (iw & 0xffffu) * kHullChunk;
-        const int n = static_cast<int>(iw >> 16);
-        for (int i = lane; i < n; i += kWave) {
-            const size_t src = in_b + ob + base + lo + i;
-            X[i] = d.hcx[src];
-            Y[i] = d.hcy[src];
-            I[i] = d.hci[src];
-        }
-        wave_sync();
-        // Coordinates that are all floats (every obstacle point) take the
-        // register path: keys, cull, sort and duplicate drop in one pass.
-        // Other lists use the LDS forms below.
-        bool as_float = true;
-        for (int i = lane; i < n; i += kWave) {
-            const double x = X[i], y = Y[i];
-            as_float = as_float && static_cast<double>(static_cast<float>(x)) == x &&
-                       static_cast<double>(static_cast<float>(y)) == y;
-        }
-        as_float = __ballot(!as_float) == 0;
-        int ns = 0;
-        int ns_in = 0;
-        // Exact duplicates (same x and y) are adjacent after the sort.  A
-        // second copy of a point is never a hull vertex of a set with two or
-        // more distinct points (the reference's chain pops it: its turn is
-        // zero), so only the first copy stays; a list of one repeated point
-        // keeps two copies, the reference's result for it.  Vertical surfaces
-        // repeat one (x, y) once per beam, so this often shrinks a chunk
-        // several times over.  Fewer than three points are kept as they are.
-        if (as_float) {
-            if (n <= kWave)
-                ns = cull_sort_float_chunk<1>(X, Y, I, P, n, &ns_in);
-            else if (n <= 2 * kWave)
-                ns = cull_sort_float_chunk<2>(X, Y, I, P, n, &ns_in);
-            else
-                ns = cull_sort_float_chunk<4>(X, Y, I, P, n, &ns_in);
-        } else {
-        // Akl-Toussaint cull: points strictly inside the quadrilateral of the
-        // leftmost, lowest, rightmost and highest points (counter-clockwise
-        // along the hull boundary) are no hull vertices; exact tests only.
-        int ex[4] = {0, 0, 0, 0};
-        for (int i = lane; i < n; i += kWave) {
-            if (X[i] < X[ex[0]] || (X[i] == X[ex[0]] && i < ex[0])) ex[0] = i;
-            if (Y[i] < Y[ex[1]] || (Y[i] == Y[ex[1]] && i < ex[1])) ex[1] = i;
-            if (X[i] > X[ex[2]] || (X[i] == X[ex[2]] && i < ex[2])) ex[2] = i;
-            if (Y[i] > Y[ex[3]] || (Y[i] == Y[ex[3]] && i < ex[3])) ex[3] = i;
-        }
-#pragma unroll
-        for (int o = kWave / 2; o > 0; o >>= 1) {
-            int c0 = __shfl_xor(ex[0], o, kWave), c1 = __shfl_xor(ex[1], o, kWave);
-            int c2 = __shfl_xor(ex[2], o, kWave), c3 = __shfl_xor(ex[3], o, kWave);
-            if (X[c0] < X[ex[0]] || (X[c0] == X[ex[0]] && c0 < ex[0])) ex[0] = c0;
-            if (Y[c1] < Y[ex[1]] || (Y[c1] == Y[ex[1]] && c1 < ex[1])) ex[1] = c1;
-            if (X[c2] > X[ex[2]] || (X[c2] == X[ex[2]] && c2 < ex[2])) ex[2] = c2;
-            if (Y[c3] > Y[ex[3]] || (Y[c3] == Y[ex[3]] && c3 < ex[3])) ex[3] = c3;
-        }
-        // The distinct extremes, in counter-clockwise order; repeated ones
-        // (e.g. the leftmost point is also the lowest) are dropped so no edge
-        // has zero length.  With fewer than three there is no interior.
-        int poly[4];
-        int npoly = 0;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            const int v = ex[e];
-            if (npoly == 0 || X[v] != X[poly[npoly - 1]] || Y[v] != Y[poly[npoly - 1]]) poly[npoly++] = v;
-        }
-        if (npoly > 1 && X[poly[npoly - 1]] == X[poly[0]] && Y[poly[npoly - 1]] == Y[poly[0]]) --npoly;
-        for (int i0 = 0; i0 < n; i0 += kWave) {
-            const int i = i0 + lane;
-            bool keep = false;
-            if (i < n) {
-                int dummy;
-                keep = true;
-                if (npoly >= 3) {
-                    bool inside = true;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (e < npoly && inside) {
-                            const int a = poly[e], b = poly[e + 1 < npoly ? e + 1 : 0];
-                            inside = orient_exact(X[a], Y[a], X[b], Y[b], X[i], Y[i], &dummy) > 0;
-                        }
-                    }
-                    keep = !inside;
-                }
-            }
-            const uint64_t mask = __ballot(keep);
-            if (keep) P[ns + lanes_below(mask)] = static_cast<uint16_t>(i);
-            ns += static_cast<int>(__popcll(mask));
-        }
-        ns_in = ns;
-        int m = 1;
-        while (m < ns) m <<= 1;
-        for (int i = ns + lane; i < m; i += kWave) P[i] = static_cast<uint16_t>(n + i);  // padding sorts last
-        wave_sync();
-        // Bitonic sort of the permutation; padding entries (>= n) sort last.
-        for (int k = 2; k <= m; k <<= 1) {
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int q = lane; q < (m >> 1); q += kWave) {
-                    const int a = ((q & ~(j - 1)) << 1) | (q & (j - 1));
-                    const int b = a + j;
-                    const int pa = P[a], pb = P[b];
-                    const bool gt = (pa >= n) ? (pb < n || pa > pb) : (pb < n && pt_less(X, Y, I, pb, pa));
-                    const bool up = (a & k) == 0;
-                    if (gt == up) {
-                        P[a] = static_cast<uint16_t>(pb);
-                        P[b] = static_cast<uint16_t>(pa);
-                    }
-                }
-                wave_sync();
-            }
-        }
-        if (ns >= 3) {
-            int nd = 0;
-            for (int i0 = 0; i0 < ns; i0 += kWave) {
-                const int i = i0 + lane;
-                bool keep = false;
-                int p = 0;
-                if (i < ns) {
-                    p = P[i];
-                    const int q = P[i > 0 ? i - 1 : 0];
-                    keep = i == 0 || X[p] != X[q] || Y[p] != Y[q];
-                }
-                const uint64_t mk = __ballot(keep);
-                if (keep) S[nd + lanes_below(mk)] = static_cast<uint16_t>(p);
-                nd += static_cast<int>(__popcll(mk));
-            }
-            if (nd == 1) {
-                if (lane == 0) S[1] = P[1];
-                nd = 2;
-            }
-            wave_sync();
-            for (int i = lane; i < nd; i += kWave) P[i] = S[i];
-            wave_sync();
-            ns = nd;
-        }
-        }
-        // Lane 0 the lower chain, lane 1 the upper one (in S + kHullChunk);
-        // vertex i of the hull is lower[i] for i < kl, then upper[i - kl + 1].
-        // Fewer than three input points take the reference's short path; two
-        // distinct points left after the duplicates go through the chain,
-        // which returns them in (x, y) order.
-        if (ns_in < 3) {
-            if (lane == 0) {
-                uint32_t inexact = 0;
-                nlo[w] = chain_hull(X, Y, I, P, ns, S, &inexact);
-                nup[w] = 2;
-            }
-        } else {
-            int cl, cu;
-            split_by_chord(X, Y, P, ns, lol[w], upl[w], &cl, &cu);
-            wave_sync();
-            bool dl, du;
-            uint32_t inexact = 0;
-            cl = prune_chain(X, Y, lol[w], S, cl, 1, kPrunePasses, &dl, &inexact);
-            cu = prune_chain(X, Y, upl[w], S + kHullChunk, cu, -1, kPrunePasses, &du, &inexact);
-            if (dl && du) {
-                // Both halves are already chains: lower as listed, upper
-                // from the right end back.
-                for (int i = lane; i < cl; i += kWave) S[i] = lol[w][i];
-                for (int i = lane; i < cu; i += kWave) S[kHullChunk + i] = upl[w][cu - 1 - i];
-                if (lane == 0) {
-                    nlo[w] = cl;
-                    nup[w] = cu;
-                }
-            } else if (max(cl, cu) > kMergeChain) {
-                // Long halves: the wavefront's divide-and-conquer chain.
-                const int kl2 = merge_half_chain(X, Y, lol[w], cl, false, S, &inexact);
-                const int ku2 = merge_half_chain(X, Y, upl[w], cu, true, S + kHullChunk, &inexact);
-                if (lane == 0) {
-                    nlo[w] = kl2;
-                    nup[w] = ku2;
-                }
-            } else if (lane < 2) {
-                // One call with per-lane arguments, so the two chains run in
-                // lock-step instead of one after the other.
-                const int len = half_chain(X, Y, lane == 0 ? lol[w] : upl[w], lane == 0 ? cl : cu, lane == 1,
-                                           lane == 1 ? S + kHullChunk : S, &inexact);
-                if (lane == 0)
-                    nlo[w] = len;
-                else
-                    nup[w] = len;
-            }
-            inexact = wave_sum(inexact);
-            if (lane == 0 && inexact) {
-                atomicAdd(&d.fs[f * kFsCount + kFsHullInexact], inexact);
-                atomicOr(&d.hull_flag[ob + c], 1u);
-            }
-        }
-        wave_sync();
-        const int kl = nlo[w];
-        const int kk = kl + nup[w] - 2;
-        auto vert = [&](int i) -> int { return i < kl ? S[i] : S[kHullChunk + i - kl + 1]; };
-        if (final_chunk) {
-            for (int i = lane; i < kk; i += kWave) d.hull_idx[ob + base + i] = I[vert(i)];
-            if (lane == 0) d.hull_count[ob + c] = static_cast<uint32_t>(kk);
-        } else {
-            uint32_t pos = 0;
-            if (lane == 0) pos = atomicAdd(&d.hc_count[out_b + ob + c], static_cast<uint32_t>(kk));
-            pos = __shfl(pos, 0, kWave);
-            for (int i = lane; i < kk; i += kWave) {
-                const size_t dst = out_b + ob + base + pos + i;
-                const int v = vert(i);
-                d.hcx[dst] = X[v];
-                d.hcy[dst] = Y[v];
-                d.hci[dst] = I[v];
-            }
-        }
+        const int kk = chunk_hull(lds[w], d, L, f, c, ob + base + lo, static_cast<int>(iw >> 16));
+        if (cw >> 31)
+            put_hull(lds[w], d, ob, c, base, kk);
+        else
+            put_candidates(lds[w], d, BN + ob + base, &d.hc_count[BN + ob + c], kk);
         wave_sync();
     }
+}
+
+constexpr int kResetTiles = 16;
+
+// The rounds after the first, a workgroup for each cluster of more than one
+// chunk: its wavefronts take the chunks of its candidates, and the round's
+// vertices are the next round's candidates.  A plan and a launch per round,
+// over chunks of all clusters, kept more wavefronts busy but waited for the
+// slowest chunk of the frame and for the plan each time (two rounds and the
+// table of one 64x2048 frame 39 -> 21 us; eight 128x2048 frames at a time 129
+// -> 101 us).  512 threads for few frames: with 256 the clusters of more than four chunks take
+// their chunks in turns (the eight frames 120 us), 1024 leave one workgroup to
+// a CU (one frame 32 us).  Workgroups from `tiles` on clear the voxel table's
+// used slots, which no later kernel reads.
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_hull_merge(DevBuf d, Layout L, int tiles) {
+    __shared__ ChunkLds lds[kThreads / kWave];
+    __shared__ uint32_t next;
+    int tile, f;
+    xcd_tile_frame(tile, f);
+    if (tile >= tiles) {
+        reset_slots(d, L, f, d.vlist, kFsVoxels, (tile - tiles) * kThreads + static_cast<int>(threadIdx.x),
+                    (static_cast<int>(gridDim.x) - tiles) * kThreads);
+        return;
+    }
+    const uint32_t open = d.fs[f * kFsCount + kFsHullOpen];
+    const int w = threadIdx.x / kWave;
+    const size_t ob = (size_t)f * L.N;
+    const size_t BN = (size_t)L.B * L.N;
+    for (uint32_t j = tile; j < open; j += tiles) {
+        const int c = static_cast<int>(d.hc_open[ob + j]);
+        const uint32_t base = d.cl_off[ob + c];
+        uint32_t cnt = d.hc_count[BN + ob + c];
+        bool final_chunk = false;
+        for (int r = 1; r < kHullRounds && !final_chunk; ++r) {
+            const size_t in = (size_t)(r & 1) * BN + ob + base, out = (size_t)((r + 1) & 1) * BN + ob + base;
+            final_chunk = cnt <= static_cast<uint32_t>(kHullChunk);
+            if (threadIdx.x == 0) next = 0;
+            __syncthreads();
+            for (uint32_t lo = w * kHullChunk; lo < cnt; lo += kThreads / kWave * kHullChunk) {
+                const int n = static_cast<int>(min(cnt - lo, static_cast<uint32_t>(kHullChunk)));
+                const int kk = chunk_hull(lds[w], d, L, f, c, in + lo, n);
+                if (final_chunk)
+                    put_hull(lds[w], d, ob, c, base, kk);
+                else
+                    put_candidates(lds[w], d, out, &next, kk);
+                wave_sync();
+            }
+            __syncthreads();
+            cnt = next;
+            __syncthreads();
+        }
+        // Left to k_hull_big, which reads the buffer the last round wrote.
+        if (!final_chunk && threadIdx.x == 0) d.hc_count[(size_t)(kHullRounds & 1) * BN + ob + c] = cnt;
+    }
+}
+
+// Coordinates of member m of the cluster at `base`: the obstacle point, or
+// for standalone lists the staged (x, y) pair.
+__device__ __forceinline__ void member_xy(const DevBuf& d, const double2* list_xy, size_t ob, uint32_t base, int32_t m,
+                                          double& x, double& y) {
+    if (list_xy) {
+        x = list_xy[base + m].x;
+        y = list_xy[base + m].y;
+    } else {
+        x = d.ox[ob + m];
+        y = d.oy[ob + m];
+    }
+}
+
+// Clusters where some orientation test's double value had another sign than
+// the exact one: the chunked, culled hull above is the exact hull, which the
+// reference's rounded predicate need not produce.  Such a cluster is redone
+// as polygonizer.cpp:33-91 computes it: all its points sorted by (x, y), then
+// Andrew's chain popping while the double expression
+// (p2.x-p1.x)*(p3.y-p1.y) - (p2.y-p1.y)*(p3.x-p1.x) <= 0, evaluated without
+// contraction.  One workgroup per flagged cluster; the points are sorted in
+// the first candidate buffer (free after the chunk hulls) by an ascending-only
+// bitonic network whose padding positions never move, and the lower and
+// upper chains run on lanes 0 and 1 with their stacks in the second buffer.
+// Exact duplicates may be ordered either way (their coordinates agree);
+// distinct x closer than DBL_EPSILON, where the reference's comparator
+// treats x as equal and is not an ordering, are reported as an error.
+__device__ __forceinline__ bool ref_ccw_or_collinear(double ax, double ay, double bx, double by, double cx,
+                                                     double cy) {
+    return (bx - ax) * (cy - ay) - (by - ay) * (cx - ax) <= 0;
+}
+
+__device__ __forceinline__ bool rec_less(const double* X, const double* Y, const int32_t* I, int a, int b) {
+    if (X[a] != X[b]) return X[a] < X[b];
+    if (Y[a] != Y[b]) return Y[a] < Y[b];
+    return I[a] < I[b];
+}
+
+__device__ void ref_hull(const DevBuf& d, const Layout& L, const double2* list_xy, int f, int c, int* nlo, int* nup) {
+    const int tid = threadIdx.x;
+    const size_t ob = (size_t)f * L.N;
+    const size_t BN = (size_t)L.B * L.N;
+    const int n = static_cast<int>(d.cl_size[ob + c]);
+    if (n < 3) return;
+    const uint32_t base = d.cl_off[ob + c];
+    double* X = d.hcx + ob + base;
+    double* Y = d.hcy + ob + base;
+    int32_t* I = d.hci + ob + base;
+    const int32_t* members = d.cl_members + ob + base;
+    for (int i = tid; i < n; i += blockDim.x) {
+        const int32_t m = members[i];
+        double x, y;
+        member_xy(d, list_xy, ob, base, m, x, y);
+        X[i] = x;
+        Y[i] = y;
+        I[i] = m;
+    }
+    __syncthreads();
+    int m2 = 1;
+    while (m2 < n) m2 <<= 1;
+    for (int k = 2; k <= m2; k <<= 1) {
+        for (int j = k >> 1; j > 0; j >>= 1) {
+            for (int q = tid; q < (m2 >> 1); q += blockDim.x) {
+                int a, b;
+                if (j == (k >> 1)) {
+                    // First step of a merge: mirror pairs inside each block of k.
+                    const int blk = q / j, t = q % j;
+                    a = blk * k + t;
+                    b = blk * k + k - 1 - t;
+                } else {
+                    a = ((q & ~(j - 1)) << 1) | (q & (j - 1));
+                    b = a + j;
+                }
+                if (b < n && rec_less(X, Y, I, b, a)) {
+                    const double tx = X[a], ty = Y[a];
+                    const int32_t ti = I[a];
+                    X[a] = X[b];
+                    Y[a] = Y[b];
+                    I[a] = I[b];
+                    X[b] = tx;
+                    Y[b] = ty;
+                    I[b] = ti;
+                }
+            }
+            __syncthreads();
+        }
+    }
+    for (int i = 1 + tid; i < n; i += blockDim.x)
+        if (X[i] != X[i - 1] && fabs(X[i] - X[i - 1]) < DBL_EPSILON)
+            atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullFuzzyOrder);
+    // Stacks of sorted positions: lower in [0, n), upper in [n, 2n) of
+    // the second buffer's doubles viewed as int32 (2n entries fit).
+    int32_t* SL = reinterpret_cast<int32_t*>(d.hcx + BN + ob + base);
+    int32_t* SU = SL + n;
+    if (tid == 0) {
+        int k = 0;
+        for (int i = 0; i < n; ++i) {
+            while (k > 1 && ref_ccw_or_collinear(X[SL[k - 2]], Y[SL[k - 2]], X[SL[k - 1]], Y[SL[k - 1]], X[i], Y[i]))
+                --k;
+            SL[k++] = i;
+        }
+        *nlo = k;
+    } else if (tid == 1) {
+        // The reference's upper loop continues on the lower stack with
+        // t = k + 1; it never pops below the last point, so it is the
+        // same chain started from that point.
+        int k = 0;
+        SU[k++] = n - 1;
+        for (int i = n - 2; i >= 0; --i) {
+            while (k > 1 && ref_ccw_or_collinear(X[SU[k - 2]], Y[SU[k - 2]], X[SU[k - 1]], Y[SU[k - 1]], X[i], Y[i]))
+                --k;
+            SU[k++] = i;
+        }
+        *nup = k;
+    }
+    __syncthreads();
+    const int kl = *nlo;
+    const int kk = kl + *nup - 2;  // indices.resize(k - 1)
+    if (kk > n) {
+        if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullCapacity);
+    } else {
+        for (int i = tid; i < kk; i += blockDim.x) d.hull_idx[ob + base + i] = I[i < kl ? SL[i] : SU[i - kl + 1]];
+        if (tid == 0) {
+            d.hull_count[ob + c] = static_cast<uint32_t>(kk);
+            atomicAdd(&d.fs[f * kFsCount + kFsHullRounded], 1u);
+        }
+    }
+    __syncthreads();
 }
 
 // Clusters whose candidates still exceed one chunk after the rounds (hulls
 // with hundreds of vertices): one workgroup sorts up to kHullBig candidates
 // in LDS and chains them.
-__global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, int r_in) {
+// The same workgroups then redo the flagged clusters (ref_hull).
+__global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, const double2* list_xy) {
     __shared__ double X[kHullBig];
     __shared__ double Y[kHullBig];
     __shared__ int32_t I[kHullBig];
@@ -995,6 +1191,7 @@ __global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, int r_in)
     const int tid = threadIdx.x;
     const size_t ob = (size_t)f * L.N;
     const size_t BN = (size_t)L.B * L.N;
+    constexpr int r_in = kHullRounds;
     const size_t in_b = (size_t)(r_in & 1) * BN;
     // Workgroup x takes the clusters c = x (mod gridDim.x): its threads test
     // 1024 of them at once and list those without a hull yet.
@@ -1132,140 +1329,15 @@ __global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, int r_in)
         }
         __syncthreads();
     }
-}
-
-// Coordinates of member m of the cluster at `base`: the obstacle point, or
-// for standalone lists the staged (x, y) pair.
-__device__ __forceinline__ void member_xy(const DevBuf& d, const double2* list_xy, size_t ob, uint32_t base, int32_t m,
-                                          double& x, double& y) {
-    if (list_xy) {
-        x = list_xy[base + m].x;
-        y = list_xy[base + m].y;
-    } else {
-        x = d.ox[ob + m];
-        y = d.oy[ob + m];
-    }
-}
-
-// Clusters where some orientation test's double value had another sign than
-// the exact one: the chunked, culled hull above is the exact hull, which the
-// reference's rounded predicate need not produce.  Such a cluster is redone
-// as polygonizer.cpp:33-91 computes it: all its points sorted by (x, y), then
-// Andrew's chain popping while the double expression
-// (p2.x-p1.x)*(p3.y-p1.y) - (p2.y-p1.y)*(p3.x-p1.x) <= 0, evaluated without
-// contraction.  One workgroup per flagged cluster; the points are sorted in
-// the first candidate buffer (free after k_hull_big) by an ascending-only
-// bitonic network whose padding positions never move, and the lower and
-// upper chains run on lanes 0 and 1 with their stacks in the second buffer.
-// Exact duplicates may be ordered either way (their coordinates agree);
-// distinct x closer than DBL_EPSILON, where the reference's comparator
-// treats x as equal and is not an ordering, are reported as an error.
-__device__ __forceinline__ bool ref_ccw_or_collinear(double ax, double ay, double bx, double by, double cx,
-                                                     double cy) {
-    return (bx - ax) * (cy - ay) - (by - ay) * (cx - ax) <= 0;
-}
-
-__device__ __forceinline__ bool rec_less(const double* X, const double* Y, const int32_t* I, int a, int b) {
-    if (X[a] != X[b]) return X[a] < X[b];
-    if (Y[a] != Y[b]) return Y[a] < Y[b];
-    return I[a] < I[b];
-}
-
-__global__ __launch_bounds__(256) void k_hull_ref(DevBuf d, Layout L, const double2* list_xy) {
-    __shared__ int nlo, nup;
-    int tile, f;
-    xcd_tile_frame(tile, f);
-    const int K = static_cast<int>(d.fs[f * kFsCount + kFsClusters]);
-    const int tid = threadIdx.x;
-    const size_t ob = (size_t)f * L.N;
-    const size_t BN = (size_t)L.B * L.N;
-    for (int c = tile; c < K; c += gridDim.x) {
-        if (d.hull_flag[ob + c] == 0) continue;
-        const int n = static_cast<int>(d.cl_size[ob + c]);
-        if (n < 3) continue;
-        const uint32_t base = d.cl_off[ob + c];
-        double* X = d.hcx + ob + base;
-        double* Y = d.hcy + ob + base;
-        int32_t* I = d.hci + ob + base;
-        const int32_t* members = d.cl_members + ob + base;
-        for (int i = tid; i < n; i += blockDim.x) {
-            const int32_t m = members[i];
-            double x, y;
-            member_xy(d, list_xy, ob, base, m, x, y);
-            X[i] = x;
-            Y[i] = y;
-            I[i] = m;
-        }
+    for (int cb = 0; cb < K; cb += 1024 * T) {
+        if (tid == 0) open_n = 0;
         __syncthreads();
-        int m2 = 1;
-        while (m2 < n) m2 <<= 1;
-        for (int k = 2; k <= m2; k <<= 1) {
-            for (int j = k >> 1; j > 0; j >>= 1) {
-                for (int q = tid; q < (m2 >> 1); q += blockDim.x) {
-                    int a, b;
-                    if (j == (k >> 1)) {
-                        // First step of a merge: mirror pairs inside each block of k.
-                        const int blk = q / j, t = q % j;
-                        a = blk * k + t;
-                        b = blk * k + k - 1 - t;
-                    } else {
-                        a = ((q & ~(j - 1)) << 1) | (q & (j - 1));
-                        b = a + j;
-                    }
-                    if (b < n && rec_less(X, Y, I, b, a)) {
-                        const double tx = X[a], ty = Y[a];
-                        const int32_t ti = I[a];
-                        X[a] = X[b];
-                        Y[a] = Y[b];
-                        I[a] = I[b];
-                        X[b] = tx;
-                        Y[b] = ty;
-                        I[b] = ti;
-                    }
-                }
-                __syncthreads();
-            }
-        }
-        for (int i = 1 + tid; i < n; i += blockDim.x)
-            if (X[i] != X[i - 1] && fabs(X[i] - X[i - 1]) < DBL_EPSILON)
-                atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullFuzzyOrder);
-        // Stacks of sorted positions: lower in [0, n), upper in [n, 2n) of
-        // the second buffer's doubles viewed as int32 (2n entries fit).
-        int32_t* SL = reinterpret_cast<int32_t*>(d.hcx + BN + ob + base);
-        int32_t* SU = SL + n;
-        if (tid == 0) {
-            int k = 0;
-            for (int i = 0; i < n; ++i) {
-                while (k > 1 && ref_ccw_or_collinear(X[SL[k - 2]], Y[SL[k - 2]], X[SL[k - 1]], Y[SL[k - 1]], X[i], Y[i]))
-                    --k;
-                SL[k++] = i;
-            }
-            nlo = k;
-        } else if (tid == 1) {
-            // The reference's upper loop continues on the lower stack with
-            // t = k + 1; it never pops below the last point, so it is the
-            // same chain started from that point.
-            int k = 0;
-            SU[k++] = n - 1;
-            for (int i = n - 2; i >= 0; --i) {
-                while (k > 1 && ref_ccw_or_collinear(X[SU[k - 2]], Y[SU[k - 2]], X[SU[k - 1]], Y[SU[k - 1]], X[i], Y[i]))
-                    --k;
-                SU[k++] = i;
-            }
-            nup = k;
-        }
+        const int ct = cb + tid * T + static_cast<int>(blockIdx.x);
+        if (ct < K && __hip_atomic_load(&d.hull_flag[ob + ct], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+            open_list[atomicAdd(&open_n, 1)] = ct;
         __syncthreads();
-        const int kl = nlo;
-        const int kk = kl + nup - 2;  // indices.resize(k - 1)
-        if (kk > n) {
-            if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullCapacity);
-        } else {
-            for (int i = tid; i < kk; i += blockDim.x) d.hull_idx[ob + base + i] = I[i < kl ? SL[i] : SU[i - kl + 1]];
-            if (tid == 0) {
-                d.hull_count[ob + c] = static_cast<uint32_t>(kk);
-                atomicAdd(&d.fs[f * kFsCount + kFsHullRounded], 1u);
-            }
-        }
+        const int flagged = open_n;
+        for (int jo = 0; jo < flagged; ++jo) ref_hull(d, L, list_xy, f, open_list[jo], &nlo, &nup);
         __syncthreads();
     }
 }
@@ -1282,21 +1354,28 @@ __global__ __launch_bounds__(256) void k_hull_ref(DevBuf d, Layout L, const doub
 // order) also go to the second candidate buffer, free once the hulls are
 // done, where the box stage reads its polygons.
 //
-// One workgroup per cluster: the hull (up to kLocalMax vertices) is staged in
-// LDS with a hash of its coordinates; one pass over the members lowers each
-// vertex's index to the smallest member index with its coordinates, a second
-// pass bins every member by the number of (sorted) vertex indices not above
-// it, and the prefix sums of the bins are the ranks.  Each thread takes four
-// members at a time so their loads and searches overlap.  Larger hulls take
-// one wavefront per vertex.
-// Two launches split the clusters: those with at most kLocalSmallV hull
-// vertices and kLocalSmallSize members (most of them) take one wavefront
-// each, with 2.6 KiB of LDS, so a CU holds as many clusters as it holds
-// wavefronts; the others take a 1024-thread workgroup with room for
-// kLocalMax vertices, taken from a per-frame list the first launch writes.
+// The hull (up to kLocalMax vertices) is staged in LDS with a hash of its
+// coordinates; one pass over the members lowers each vertex's index to the
+// smallest member index with its coordinates, a second pass bins every member
+// by the number of (sorted) vertex indices not above it, and the prefix sums of
+// the bins are the ranks.  Each thread takes four members at a time so their
+// loads and searches overlap.  Larger hulls take one wavefront per vertex.
+// A workgroup takes a run of clusters, at most one for each of its wavefronts:
+// first all of at most kLocalSmallV hull vertices and kLocalSmallSize members
+// (most of them), a wavefront each, then the others one after the other with
+// all its threads.  The place of its run's vertices in the frame's hull array
+// is the sum of the vertex counts before it, which it adds up itself.  (As
+// three launches, a scan of the counts, the small clusters and the listed large
+// ones, each waited for its slowest cluster: one 64x2048 frame 46 -> 25 us, one
+// 32x1024 frame 37 -> 11 us, eight mixed frames at a time 61 -> 44 us.)  Runs
+// of one or two clusters, the case of few frames, leave most wavefronts idle,
+// so there a cluster of more than kLocalShortSize members has the workgroup
+// (32x1024 31 -> 11 us); longer runs would take many such clusters in turns.
 constexpr int kLocalMax = 512;
 constexpr int kLocalSmallV = 64;
 constexpr int kLocalSmallSize = 1024;
+constexpr int kLocalShortRun = 2;
+constexpr int kLocalShortSize = 256;
 constexpr int kLocalUnroll = 4;
 
 // Hash of a coordinate pair that agrees with ==: +0.0 and -0.0 hash alike.
@@ -1308,185 +1387,248 @@ __device__ __forceinline__ uint32_t xy_hash(double x, double y) {
     return static_cast<uint32_t>(h);
 }
 
-template <int kLocalThreads, int kVMax, bool kSmall>
-__global__ __launch_bounds__(kLocalThreads) void k_hull_local(DevBuf d, Layout L, const double2* list_xy) {
+template <int kVMax>
+struct LocalLds {
+    double vx[kVMax];
+    double vy[kVMax];
+    int32_t canon[kVMax];
+    int32_t sorted[kVMax];
+    int32_t table[2 * kVMax];
+    uint32_t bins[kVMax + 1];
+    int16_t spos[kVMax];
+};
+
+struct LocalCluster {
+    const int32_t* members;
+    int V, size;
+    uint32_t base, hoff;
+};
+
+template <int kThreads>
+__device__ __forceinline__ void local_sync() {
+    if (kThreads == kWave)
+        wave_sync();
+    else
+        __syncthreads();
+}
+
+// A cluster of at most kVMax hull vertices, by kThreads threads.
+template <int kThreads, int kVMax>
+__device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d, const double2* list_xy, size_t ob,
+                                            size_t BN, const LocalCluster& k) {
     constexpr int kLocalHash = 2 * kVMax;
-    __shared__ int32_t canon[kVMax];
-    __shared__ int32_t sorted[kVMax];
-    __shared__ int16_t spos[kVMax];
-    __shared__ int32_t table[kLocalHash];
-    __shared__ double vx[kVMax];
-    __shared__ double vy[kVMax];
-    __shared__ uint32_t bins[kVMax + 1];
+    const int tid = static_cast<int>(threadIdx.x) % kThreads;
+    const int w = tid / kWave;
+    const int lane = lane_id();
+    const int V = k.V, size = k.size;
+    const uint32_t base = k.base, hoff = k.hoff;
+    const int32_t* members = k.members;
+    const uint32_t hmask = static_cast<uint32_t>(kLocalHash - 1);
+    for (int i = tid; i < kLocalHash; i += kThreads) s.table[i] = -1;
+    for (int i = tid; i <= V; i += kThreads) s.bins[i] = 0;
+    local_sync<kThreads>();
+    for (int i = tid; i < V; i += kThreads) {
+        const int32_t idx = d.hull_idx[ob + base + i];
+        double x, y;
+        member_xy(d, list_xy, ob, base, idx, x, y);
+        s.canon[i] = idx;
+        s.vx[i] = x;
+        s.vy[i] = y;
+        if (!list_xy) {
+            d.hcx[BN + ob + hoff + i] = x;
+            d.hcy[BN + ob + hoff + i] = y;
+        }
+        uint32_t h = xy_hash(x, y) & hmask;  // load <= 1/2: a free slot exists
+        while (atomicCAS(&s.table[h], -1, i) != -1) h = (h + 1) & hmask;
+    }
+    local_sync<kThreads>();
+    // Smallest member index per vertex coordinates.
+    for (int q0 = tid; q0 < size; q0 += kThreads * kLocalUnroll) {
+        int32_t m[kLocalUnroll];
+        double mx[kLocalUnroll], my[kLocalUnroll];
+#pragma unroll
+        for (int u = 0; u < kLocalUnroll; ++u) {
+            const int q = q0 + u * kThreads;
+            m[u] = q < size ? members[q] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < kLocalUnroll; ++u)
+            if (m[u] >= 0) member_xy(d, list_xy, ob, base, m[u], mx[u], my[u]);
+#pragma unroll
+        for (int u = 0; u < kLocalUnroll; ++u) {
+            if (m[u] < 0) continue;
+            for (uint32_t h = xy_hash(mx[u], my[u]) & hmask;; h = (h + 1) & hmask) {
+                const int e = s.table[h];
+                if (e < 0) break;
+                if (s.vx[e] == mx[u] && s.vy[e] == my[u] && m[u] < s.canon[e]) atomicMin(&s.canon[e], m[u]);
+            }
+        }
+    }
+    local_sync<kThreads>();
+    // Sorted order of the vertex indices (ties, i.e. one point reported
+    // twice, in vertex order).
+    for (int i = tid; i < V; i += kThreads) {
+        const int32_t ci = s.canon[i];
+        int pos = 0;
+        for (int j = 0; j < V; ++j) {
+            const int32_t cj = s.canon[j];
+            pos += (cj < ci || (cj == ci && j < i)) ? 1 : 0;
+        }
+        s.sorted[pos] = ci;
+        s.spos[i] = static_cast<int16_t>(pos);
+        d.hull_idx[ob + base + i] = ci;
+    }
+    local_sync<kThreads>();
+    // Member m lands in bin b = number of sorted indices <= m; it is below
+    // s.sorted[k] exactly when b <= k.  Neighbouring lanes mostly share a
+    // bin: each run of equal bins adds its length once.
+    int steps = 0;
+    while ((1 << steps) <= V) ++steps;
+    // Wave-uniform trip count: the run detection below reads all lanes.
+    for (int q0 = w * kWave + lane; q0 - lane < size; q0 += kThreads * kLocalUnroll) {
+        int32_t m[kLocalUnroll];
+        int lo[kLocalUnroll], hi[kLocalUnroll];
+#pragma unroll
+        for (int u = 0; u < kLocalUnroll; ++u) {
+            const int q = q0 + u * kThreads;
+            m[u] = q < size ? members[q] : -1;
+            lo[u] = 0;
+            hi[u] = V;
+        }
+        for (int st = 0; st < steps; ++st) {
+#pragma unroll
+            for (int u = 0; u < kLocalUnroll; ++u) {
+                if (lo[u] < hi[u]) {
+                    const int mid = (lo[u] + hi[u]) >> 1;
+                    if (s.sorted[mid] <= m[u])
+                        lo[u] = mid + 1;
+                    else
+                        hi[u] = mid;
+                }
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kLocalUnroll; ++u) {
+            const int b = m[u] >= 0 ? lo[u] : -1;
+            const int prev = __shfl_up(b, 1, kWave);
+            const bool start = lane == 0 || b != prev;
+            const uint64_t starts = __ballot(start);
+            if (start && b >= 0) {
+                const uint64_t above = starts & ~((2ull << lane) - 1ull);
+                const int next = above ? __ffsll(static_cast<unsigned long long>(above)) - 1 : kWave;
+                atomicAdd(&s.bins[b], static_cast<uint32_t>(next - lane));
+            }
+        }
+    }
+    local_sync<kThreads>();
+    if (w == 0) {
+        uint32_t carry = 0;
+        for (int i0 = 0; i0 < V; i0 += kWave) {
+            const int i = i0 + lane;
+            uint32_t v = i < V ? s.bins[i] : 0u;
+#pragma unroll
+            for (int o = 1; o < kWave; o <<= 1) {
+                const uint32_t t = __shfl_up(v, o, kWave);
+                if (lane >= o) v += t;
+            }
+            if (i < V) s.bins[i] = carry + v;  // members below s.sorted[i]
+            carry += __shfl(v, kWave - 1, kWave);
+        }
+    }
+    local_sync<kThreads>();
+    for (int i = tid; i < V; i += kThreads) d.hull_local[ob + hoff + i] = static_cast<int32_t>(s.bins[s.spos[i]]);
+}
+
+// One of more hull vertices than that, a wavefront for each vertex.
+template <int kThreads>
+__device__ __forceinline__ void local_ranks_many(const DevBuf& d, const double2* list_xy, size_t ob, size_t BN,
+                                                 const LocalCluster& k) {
+    const int w = static_cast<int>(threadIdx.x) / kWave;
+    const int lane = lane_id();
+    const int V = k.V, size = k.size;
+    const uint32_t base = k.base, hoff = k.hoff;
+    const int32_t* members = k.members;
+    for (int i = w; i < V; i += kThreads / kWave) {
+        const int32_t idx = d.hull_idx[ob + base + i];
+        double px, py;
+        member_xy(d, list_xy, ob, base, idx, px, py);
+        int32_t cn = idx;
+        for (int q = lane; q < size; q += kWave) {
+            const int32_t m = members[q];
+            if (m >= cn) continue;
+            double mx, my;
+            member_xy(d, list_xy, ob, base, m, mx, my);
+            if (mx == px && my == py) cn = m;
+        }
+#pragma unroll
+        for (int o = kWave / 2; o > 0; o >>= 1) cn = min(cn, __shfl_xor(cn, o, kWave));
+        uint32_t cnt = 0;
+        for (int q = lane; q < size; q += kWave) cnt += members[q] < cn ? 1u : 0u;
+        cnt = wave_sum(cnt);
+        if (lane == 0) {
+            d.hull_idx[ob + base + i] = cn;
+            d.hull_local[ob + hoff + i] = static_cast<int32_t>(cnt);
+            if (!list_xy) {
+                d.hcx[BN + ob + hoff + i] = px;
+                d.hcy[BN + ob + hoff + i] = py;
+            }
+        }
+    }
+}
+
+template <int kThreads>
+__global__ __launch_bounds__(kThreads) void k_hull_local(DevBuf d, Layout L, const double2* list_xy) {
+    constexpr int kWaves = kThreads / kWave;
+    __shared__ union {
+        LocalLds<kLocalMax> large;
+        LocalLds<kLocalSmallV> small[kWaves];
+    } lds;
+    __shared__ LocalCluster run[kWaves];
+    __shared__ uint32_t sums[kWaves + 1];
     int tile, f;
     xcd_tile_frame(tile, f);
     const int K = static_cast<int>(d.fs[f * kFsCount + kFsClusters]);
     const int tid = threadIdx.x;
     const int w = tid / kWave;
-    const int lane = lane_id();
     const size_t ob = (size_t)f * L.N;
     const size_t BN = (size_t)L.B * L.N;
-    // The wavefront launch walks all clusters and lists the large ones; the
-    // workgroup launch takes list entries tile, tile + gridDim.x, ...
-    const int iters = kSmall ? K : static_cast<int>(d.fs[f * kFsCount + kFsHullLarge]);
-    for (int j = tile; j < iters; j += gridDim.x) {
-        const int c = kSmall ? j : d.hull_large[ob + j];
-        const int V = static_cast<int>(d.hull_count[ob + c]);
-        const uint32_t hoff = d.hull_off[ob + c];
-        const uint32_t base = d.cl_off[ob + c];
-        const int size = static_cast<int>(d.cl_size[ob + c]);
-        const int32_t* members = d.cl_members + ob + base;
-        if (kSmall && !(V <= kLocalSmallV && size <= kLocalSmallSize)) {
-            if (tid == 0) d.hull_large[ob + atomicAdd(&d.fs[f * kFsCount + kFsHullLarge], 1u)] = c;
-            continue;
+    const int tiles = static_cast<int>(gridDim.x);
+    const int per = min(kWaves, max(1, (K + tiles - 1) / tiles));
+    const int small_size = per <= kLocalShortRun ? kLocalShortSize : kLocalSmallSize;
+    if (K == 0 && tile == 0 && tid == 0) d.fs[f * kFsCount + kFsHullTotal] = 0;
+    for (int c0 = tile * per; c0 < K; c0 += tiles * per) {
+        const int cnt = min(per, K - c0);
+        if (tid < cnt) {
+            const size_t c = ob + c0 + tid;
+            run[tid].V = static_cast<int>(d.hull_count[c]);
+            run[tid].size = static_cast<int>(d.cl_size[c]);
+            run[tid].base = d.cl_off[c];
+            run[tid].members = d.cl_members + ob + run[tid].base;
+            // A cluster left without a hull ran out of the chunk rounds' and
+            // the final workgroup's capacity.
+            if (run[tid].V == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullCapacity);
         }
-        // A cluster left without a hull ran out of the chunk rounds' and the
-        // final workgroup's capacity.
-        if (V == 0 && tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullCapacity);
-        if (!kSmall && V > kVMax) {
-            for (int i = w; i < V; i += kLocalThreads / kWave) {
-                const int32_t idx = d.hull_idx[ob + base + i];
-                double px, py;
-                member_xy(d, list_xy, ob, base, idx, px, py);
-                int32_t cn = idx;
-                for (int q = lane; q < size; q += kWave) {
-                    const int32_t m = members[q];
-                    if (m >= cn) continue;
-                    double mx, my;
-                    member_xy(d, list_xy, ob, base, m, mx, my);
-                    if (mx == px && my == py) cn = m;
-                }
-#pragma unroll
-                for (int o = kWave / 2; o > 0; o >>= 1) cn = min(cn, __shfl_xor(cn, o, kWave));
-                uint32_t cnt = 0;
-                for (int q = lane; q < size; q += kWave) cnt += members[q] < cn ? 1u : 0u;
-                cnt = wave_sum(cnt);
-                if (lane == 0) {
-                    d.hull_idx[ob + base + i] = cn;
-                    d.hull_local[ob + hoff + i] = static_cast<int32_t>(cnt);
-                    if (!list_xy) {
-                        d.hcx[BN + ob + hoff + i] = px;
-                        d.hcy[BN + ob + hoff + i] = py;
-                    }
-                }
-            }
-            continue;
-        }
-        const uint32_t hmask = static_cast<uint32_t>(kLocalHash - 1);
-        for (int i = tid; i < kLocalHash; i += kLocalThreads) table[i] = -1;
-        for (int i = tid; i <= V; i += kLocalThreads) bins[i] = 0;
-        __syncthreads();
-        for (int i = tid; i < V; i += kLocalThreads) {
-            const int32_t idx = d.hull_idx[ob + base + i];
-            double x, y;
-            member_xy(d, list_xy, ob, base, idx, x, y);
-            canon[i] = idx;
-            vx[i] = x;
-            vy[i] = y;
-            if (!list_xy) {
-                d.hcx[BN + ob + hoff + i] = x;
-                d.hcy[BN + ob + hoff + i] = y;
-            }
-            uint32_t h = xy_hash(x, y) & hmask;  // load <= 1/2: a free slot exists
-            while (atomicCAS(&table[h], -1, i) != -1) h = (h + 1) & hmask;
+        uint32_t before = 0, hoff;
+        for (int i = tid; i < c0; i += kThreads) before += d.hull_count[ob + i];
+        block_exclusive_sum<kThreads>(before, sums, &hoff);
+        if (tid < cnt) {
+            for (int q = 0; q < tid; ++q) hoff += static_cast<uint32_t>(run[q].V);
+            run[tid].hoff = hoff;
+            d.hull_off[ob + c0 + tid] = hoff;
+            if (c0 + tid == K - 1) d.fs[f * kFsCount + kFsHullTotal] = hoff + static_cast<uint32_t>(run[tid].V);
         }
         __syncthreads();
-        // Smallest member index per vertex coordinates.
-        for (int q0 = tid; q0 < size; q0 += kLocalThreads * kLocalUnroll) {
-            int32_t m[kLocalUnroll];
-            double mx[kLocalUnroll], my[kLocalUnroll];
-#pragma unroll
-            for (int u = 0; u < kLocalUnroll; ++u) {
-                const int q = q0 + u * kLocalThreads;
-                m[u] = q < size ? members[q] : -1;
-            }
-#pragma unroll
-            for (int u = 0; u < kLocalUnroll; ++u)
-                if (m[u] >= 0) member_xy(d, list_xy, ob, base, m[u], mx[u], my[u]);
-#pragma unroll
-            for (int u = 0; u < kLocalUnroll; ++u) {
-                if (m[u] < 0) continue;
-                for (uint32_t h = xy_hash(mx[u], my[u]) & hmask;; h = (h + 1) & hmask) {
-                    const int e = table[h];
-                    if (e < 0) break;
-                    if (vx[e] == mx[u] && vy[e] == my[u] && m[u] < canon[e]) atomicMin(&canon[e], m[u]);
-                }
-            }
+        auto small = [&](int q) { return run[q].V <= kLocalSmallV && run[q].size <= small_size; };
+        if (w < cnt && small(w)) local_ranks<kWave, kLocalSmallV>(lds.small[w], d, list_xy, ob, BN, run[w]);
+        __syncthreads();
+        for (int q = 0; q < cnt; ++q) {
+            if (small(q)) continue;
+            if (run[q].V > kLocalMax)
+                local_ranks_many<kThreads>(d, list_xy, ob, BN, run[q]);
+            else
+                local_ranks<kThreads, kLocalMax>(lds.large, d, list_xy, ob, BN, run[q]);
+            __syncthreads();
         }
-        __syncthreads();
-        // Sorted order of the vertex indices (ties, i.e. one point reported
-        // twice, in vertex order).
-        for (int i = tid; i < V; i += kLocalThreads) {
-            const int32_t ci = canon[i];
-            int pos = 0;
-            for (int j = 0; j < V; ++j) {
-                const int32_t cj = canon[j];
-                pos += (cj < ci || (cj == ci && j < i)) ? 1 : 0;
-            }
-            sorted[pos] = ci;
-            spos[i] = static_cast<int16_t>(pos);
-            d.hull_idx[ob + base + i] = ci;
-        }
-        __syncthreads();
-        // Member m lands in bin b = number of sorted indices <= m; it is below
-        // sorted[k] exactly when b <= k.  Neighbouring lanes mostly share a
-        // bin: each run of equal bins adds its length once.
-        int steps = 0;
-        while ((1 << steps) <= V) ++steps;
-        // Wave-uniform trip count: the run detection below reads all lanes.
-        for (int q0 = w * kWave + lane; q0 - lane < size; q0 += kLocalThreads * kLocalUnroll) {
-            int32_t m[kLocalUnroll];
-            int lo[kLocalUnroll], hi[kLocalUnroll];
-#pragma unroll
-            for (int u = 0; u < kLocalUnroll; ++u) {
-                const int q = q0 + u * kLocalThreads;
-                m[u] = q < size ? members[q] : -1;
-                lo[u] = 0;
-                hi[u] = V;
-            }
-            for (int st = 0; st < steps; ++st) {
-#pragma unroll
-                for (int u = 0; u < kLocalUnroll; ++u) {
-                    if (lo[u] < hi[u]) {
-                        const int mid = (lo[u] + hi[u]) >> 1;
-                        if (sorted[mid] <= m[u])
-                            lo[u] = mid + 1;
-                        else
-                            hi[u] = mid;
-                    }
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kLocalUnroll; ++u) {
-                const int b = m[u] >= 0 ? lo[u] : -1;
-                const int prev = __shfl_up(b, 1, kWave);
-                const bool start = lane == 0 || b != prev;
-                const uint64_t starts = __ballot(start);
-                if (start && b >= 0) {
-                    const uint64_t above = starts & ~((2ull << lane) - 1ull);
-                    const int next = above ? __ffsll(static_cast<unsigned long long>(above)) - 1 : kWave;
-                    atomicAdd(&bins[b], static_cast<uint32_t>(next - lane));
-                }
-            }
-        }
-        __syncthreads();
-        if (w == 0) {
-            uint32_t carry = 0;
-            for (int i0 = 0; i0 < V; i0 += kWave) {
-                const int i = i0 + lane;
-                uint32_t v = i < V ? bins[i] : 0u;
-#pragma unroll
-                for (int o = 1; o < kWave; o <<= 1) {
-                    const uint32_t t = __shfl_up(v, o, kWave);
-                    if (lane >= o) v += t;
-                }
-                if (i < V) bins[i] = carry + v;  // members below sorted[i]
-                carry += __shfl(v, kWave - 1, kWave);
-            }
-        }
-        __syncthreads();
-        for (int i = tid; i < V; i += kLocalThreads) d.hull_local[ob + hoff + i] = static_cast<int32_t>(bins[spos[i]]);
-        __syncthreads();
     }
 }
 
@@ -1503,7 +1645,7 @@ __global__ void k_hull_lists_init(DevBuf d, Layout L, const int32_t* offsets, in
         d.fs[kFsErr] = 0;
         d.fs[kFsHullInexact] = 0;
         d.fs[kFsHullRounded] = 0;
-        d.fs[kFsHullLarge] = 0;
+        d.fs[kFsHullOpen] = 0;
     }
     if (t < K) {
         d.cl_off[t] = static_cast<uint32_t>(offsets[t]);
@@ -1528,7 +1670,7 @@ __global__ void k_hull_lists_init(DevBuf d, Layout L, const int32_t* offsets, in
 
 void launch_hull_lists(lp_context* c, int num_lists, int total_points) {
     const int n = std::max(num_lists, total_points);
-    const int32_t* offs = reinterpret_cast<const int32_t*>(c->d.hc_choff);  // staged by the caller
+    const int32_t* offs = reinterpret_cast<const int32_t*>(c->d.hc_open);  // staged by the caller
     double2* list_xy = reinterpret_cast<double2*>(c->d.dsort);
     hipLaunchKernelGGL(k_hull_lists_init, dim3((n + 255) / 256), dim3(256), 0, c->stream, c->d, c->L, offs,
                        num_lists, total_points, list_xy);
@@ -1539,35 +1681,42 @@ void launch_hull(lp_context* c, int B, const double2* list_xy) {
     DevBuf& d = c->d;
     const Layout& L = c->L;
     hipStream_t st = c->stream;
-    // Stage marks around the single-kernel steps ("hull_round" three
-    // times), so profiled runs time each round launch on its own.
+    // Stage marks around the single-kernel steps, so profiled runs time each
+    // launch on its own.
     // Chunk wavefronts loop over the frame's chunks: about 2048 workgroups
     // in all, at most 512 per frame; workgroups beyond that would mostly
     // find no chunk and only cost dispatch.
     const int round_grid = std::min(512, std::max(8, 2048 / B));
-    for (int r = 0; r < kHullRounds; ++r) {
-        stage_mark(c, "hull");
-        hipLaunchKernelGGL(k_hull_plan, dim3(B), dim3(kPlanThreads), 0, st, d, L, r);
-        stage_mark(c, "hull_round");
-        hipLaunchKernelGGL(k_hull_round, dim3(round_grid, B), dim3(256), 0, st, d, L, r);
-    }
-    stage_mark(c, "hull_big");
-    hipLaunchKernelGGL(k_hull_big, dim3(16, B), dim3(1024), 0, st, d, L, kHullRounds);
-    stage_mark(c, "hull_ref");
-    hipLaunchKernelGGL(k_hull_ref, dim3(16, B), dim3(256), 0, st, d, L, list_xy);
     stage_mark(c, "hull");
-    launch_scan_small(c, B, d.hull_count, d.hull_off, L.N, kCountSlot, kFsClusters, kFsHullTotal);
+    hipLaunchKernelGGL(k_hull_plan, dim3(B), dim3(kPlanThreads), 0, st, d, L);
+    stage_mark(c, "hull_round");
+    hipLaunchKernelGGL(k_hull_round, dim3(round_grid, B), dim3(256), 0, st, d, L);
+    // The clusters of more than one chunk are a few dozen per frame at most:
+    // 16 to 256 workgroups per frame, so each takes about one.
+    const int merge_grid = std::min(256, std::max(16, 2048 / B));
+    const int reset_grid = list_xy ? 0 : kResetTiles;
+    // Few frames: large workgroups, so the largest clusters end sooner.  From
+    // 16 frames on the chip is full of clusters and the idle wavefronts of a
+    // large workgroup cost more than its tail: 128 frames in four lanes
+    // 6.64 ms with the large ones, 6.52 ms with these; 16 frames of 128x2048
+    // in two lanes 1.85 ms with the large ones, 1.91 ms with these.
+    const bool wide = B < 16;
+    auto local_grid = [&](int threads) { return std::min(256, std::max(8, 16384 / (threads / kWave) / B)); };
+    stage_mark(c, "hull_merge");
+    const dim3 mg(merge_grid + reset_grid, B);
+    if (wide)
+        hipLaunchKernelGGL(k_hull_merge<512>, mg, dim3(512), 0, st, d, L, merge_grid);
+    else
+        hipLaunchKernelGGL(k_hull_merge<256>, mg, dim3(256), 0, st, d, L, merge_grid);
+    stage_mark(c, "hull_big");
+    hipLaunchKernelGGL(k_hull_big, dim3(16, B), dim3(1024), 0, st, d, L, list_xy);
+    // A wavefront for about each cluster, and at most 256 workgroups a frame,
+    // so that a run holds few clusters while the chip has room.
     stage_mark(c, "hull_local");
-    // About 16384 wavefronts for the small clusters (about one cluster each
-    // on 128 frames), at least 8 per frame.
-    const int small_grid = std::min(1024, std::max(8, 16384 / B));
-    hipLaunchKernelGGL((k_hull_local<kWave, kLocalSmallV, true>), dim3(small_grid, B), dim3(kWave), 0, st, d, L,
-                       list_xy);
-    // The large clusters, listed by the launch above, are a few dozen per
-    // frame at most: 16 to 256 workgroups per frame, so each takes about one.
-    const int large_grid = std::min(256, std::max(16, 2048 / B));
-    hipLaunchKernelGGL((k_hull_local<1024, kLocalMax, false>), dim3(large_grid, B), dim3(1024), 0, st, d, L,
-                       list_xy);
+    if (wide)
+        hipLaunchKernelGGL(k_hull_local<1024>, dim3(local_grid(1024), B), dim3(1024), 0, st, d, L, list_xy);
+    else
+        hipLaunchKernelGGL(k_hull_local<512>, dim3(local_grid(512), B), dim3(512), 0, st, d, L, list_xy);
 }
 
 }  // namespace lp

@@ -179,16 +179,14 @@ struct DevBuf {
     double* hcy;
     int32_t* hci;            // candidate obstacle index
     uint32_t* hc_count;      // per cluster candidates (two buffers)
-    uint32_t* hc_choff;      // their exclusive scan
-    // Per chunk of a hull round (written by the round's plan): its cluster,
+    uint32_t* hc_open;       // clusters of more than one chunk
+    // Per chunk of the first hull round (written by its plan): its cluster,
     // with bit 31 set when the chunk is the cluster's only one (= cell_items,
     // free in the hull stage); its index in the cluster and, from bit 16, its
-    // point count (= cell_zkey); the cluster's first candidate (= hull_large,
-    // free until the local ranks).
+    // point count (= cell_zkey); the cluster's first candidate.
     int32_t* hc_chunk_c;
     uint32_t* hc_chunk_i;
     uint32_t* hc_chunk_b;
-    int32_t* hull_large;     // [B][N] clusters left to the workgroup local-rank launch
     int32_t* hull_idx;       // final hull (obstacle indices), frame stride N
     uint32_t* hull_count;    // per cluster
     uint32_t* hull_off;      // per cluster (+1)
@@ -250,7 +248,7 @@ enum FsSlot : int {
     kFsHullRounded,    // clusters whose hull was redone with the reference's rounded predicate
     kFsErr,
     kFsBoxes,          // clusters with a box
-    kFsHullLarge,      // clusters listed for the workgroup local-rank launch
+    kFsHullOpen,       // clusters of more than one chunk
     kFsCellPoints,     // points in polar cells
     kFsCellsSmall,     // non-empty polar cells of up to 16 points
     kFsCellsLarge,     // larger ones

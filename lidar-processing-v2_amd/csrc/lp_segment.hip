@@ -11,6 +11,7 @@
 // arrays of cells / pixels / queue entries use fixed frame strides.  Grids
 // are (tiles, frames) and sized for the batch capacity so one launch
 // sequence (and one captured graph) serves every batch of a shape bucket.
+#include "lp_hash.h"
 #include "lp_kernels.h"
 #include "lp_queue.h"
 
@@ -880,26 +881,10 @@ void launch_clear(lp_context* c, int B) {
     hipLaunchKernelGGL(k_clear, dim3(256, B), dim3(256), 0, c->stream, c->d, c->L);
 }
 
-// Hash slots back to their clean state: key -1 (free), count 0, aux
-// kHashMinClean.  k_hash_reset takes the slots a stage occupied (slots[0 ..
-// fs[count_slot]) per frame); k_hash_init clears every slot (context
-// creation, or a frame whose list is incomplete).
+// k_hash_reset clears the slots a stage occupied; k_hash_init clears every slot
+// (context creation).
 __global__ void k_hash_reset(DevBuf d, Layout L, const int32_t* slots, int count_slot) {
-    const int f = blockIdx.y;
-    const uint32_t cnt = d.fs[f * kFsCount + count_slot];
-    const size_t ho = (size_t)f * L.hash_cap;
-    const int stride = gridDim.x * blockDim.x;
-    const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
-    if (cnt > static_cast<uint32_t>(L.N)) {
-        for (int h = t0; h < L.hash_cap; h += stride) {
-            d.hslot[ho + h] = HashSlot{-1, 0u, 0, kHashMinClean};
-        }
-        return;
-    }
-    for (int v = t0; v < static_cast<int>(cnt); v += stride) {
-        const int32_t h = slots[(size_t)f * L.N + v];
-        d.hslot[ho + h] = HashSlot{-1, 0u, 0, kHashMinClean};
-    }
+    reset_slots(d, L, blockIdx.y, slots, count_slot, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 __global__ void k_hash_init(DevBuf d, Layout L) {
