@@ -443,6 +443,48 @@ __device__ __forceinline__ void block_reserve(uint32_t* ctr, const bool (&flag)[
     __syncthreads();
 }
 
+// Two of them at once, with their atomics in flight together.
+template <int R>
+__device__ __forceinline__ void block_reserve2(uint32_t* ctr_a, const bool (&flag_a)[R], uint32_t (&out_a)[R],
+                                               uint32_t* lds_a, uint32_t* ctr_b, const bool (&flag_b)[R],
+                                               uint32_t (&out_b)[R], uint32_t* lds_b) {
+    const int NW = static_cast<int>(blockDim.x) / kWave;
+    const int w = static_cast<int>(threadIdx.x) / kWave;
+    uint64_t a[R], b[R];
+    uint32_t ta = 0, tb = 0;
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+        a[s] = __ballot(flag_a[s]);
+        b[s] = __ballot(flag_b[s]);
+        ta += static_cast<uint32_t>(__popcll(a[s]));
+        tb += static_cast<uint32_t>(__popcll(b[s]));
+    }
+    if (lane_id() == 0) {
+        lds_a[w] = ta;
+        lds_b[w] = tb;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+        uint32_t* lds = threadIdx.x == 0 ? lds_a : lds_b;
+        uint32_t run = 0;
+        for (int q = 0; q < NW; ++q) {
+            const uint32_t t = lds[q];
+            lds[q] = run;
+            run += t;
+        }
+        lds[NW] = run ? atomicAdd(threadIdx.x == 0 ? ctr_a : ctr_b, run) : 0u;
+    }
+    __syncthreads();
+    uint32_t base_a = lds_a[NW] + lds_a[w], base_b = lds_b[NW] + lds_b[w];
+#pragma unroll
+    for (int s = 0; s < R; ++s) {
+        out_a[s] = base_a + lanes_below(a[s]);
+        out_b[s] = base_b + lanes_below(b[s]);
+        base_a += static_cast<uint32_t>(__popcll(a[s]));
+        base_b += static_cast<uint32_t>(__popcll(b[s]));
+    }
+}
+
 // Stream compaction inside one tile of NT * R elements held row by row
 // (element k * NT + threadIdx.x of the tile is the thread's element of row
 // k, so every row is read and written with coalesced accesses).  bits has

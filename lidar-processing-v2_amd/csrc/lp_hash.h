@@ -5,6 +5,8 @@
 
 namespace lp {
 
+constexpr int kResetTiles = 16;  // workgroups per frame that a launch adds to clear the table
+
 // Slots a stage occupied (slots[0 .. fs[count_slot])) back to their clean
 // state, key -1 (free), count 0, aux kHashMinClean, by the threads t0, t0 +
 // stride, ...; the whole table when the list is incomplete.

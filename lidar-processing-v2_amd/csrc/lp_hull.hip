@@ -986,8 +986,6 @@ __global__ __launch_bounds__(256, 3) void k_hull_round(DevBuf d, Layout L) {
     }
 }
 
-constexpr int kResetTiles = 16;
-
 // The rounds after the first, a workgroup for each cluster of more than one
 // chunk: its wavefronts take the chunks of its candidates, and the round's
 // vertices are the next round's candidates.  A plan and a launch per round,

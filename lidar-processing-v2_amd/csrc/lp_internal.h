@@ -248,6 +248,7 @@ enum FsSlot : int {
     kFsHullRounded,    // clusters whose hull was redone with the reference's rounded predicate
     kFsErr,
     kFsBoxes,          // clusters with a box
+    kFsNoisePlaced,    // cell-sorted places given to cells
     kFsHullOpen,       // clusters of more than one chunk
     kFsCellPoints,     // points in polar cells
     kFsCellsSmall,     // non-empty polar cells of up to 16 points

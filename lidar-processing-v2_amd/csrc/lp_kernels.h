@@ -28,17 +28,6 @@ enum ScanCount : int { kCountPoints = 0, kCountPixels = 1, kCountSlot = 2, kCoun
 // fs[f][total_slot] (if >= 0).
 void launch_scan(lp_context* c, int B, const uint32_t* in, uint32_t* out, size_t stride, ScanCount kind,
                  int count_slot, int total_slot);
-// The same in one launch, one workgroup per frame: for cluster-sized counts.
-void launch_scan_small(lp_context* c, int B, const uint32_t* in, uint32_t* out, size_t stride, ScanCount kind,
-                       int count_slot, int total_slot);
-// The same with element i of frame f read as
-// in[(f * in_stride + gather[f * stride + i]) * elem] (a field of a record array).
-void launch_scan_gather(lp_context* c, int B, const uint32_t* in, size_t in_stride, int elem, const int32_t* gather,
-                        uint32_t* out, size_t stride, ScanCount kind, int count_slot, int total_slot);
-// The same, each result written back through the gather index into another
-// field of the record array (`field` is that field of record 0).
-void launch_scan_gather_into(lp_context* c, int B, const uint32_t* in, size_t in_stride, int elem,
-                             const int32_t* gather, uint32_t* field, size_t stride, ScanCount kind, int count_slot);
 
 void launch_mt19937(uint32_t* out, int count, hipStream_t st);
 // Resets the hash slots slots[f * N .. + fs[count_slot]) of every frame to
@@ -61,8 +50,9 @@ void launch_hull(lp_context* c, int B, const double2* list_xy = nullptr);
 // second the reference object's KD-tree search.
 void launch_noise(lp_context* c, int B, bool compact);
 void launch_noise_kdtree(lp_context* c, int B, bool compact);
-// Kept points (keep flags of the noise stage) into the segmenter's inputs.
-void launch_noise_compact(lp_context* c, int B);
+// Kept points (keep flags of the noise stage) into the segmenter's inputs; after
+// the radius rule also the noise count, and its cells' hash slots are cleared.
+void launch_noise_compact(lp_context* c, int B, bool radius_rule);
 // Tree levels built range by range before the per-subtree LDS kernel.
 int kd_small_level_host(int n);
 // Oriented boxes of the polygons in the second hull candidate buffer: the

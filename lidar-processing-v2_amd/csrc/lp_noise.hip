@@ -16,12 +16,12 @@
 //
 // Layout: the frame's points are bucketed into 1 m grid cells through an
 // open-addressing hash of cell keys (one slot per occupied cell, load at most
-// the context's hash load factor), counted, scanned and scattered into a
+// the context's hash load factor), counted, placed and scattered into a
 // cell-sorted float4 array (w holds the cell's hash slot).  The same pass
 // that runs the input-order test inserts the point and takes its place in
 // the cell from the cell count's atomic add, so the scatter needs no
-// atomics.  The grid count runs in two passes.  The first, one
-// thread per open point, checks the point's own cell outward from its own
+// atomics.  The grid count runs in two passes.  The first, eight
+// lanes per open point, checks the point's own cell outward from its own
 // position (points next to each other in scan order are mostly neighbours in
 // space), so almost every open point of a dense surface reaches
 // min_neighbours after a few distance tests; a point whose ball lies inside
@@ -30,6 +30,7 @@
 // point, visits the cube of cells within ceil(r) + 1 nearest first: the slow
 // searches run side by side instead of holding up wavefronts of easy points.
 #include "lp_device.h"
+#include "lp_hash.h"
 #include "lp_internal.h"
 #include "lp_kernels.h"
 
@@ -97,6 +98,7 @@ __global__ void k_noise_clear(DevBuf d, Layout L) {
         d.fs[f * kFsCount + kFsNoiseOpen] = 0;
         d.fs[f * kFsCount + kFsNoiseHard] = 0;
         d.fs[f * kFsCount + kFsNoiseCells] = 0;
+        d.fs[f * kFsCount + kFsNoisePlaced] = 0;
         d.fs[f * kFsCount + kFsNoiseErr] = 0;
     }
 }
@@ -118,7 +120,7 @@ constexpr int kPrepTile = 256 * kPrepRows;
 // round trips, and two points per thread halve the waits per point.
 __global__ __launch_bounds__(256) void k_noise_prep(DevBuf d, Layout L) {
     __shared__ float4 tile_pts[kPrepTile + 2 * kNearWindow];
-    __shared__ uint32_t rsv[256 / kWave + 1];
+    __shared__ uint32_t rsv[2][256 / kWave + 1];
     int tile, f;
     xcd_tile_frame(tile, f);
     const FrameDesc& fd = d.frames[f];
@@ -163,12 +165,6 @@ __global__ __launch_bounds__(256) void k_noise_prep(DevBuf d, Layout L) {
         // nothing.
         key[s] = in_frame ? noise_key(cxs[s], cys[s], cz) : -2;
     }
-    uint32_t q[kPrepRows];
-    block_reserve<kPrepRows>(&d.fs[f * kFsCount + kFsNoiseOpen], open, q, rsv);
-#pragma unroll
-    for (int s = 0; s < kPrepRows; ++s)
-        if (open[s]) d.nopen[po + q[s]] = i[s];
-
     // A run of lanes with the same cell (consecutive points mostly share one)
     // inserts once: its lowest lane probes and adds the run's count; all
     // runs of both rows at once.
@@ -202,12 +198,15 @@ __global__ __launch_bounds__(256) void k_noise_prep(DevBuf d, Layout L) {
             atomicOr(&d.nocc[(size_t)f * kNoiseOccWords + cys[s] * 32 + (cxs[s] >> 5)], 1u << (cxs[s] & 31));
         }
     }
-    // Every occupied cell gets a dense id (in any order): the cell counts are
-    // scanned over the ids, not over the whole table.
-    uint32_t id[kPrepRows];
-    block_reserve<kPrepRows>(&d.fs[f * kFsCount + kFsNoiseCells], fresh, id, rsv);
+    // Every occupied cell gets a dense id (in any order): places are given to
+    // the cells over the ids, not over the whole table.  The open list's places
+    // are taken at the same time.
+    uint32_t id[kPrepRows], q[kPrepRows];
+    block_reserve2<kPrepRows>(&d.fs[f * kFsCount + kFsNoiseCells], fresh, id, rsv[0],
+                              &d.fs[f * kFsCount + kFsNoiseOpen], open, q, rsv[1]);
 #pragma unroll
     for (int s = 0; s < kPrepRows; ++s) {
+        if (open[s]) d.nopen[po + q[s]] = i[s];
         if (fresh[s]) {
             d.ncell_slot[(size_t)f * L.N + id[s]] = static_cast<int32_t>(h[s]);
             d.hslot[ho + h[s]].dense = static_cast<int32_t>(id[s]);
@@ -221,9 +220,36 @@ __global__ __launch_bounds__(256) void k_noise_prep(DevBuf d, Layout L) {
     }
 }
 
-// Each slot's aux holds its cell's first cell-sorted position on entry (the
-// exclusive scan of the cell counts by dense id); each point goes to that
-// start plus its place in the cell.
+// Every cell's first cell-sorted position into its slot's aux: a workgroup
+// takes the places of its cells in one piece, in any order (which cell lies
+// where changes no result).  A scan of the counts over the dense ids took two
+// launches (one 64x2048 frame 13.4 -> 4.9 us, 32 frames at a time 31 -> 14).
+__global__ __launch_bounds__(256) void k_noise_cells(DevBuf d, Layout L) {
+    __shared__ uint32_t lds[256 / kWave + 1];
+    __shared__ uint32_t first;
+    int tile, f;
+    xcd_tile_frame(tile, f);
+    const uint32_t cells = d.fs[f * kFsCount + kFsNoiseCells];
+    const size_t ho = (size_t)f * L.hash_cap;
+    for (uint32_t base = tile * 256; base < cells; base += gridDim.x * 256) {
+        const uint32_t id = base + threadIdx.x;
+        HashSlot* s = nullptr;
+        uint32_t n = 0;
+        if (id < cells) {
+            s = d.hslot + ho + d.ncell_slot[(size_t)f * L.N + id];
+            n = s->count;
+        }
+        uint32_t total;
+        const uint32_t ex = block_exclusive_sum<256>(n, lds, &total);
+        if (threadIdx.x == 0) first = atomicAdd(&d.fs[f * kFsCount + kFsNoisePlaced], total);
+        __syncthreads();
+        if (s) s->aux = static_cast<int32_t>(first + ex);
+        __syncthreads();
+    }
+}
+
+// Each slot's aux holds its cell's first cell-sorted position on entry; each
+// point goes to that start plus its place in the cell.
 __global__ void k_noise_scatter(DevBuf d, Layout L) {
     int tile, f;
     xcd_tile_frame(tile, f);
@@ -250,89 +276,100 @@ __device__ __forceinline__ float cell_gap_sqr(float fx, float fy, float fz, int 
     return gx * gx + gy * gy + gz * gz;
 }
 
-// Writes the label of point i and counts NOISE labels per wavefront.
-__device__ __forceinline__ void noise_label(const DevBuf& d, int f, size_t po, int i, bool noise) {
-    d.noise[po + i] = noise ? 1 : 0;
-    const uint64_t m = __ballot(noise);
-    if (m && lane_id() == __ffsll(static_cast<unsigned long long>(m)) - 1)
-        atomicAdd(&d.fs[f * kFsCount + kFsNoise], static_cast<uint32_t>(__popcll(m)));
-}
-
 constexpr int kOwnCellBudget = 64;  // distance tests of the own-cell pass
-
-// Own-cell test of point i at cell-sorted position pos (see k_noise_count).
-__device__ __forceinline__ void noise_own_cell(const DevBuf& d, const NoiseConst& nc, int f, size_t po, size_t ho,
-                                               int i, int pos) {
-    const float4 t = d.dsort[po + pos];
-    const float r2 = noise_radius_sqr(nc, t.x, t.y);
-    const uint32_t k = nc.k;
-    int state;  // 0 VALID, 1 NOISE, 2 listed
-    uint32_t carry = 0;  // listed: own-cell count and how far the scan got
-    if (k == 0) {
-        state = 0;
-    } else if (!(r2 >= 0.0f)) {
-        state = 1;  // a NaN radius admits no point
-    } else {
-        const int h = __float_as_int(t.w);
-        const HashSlot hv = d.hslot[ho + h];
-        const int s0 = hv.aux;
-        const int s1 = s0 + static_cast<int>(hv.count);
-        uint32_t cnt = 0;
-        int budget = kOwnCellBudget;
-        int up = pos, dn = pos - 1;
-        while (cnt < k && budget > 0 && (up < s1 || dn >= s0)) {
-            // Alternate after and before the point (its scan-order neighbours).
-            const bool fwd = up < s1 && (dn < s0 || ((budget & 1) == 0));
-            const int s = fwd ? up++ : dn--;
-            cnt += noise_dist(t, d.dsort[po + s]) <= r2 ? 1u : 0u;
-            --budget;
-        }
-        if (cnt >= k) {
-            state = 0;
-        } else {
-            state = 2;
-            carry = cnt | static_cast<uint32_t>(up - pos) << 8 | static_cast<uint32_t>(pos - 1 - dn) << 16;
-            const float r = sqrtf(r2);
-            int cx, cy, cz;
-            noise_cell(t.x, t.y, t.z, cx, cy, cz);
-            const bool whole = up >= s1 && dn < s0;
-            const bool interior = cx > 0 && cx < 1023 && cy > 0 && cy < 1023 && cz > 0 && cz < 2047;
-            if (whole && interior && r < static_cast<float>(kNoiseMaxExtent - 1)) {
-                const float fx = t.x - floorf(t.x), fy = t.y - floorf(t.y), fz = t.z - floorf(t.z);
-                const float reach = (r + kNoiseCellSlack) * (r + kNoiseCellSlack);
-                if (cell_gap_sqr(fx, fy, fz, -1, 0, 0) > reach && cell_gap_sqr(fx, fy, fz, 1, 0, 0) > reach &&
-                    cell_gap_sqr(fx, fy, fz, 0, -1, 0) > reach && cell_gap_sqr(fx, fy, fz, 0, 1, 0) > reach &&
-                    cell_gap_sqr(fx, fy, fz, 0, 0, -1) > reach && cell_gap_sqr(fx, fy, fz, 0, 0, 1) > reach)
-                    state = 1;
-            }
-        }
-    }
-    if (state == 2) {
-        const uint32_t q = wave_atomic_inc(&d.fs[f * kFsCount + kFsNoiseHard]);
-        d.vslot[po + q] = pos;  // the listed point: position, input index and carry, loaded side by side
-        d.nloc[po + q] = i;
-        d.obs_src[po + q] = static_cast<int32_t>(carry);
-    } else {
-        noise_label(d, f, po, i, state == 1);
-    }
-}
+constexpr int kOwnLanes = 8;        // lanes per open point
+constexpr int kOwnTests = 16;       // tests a step
 
 // Own-cell pass over the open list (a grid-stride loop).  A point is VALID
 // once min_neighbours points of its cell are within its radius (the count
 // includes itself, and the search order does not change the outcome), NOISE
 // when its whole cell has been checked and no other cell comes within its
-// radius, and listed for the neighbour-cell pass otherwise.
+// radius, and listed for the neighbour-cell pass otherwise.  Eight lanes take
+// a point and test 16 points of its cell at a time, half after and half before
+// it (its scan-order neighbours): the pass waits for chains of loads, and one
+// lane testing one point at a time made them up to 64 tests long (one 64x2048
+// frame 29 -> 7.5 us, a snowy 64x1801 one 30 -> 12, 32 frames at a time 37 ->
+// 19).
 __global__ __launch_bounds__(256) void k_noise_count(DevBuf d, Layout L) {
+    __shared__ uint32_t rsv[256 / kWave + 1];
     int tile, f;
     xcd_tile_frame(tile, f);
     const int nopen = static_cast<int>(d.fs[f * kFsCount + kFsNoiseOpen]);
     const NoiseConst nc = *d.nc;
     const size_t po = (size_t)f * L.N;
     const size_t ho = (size_t)f * L.hash_cap;
-    for (int q = tile * blockDim.x + threadIdx.x; q < nopen; q += gridDim.x * blockDim.x) {
-        const int i = d.nopen[po + q];
+    const int sub = static_cast<int>(threadIdx.x) % kOwnLanes;
+    const int group = lane_id() & ~(kOwnLanes - 1);  // the group's first lane
+    constexpr int kPoints = 256 / kOwnLanes;
+    const uint32_t k = nc.k;
+    for (int q0 = tile * kPoints; q0 < nopen; q0 += static_cast<int>(gridDim.x) * kPoints) {
+        // Past the list's end the last point is tested again and not written.
+        const int q = q0 + static_cast<int>(threadIdx.x) / kOwnLanes;
+        const int i = d.nopen[po + min(q, nopen - 1)];
         const int pos = d.spos[po + i];
-        noise_own_cell(d, nc, f, po, ho, i, pos);
+        const float4 t = d.dsort[po + pos];
+        const float r2 = noise_radius_sqr(nc, t.x, t.y);
+        int state;  // 0 VALID, 1 NOISE, 2 listed
+        uint32_t carry = 0;  // listed: own-cell count and how far the scan got
+        if (k == 0) {
+            state = 0;
+        } else if (!(r2 >= 0.0f)) {
+            state = 1;  // a NaN radius admits no point
+        } else {
+            const HashSlot hv = d.hslot[ho + __float_as_int(t.w)];
+            const int s0 = hv.aux;
+            const int s1 = s0 + static_cast<int>(hv.count);
+            uint32_t cnt = 0;
+            int up = pos, dn = pos - 1;  // [dn + 1, up) is tested
+            while (cnt < k && up - 1 - dn < kOwnCellBudget && (up < s1 || dn >= s0)) {
+                const int after = min(s1 - up, max(kOwnTests / 2, kOwnTests - (dn + 1 - s0)));
+                const int before = min(dn + 1 - s0, kOwnTests - after);
+                float4 p[kOwnTests / kOwnLanes];
+#pragma unroll
+                for (int u = 0; u < kOwnTests / kOwnLanes; ++u) {
+                    const int e = min(u * kOwnLanes + sub, after + before - 1);
+                    p[u] = d.dsort[po + (e < after ? up + e : dn - (e - after))];
+                }
+#pragma unroll
+                for (int u = 0; u < kOwnTests / kOwnLanes; ++u) {
+                    const bool hit = u * kOwnLanes + sub < after + before && noise_dist(t, p[u]) <= r2;
+                    cnt += static_cast<uint32_t>(__popcll((__ballot(hit) >> group) & ((1ull << kOwnLanes) - 1ull)));
+                }
+                up += after;
+                dn -= before;
+            }
+            if (cnt >= k) {
+                state = 0;
+            } else {
+                state = 2;
+                carry = cnt | static_cast<uint32_t>(up - pos) << 8 | static_cast<uint32_t>(pos - 1 - dn) << 16;
+                const float r = sqrtf(r2);
+                int cx, cy, cz;
+                noise_cell(t.x, t.y, t.z, cx, cy, cz);
+                const bool whole = up >= s1 && dn < s0;
+                const bool interior = cx > 0 && cx < 1023 && cy > 0 && cy < 1023 && cz > 0 && cz < 2047;
+                if (whole && interior && r < static_cast<float>(kNoiseMaxExtent - 1)) {
+                    const float fx = t.x - floorf(t.x), fy = t.y - floorf(t.y), fz = t.z - floorf(t.z);
+                    const float reach = (r + kNoiseCellSlack) * (r + kNoiseCellSlack);
+                    if (cell_gap_sqr(fx, fy, fz, -1, 0, 0) > reach && cell_gap_sqr(fx, fy, fz, 1, 0, 0) > reach &&
+                        cell_gap_sqr(fx, fy, fz, 0, -1, 0) > reach && cell_gap_sqr(fx, fy, fz, 0, 1, 0) > reach &&
+                        cell_gap_sqr(fx, fy, fz, 0, 0, -1) > reach && cell_gap_sqr(fx, fy, fz, 0, 0, 1) > reach)
+                        state = 1;
+                }
+            }
+        }
+        const bool writes = sub == 0 && q < nopen;
+        const bool listed[1] = {writes && state == 2};
+        uint32_t p[1];
+        block_reserve<1>(&d.fs[f * kFsCount + kFsNoiseHard], listed, p, rsv);
+        if (listed[0]) {
+            d.vslot[po + p[0]] = pos;  // the listed point: position, input index and carry, loaded side by side
+            d.nloc[po + p[0]] = i;
+            d.obs_src[po + p[0]] = static_cast<int32_t>(carry);
+        } else if (writes) {
+            d.noise[po + i] = state == 1 ? 1 : 0;
+        }
+        __syncthreads();
     }
 }
 
@@ -346,13 +383,26 @@ __global__ __launch_bounds__(256) void k_noise_count(DevBuf d, Layout L) {
 // occupied (one bit per 1 m (x, y) column), cell present in the hash.  The
 // search stops at the min_neighbours-th hit.  Radii of 3 m and more (ranges
 // beyond ~150 m) scan the whole frame.
+// Runs of 64 points whose loads are in flight together.  The pass waits for
+// the wavefronts that scan full cells, run after run, so this decides its time:
+// one 64x2048 frame 20.7 us with one run, 14.4 with four, no less with eight
+// (and 28.8 with a quarter of the wavefronts and their atomics on one noise
+// counter); the snowy 64x1801 one 23.5, now 15.9 (33.8).
+constexpr int kScanRows = 4;
+constexpr int kFoundRows = 4;
+
 __device__ __forceinline__ uint32_t wave_count_range(const DevBuf& d, size_t po, const float4& t, float r2, int a,
                                                      int b, uint32_t cnt, uint32_t k) {
     const int lane = lane_id();
-    for (int base = a; base < b && cnt < k; base += kWave) {
-        const int s = base + lane;
-        const bool hit = s < b && noise_dist(t, d.dsort[po + s]) <= r2;
-        cnt += static_cast<uint32_t>(__popcll(__ballot(hit)));
+    for (int base = a; base < b && cnt < k; base += kScanRows * kWave) {
+        float4 p[kScanRows];
+#pragma unroll
+        for (int u = 0; u < kScanRows; ++u) p[u] = d.dsort[po + min(base + u * kWave + lane, b - 1)];
+#pragma unroll
+        for (int u = 0; u < kScanRows; ++u) {
+            const bool hit = base + u * kWave + lane < b && noise_dist(t, p[u]) <= r2;
+            cnt += static_cast<uint32_t>(__popcll(__ballot(hit)));
+        }
     }
     return cnt;
 }
@@ -371,7 +421,6 @@ __global__ __launch_bounds__(256) void k_noise_search(DevBuf d, Layout L) {
     const uint32_t mask = static_cast<uint32_t>(L.hash_cap) - 1;
     const uint32_t k = nc.k;
     const uint32_t* occ = d.nocc + (size_t)f * kNoiseOccWords;
-    uint32_t noise_here = 0;
     for (int q = tile * (blockDim.x / kWave) + threadIdx.x / kWave; q < nhard; q += waves) {
         const int pos = d.vslot[po + q];
         const int i = d.nloc[po + q];
@@ -421,20 +470,27 @@ __global__ __launch_bounds__(256) void k_noise_search(DevBuf d, Layout L) {
                     const int incl = wave_inclusive_sum(c_n);
                     const int found = __shfl(incl, kWave - 1, kWave);
                     const int start = c_a - (incl - c_n);  // point g of this lane's cell: start + g
-                    for (int base = 0; base < found && cnt < k; base += kWave) {
-                        const int g = base + lane;
-                        int lo = 0, hi = kWave - 1;
+                    for (int base = 0; base < found && cnt < k; base += kFoundRows * kWave) {
+                        float4 p[kFoundRows];
 #pragma unroll
-                        for (int it = 0; it < 6; ++it) {
-                            const int mid = (lo + hi) >> 1;
-                            if (__shfl(incl, mid, kWave) > g)
-                                hi = mid;
-                            else
-                                lo = mid + 1;
+                        for (int u = 0; u < kFoundRows; ++u) {
+                            const int g = min(base + u * kWave + lane, found - 1);
+                            int lo = 0, hi = kWave - 1;
+#pragma unroll
+                            for (int it = 0; it < 6; ++it) {
+                                const int mid = (lo + hi) >> 1;
+                                if (__shfl(incl, mid, kWave) > g)
+                                    hi = mid;
+                                else
+                                    lo = mid + 1;
+                            }
+                            p[u] = d.dsort[po + __shfl(start, lo, kWave) + g];
                         }
-                        const int sp = __shfl(start, lo, kWave) + g;
-                        const bool hit = g < found && noise_dist(t, d.dsort[po + sp]) <= r2;
-                        cnt += static_cast<uint32_t>(__popcll(__ballot(hit)));
+#pragma unroll
+                        for (int u = 0; u < kFoundRows; ++u) {
+                            const bool hit = base + u * kWave + lane < found && noise_dist(t, p[u]) <= r2;
+                            cnt += static_cast<uint32_t>(__popcll(__ballot(hit)));
+                        }
                     }
                 }
             }
@@ -442,23 +498,21 @@ __global__ __launch_bounds__(256) void k_noise_search(DevBuf d, Layout L) {
             // Radius beyond the cell cube (range > ~150 m) or infinite.
             cnt = wave_count_range(d, po, t, r2, 0, n, 0u, k);
         }
-        if (lane == 0) {
-            const bool noise = cnt < k;
-            d.noise[po + i] = noise ? 1 : 0;
-            noise_here += noise ? 1u : 0u;
-        }
+        if (lane == 0) d.noise[po + i] = cnt < k ? 1 : 0;
     }
-    if (lane == 0 && noise_here) atomicAdd(&d.fs[f * kFsCount + kFsNoise], noise_here);
 }
 
 // Stable compaction of the kept points (label 0) into the segmenter's
-// inputs, in two passes over tiles of 2048 points (eight rows of 256, each
+// inputs, in two passes over tiles of 1024 points (two rows of 512, each
 // read and written with coalesced accesses): the kept count of every tile,
 // then each tile's compaction after the counts of the tiles before it, which
 // moves x, y, z, ring to their places.  The keep flags are the label bytes;
 // the last tile writes the kept count, which becomes the frame's point count.
-constexpr int kKeepThreads = 256;
-constexpr int kKeepRows = 8;
+// Workgroups of the first pass from `tiles` on clear the cells' hash slots.
+// (One 64x2048 frame: both passes and the table's clearing 21 -> 10.5 us,
+// of which the second pass 5.6; with eight rows of 256 it took 11.7.)
+constexpr int kKeepThreads = 512;
+constexpr int kKeepRows = 2;
 constexpr int kKeepTile = kKeepThreads * kKeepRows;
 
 __device__ __forceinline__ uint32_t keep_bits(const uint8_t* lab, int base, int n) {
@@ -471,9 +525,15 @@ __device__ __forceinline__ uint32_t keep_bits(const uint8_t* lab, int base, int 
     return m;
 }
 
-__global__ __launch_bounds__(kKeepThreads) void k_keep_count(DevBuf d, Layout L) {
+__global__ __launch_bounds__(kKeepThreads) void k_keep_count(DevBuf d, Layout L, int tiles) {
     __shared__ uint32_t lds[kKeepThreads / kWave + 1];
     const int f = blockIdx.y;
+    if (static_cast<int>(blockIdx.x) >= tiles) {
+        reset_slots(d, L, f, d.ncell_slot, kFsNoiseCells,
+                    (static_cast<int>(blockIdx.x) - tiles) * kKeepThreads + static_cast<int>(threadIdx.x),
+                    (static_cast<int>(gridDim.x) - tiles) * kKeepThreads);
+        return;
+    }
     const int n = d.frames[f].n_raw;
     const int base = blockIdx.x * kKeepTile;
     if (base >= n) return;
@@ -483,7 +543,7 @@ __global__ __launch_bounds__(kKeepThreads) void k_keep_count(DevBuf d, Layout L)
     if (threadIdx.x == 0) d.blk[(size_t)f * L.blk_stride + blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(kKeepThreads) void k_keep_move(DevBuf d, Layout L) {
+__global__ __launch_bounds__(kKeepThreads) void k_keep_move(DevBuf d, Layout L, bool count_noise) {
     __shared__ uint32_t lds[kKeepRows * kKeepThreads / kWave + 1];
     const int f = blockIdx.y;
     FrameDesc& fd = d.frames[f];
@@ -521,6 +581,7 @@ __global__ __launch_bounds__(kKeepThreads) void k_keep_move(DevBuf d, Layout L) 
     if (threadIdx.x == 0 && base + kKeepTile >= n) {
         const uint32_t kept = pre_total + total;
         d.fs[f * kFsCount + kFsKept] = kept;
+        if (count_noise) d.fs[f * kFsCount + kFsNoise] = static_cast<uint32_t>(n) - kept;
         fd.n = static_cast<int32_t>(kept);
     }
 }
@@ -535,29 +596,30 @@ void launch_noise(lp_context* c, int B, bool compact) {
     stage_mark(c, "noise");
     hipLaunchKernelGGL(k_noise_clear, dim3(256, B), dim3(256), 0, st, d, L);
     hipLaunchKernelGGL(k_noise_prep, dim3((L.N + kPrepTile - 1) / kPrepTile, B), dim3(256), 0, st, d, L);
-    // Cell starts (exclusive scan of the counts by dense id) straight into
-    // the slots' aux fields.
-    launch_scan_gather_into(c, B, &d.hslot[0].count, L.hash_cap, 4, d.ncell_slot,
-                            reinterpret_cast<uint32_t*>(&d.hslot[0].aux), L.N, kCountSlot, kFsNoiseCells);
+    // About the cells of a 64x2048 frame per 32 workgroups.
+    hipLaunchKernelGGL(k_noise_cells, dim3(std::min(nb, 64), B), dim3(256), 0, st, d, L);
     hipLaunchKernelGGL(k_noise_scatter, dim3(nb, B), dim3(256), 0, st, d, L);
     stage_mark(c, "noise_count");
-    // The open list is a few percent of the points: a quarter of the point
-    // grid, striding over the list.
+    // The open list is a few percent of the points, eight lanes for each: a
+    // quarter of the point grid, striding over the list.
     hipLaunchKernelGGL(k_noise_count, dim3((nb + 3) / 4, B), dim3(256), 0, st, d, L);
     stage_mark(c, "noise_search");
     // About 8192 wavefronts in all (8 per SIMD: the search is latency-bound),
-    // at least 128 and at most 1024 per frame.
-    const int sb = std::min(256, std::max(32, 2048 / B));
+    // at least 128 and at most 4096 per frame.
+    const int sb = std::min(1024, std::max(32, 2048 / B));
     hipLaunchKernelGGL(k_noise_search, dim3(sb, B), dim3(256), 0, st, d, L);
-    launch_hash_reset(c, B, d.ncell_slot, kFsNoiseCells);
     stage_mark(c, "noise_compact");
-    if (compact) launch_noise_compact(c, B);
+    if (compact)
+        launch_noise_compact(c, B, true);
+    else
+        launch_hash_reset(c, B, d.ncell_slot, kFsNoiseCells);
 }
 
-void launch_noise_compact(lp_context* c, int B) {
+void launch_noise_compact(lp_context* c, int B, bool radius_rule) {
     const int nt = (c->L.N + kKeepTile - 1) / kKeepTile;  // at most blk_stride tiles
-    hipLaunchKernelGGL(k_keep_count, dim3(nt, B), dim3(kKeepThreads), 0, c->stream, c->d, c->L);
-    hipLaunchKernelGGL(k_keep_move, dim3(nt, B), dim3(kKeepThreads), 0, c->stream, c->d, c->L);
+    hipLaunchKernelGGL(k_keep_count, dim3(nt + (radius_rule ? kResetTiles : 0), B), dim3(kKeepThreads), 0, c->stream,
+                       c->d, c->L, nt);
+    hipLaunchKernelGGL(k_keep_move, dim3(nt, B), dim3(kKeepThreads), 0, c->stream, c->d, c->L, radius_rule);
 }
 
 }  // namespace lp

@@ -795,7 +795,7 @@ void launch_noise_kdtree(lp_context* c, int B, bool compact) {
     stage_mark(c, "noise_search");
     hipLaunchKernelGGL(k_kd_resolve, dim3(B), dim3(kKdResolveThreads), 0, st, d, L);
     stage_mark(c, "noise_compact");
-    if (compact) launch_noise_compact(c, B);
+    if (compact) launch_noise_compact(c, B, false);
 }
 
 }  // namespace lp
