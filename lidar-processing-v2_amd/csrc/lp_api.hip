@@ -406,7 +406,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.state, B * P);
     go(x.mapping, B * P);
     go(x.pxyz, B * P);
-    go(x.qflag, B * P);
+    go(x.qmask, B * static_cast<size_t>(L.qruns));
     go(x.qmap, B * P);
     go(x.qlist, B * P);
     go(x.qrow, B * (L.H + 1));
@@ -861,6 +861,7 @@ int create_lane(const lp_capacity* cap, lp_context** out) {
     L.blk_stride = std::max((std::max({L.N, L.P, L.hash_cap}) + 2047) / 2048, (L.N + 1023) / 1024) + 1;
     L.box_stride = L.N / 3 + 1024;
     L.obs_rows = (L.N + 63) / 64;
+    L.qruns = L.H * ((L.W + 63) / 64);
     const size_t bytes = layout_bytes(L, nullptr, nullptr);
     hipError_t e = hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking);
     if (e == hipSuccess) e = hipMalloc(&c->arena, bytes);

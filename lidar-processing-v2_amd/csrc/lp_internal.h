@@ -151,7 +151,7 @@ struct DevBuf {
     uint8_t* state;
     int32_t* mapping;
     float4* pxyz;            // per pixel: the winner's x, y, z and its index (int bits, -1 when empty)
-    uint8_t* qflag;          // 1: the pixel joins the JCP queue
+    uint64_t* qmask;         // [frame][qruns] per 64 columns of a row, the pixels that join the JCP queue
     int32_t* qmap;
     // JCP queue (frame stride pix_stride)
     int32_t* qlist;
@@ -275,6 +275,7 @@ struct Layout {
     int32_t blk_stride;     // scan block sums per frame
     int32_t box_stride;     // oriented boxes per frame (capacity)
     int32_t obs_rows;       // runs of 64 points per frame
+    int32_t qruns;          // runs of 64 columns per frame
 };
 
 }  // namespace lp

@@ -47,7 +47,11 @@ constexpr int32_t kSrcObstacle = -3;
 // clipped to the image (the dilated red channel of segmenter.cpp:484-513).
 // Each workgroup takes T columns of one row (T = 64, 128 or 256, the
 // tile width the launch chooses) and stages rows r-2..r+2 of columns
-// c0-2..c0+T+1 in LDS (out-of-image pixels read as empty).
+// c0-2..c0+T+1 in LDS (out-of-image pixels read as empty).  The flags of a
+// wavefront's 64 columns leave as one word, bit b for column 64 * k + b of the
+// row's run k.
+__device__ __forceinline__ int queue_runs(int W) { return (W + kWave - 1) / kWave; }  // runs per row
+
 template <int T>
 __global__ __launch_bounds__(T) void k_jcp_mark(DevBuf d, Layout L) {
     constexpr int kSpan = T + 4;
@@ -65,89 +69,72 @@ __global__ __launch_bounds__(T) void k_jcp_mark(DevBuf d, Layout L) {
     }
     __syncthreads();
     const int c = c0 + static_cast<int>(threadIdx.x);
-    if (c >= W) return;
     uint32_t q = 0;
-    if (win[2][threadIdx.x + 2] == kGround) {
+    if (c < W && win[2][threadIdx.x + 2] == kGround) {
 #pragma unroll
         for (int dr = 0; dr < 5; ++dr)
 #pragma unroll
             for (int dc = 0; dc < 5; ++dc) q |= win[dr][threadIdx.x + dc] == kObstacle ? 1u : 0u;
     }
-    d.qflag[(size_t)f * L.P + r * W + c] = static_cast<uint8_t>(q);
+    const uint64_t mask = __ballot(q != 0);
+    if (lane_id() == 0 && c < W) d.qmask[(size_t)f * L.qruns + r * queue_runs(W) + c / kWave] = mask;
 }
 
-// The queue in raster order, from the flags in two passes over tiles of 2048
-// pixels (eight rows of 256, coalesced): the queue count of every tile, then
-// each tile's compaction after the counts of the tiles before it.  qlist[j]
-// is the pixel of queue entry j, qmap[p] the queue index of pixel p or, for a
-// pixel that is not queued, its static label source (negative), qrow[r] the
-// first queue index at or after row r's first pixel (kept for the row solve);
-// the last tile writes the queue length.
-constexpr int kQueueThreads = 256;
-constexpr int kQueueRows = 8;
-constexpr int kQueueTile = kQueueThreads * kQueueRows;
+// The queue in raster order: a workgroup compacts 32 runs of 64 pixels, after
+// the queue pixels of the runs before, which it counts itself (a launch that
+// left the count of every tile cost more: one 64x2048 frame 13.3 -> 7.5 us).
+// qlist[j] is the pixel of queue entry j, qmap[p] the queue index of pixel p
+// or, for a pixel that is not queued, its static label source (negative),
+// qrow[r] the first queue index at or after row r's first pixel (kept for the
+// row solve); the last tile writes the queue length.
+constexpr int kFillThreads = 256;
+constexpr int kFillRuns = 8;  // per wavefront, their loads in flight together
+constexpr int kFillTile = kFillRuns * kFillThreads / kWave;
 
-__device__ __forceinline__ uint32_t queue_bits(const uint8_t* qf, int base, int P) {
-    uint32_t m = 0;
-#pragma unroll
-    for (int k = 0; k < kQueueRows; ++k) {
-        const int p = base + k * kQueueThreads + static_cast<int>(threadIdx.x);
-        m |= (p < P && qf[p] != 0) ? (1u << k) : 0u;
-    }
-    return m;
-}
-
-__global__ __launch_bounds__(kQueueThreads) void k_jcp_count(DevBuf d, Layout L) {
-    __shared__ uint32_t lds[kQueueThreads / kWave + 1];
-    const int f = blockIdx.y;
-    const FrameDesc& fd = d.frames[f];
-    const int P = fd.sc.H * fd.sc.W;
-    const int base = blockIdx.x * kQueueTile;
-    if (base >= P) return;
-    const uint32_t m = queue_bits(d.qflag + (size_t)f * L.P, base, P);
-    uint32_t total;
-    block_exclusive_sum<kQueueThreads>(static_cast<uint32_t>(__popc(m)), lds, &total);
-    if (threadIdx.x == 0) d.blk[(size_t)f * L.blk_stride + blockIdx.x] = total;
-}
-
-__global__ __launch_bounds__(kQueueThreads) void k_jcp_fill(DevBuf d, Layout L) {
-    __shared__ uint32_t lds[kQueueRows * kQueueThreads / kWave + 1];
+__global__ __launch_bounds__(kFillThreads) void k_jcp_fill(DevBuf d, Layout L) {
+    __shared__ uint32_t lds[kFillThreads / kWave + 1];
     const int f = blockIdx.y;
     const FrameDesc& fd = d.frames[f];
     const int W = fd.sc.W;
-    const int P = fd.sc.H * W;
-    const int tile = blockIdx.x;
-    const int base = tile * kQueueTile;
-    if (base >= P) {
-        if (tile == 0 && threadIdx.x == 0) d.fs[f * kFsCount + kFsQueue] = 0;
-        return;
-    }
-    const uint32_t* blk = d.blk + (size_t)f * L.blk_stride;
-    uint32_t pre = 0;
-    for (int i = threadIdx.x; i < tile; i += kQueueThreads) pre += blk[i];
-    uint32_t pre_total;
-    block_exclusive_sum<kQueueThreads>(pre, lds, &pre_total);
+    const int per_row = queue_runs(W);
+    const int runs = fd.sc.H * per_row;
+    const int first = static_cast<int>(blockIdx.x) * kFillTile;
+    if (first >= runs) return;
+    const uint64_t* mask = d.qmask + (size_t)f * L.qruns;
+    const int lane = lane_id();
+    const int w = static_cast<int>(threadIdx.x) / kWave;
     const size_t po = (size_t)f * L.P;
-    const uint32_t m = queue_bits(d.qflag + po, base, P);
-    uint32_t pos[kQueueRows];
-    const uint32_t total = tile_compact<kQueueThreads, kQueueRows>(m, pos, lds);
+    int p[kFillRuns];
+    uint8_t st[kFillRuns];
 #pragma unroll
-    for (int k = 0; k < kQueueRows; ++k) {
-        const int p = base + k * kQueueThreads + static_cast<int>(threadIdx.x);
-        if (p >= P) continue;
-        const int j = static_cast<int>(pre_total + pos[k]);
-        if (p % W == 0) d.qrow[(size_t)f * (L.H + 1) + p / W] = j;
-        if ((m >> k) & 1u) {
-            d.qlist[po + j] = p;
-            d.qmap[po + p] = j;
+    for (int k = 0; k < kFillRuns; ++k) {
+        const int run = first + w * kFillRuns + k;
+        const int c = run % per_row * kWave + lane;
+        p[k] = run < runs && c < W ? run / per_row * W + c : -1;
+        st[k] = d.state[fd.pix_off + max(p[k], 0)];
+    }
+    // Every wavefront has the tile's masks and their sums, a run per lane.
+    const uint64_t mine = lane < kFillTile && first + lane < runs ? mask[first + lane] : 0ull;
+    uint32_t before = 0, base;
+    for (int i = threadIdx.x; i < first; i += kFillThreads) before += static_cast<uint32_t>(__popcll(mask[i]));
+    block_exclusive_sum<kFillThreads>(before, lds, &base);
+    const uint32_t incl = base + wave_inclusive_sum(static_cast<uint32_t>(__popcll(mine)));
+#pragma unroll
+    for (int k = 0; k < kFillRuns; ++k) {
+        const uint64_t m = __shfl(mine, w * kFillRuns + k, kWave);
+        const uint32_t end = __shfl(incl, w * kFillRuns + k, kWave);
+        if (p[k] < 0) continue;
+        const int j = static_cast<int>(end - static_cast<uint32_t>(__popcll(m >> lane)));
+        if (p[k] % W == 0) d.qrow[(size_t)f * (L.H + 1) + p[k] / W] = j;
+        if ((m >> lane) & 1ull) {
+            d.qlist[po + j] = p[k];
+            d.qmap[po + p[k]] = j;
         } else {
-            const uint8_t st = d.state[fd.pix_off + p];
-            d.qmap[po + p] = st == kGround ? kSrcGround : (st == kObstacle ? kSrcObstacle : kSrcUnknown);
+            d.qmap[po + p[k]] = st[k] == kGround ? kSrcGround : (st[k] == kObstacle ? kSrcObstacle : kSrcUnknown);
         }
     }
-    if (threadIdx.x == 0 && base + kQueueTile >= P) d.fs[f * kFsCount + kFsQueue] = pre_total + total;
+    if (threadIdx.x == kWave - 1 && first + kFillTile >= runs) d.fs[f * kFsCount + kFsQueue] = incl;
 }
-
 
 // A queue pixel's slots, as the row solve reads them: the head slots 0..11
 // (rows -2, -1 and the two left neighbours) with their weights and label
@@ -200,111 +187,140 @@ __device__ __forceinline__ SlotVal eval_slot(const SegConst& s, int pe, float4 c
 }
 
 // Per queue pixel: the 24 slot weights w_i = u_i / sum and label sources,
-// including stale slots resolved through their writer.  Bound by the latency
-// of the neighbour reads, so all 24 records and sources of a pixel are
-// requested before the first is used (clamped into the image; a slot outside
-// it is stale and read again through its writer): 35 -> 22 us for one 64x2048
-// frame, 65 -> 49 us for 32.
-__global__ __launch_bounds__(256) void k_jcp_slots(DevBuf d, Layout L) {
+// including stale slots resolved through their writer.  A workgroup takes 64
+// queue pixels and a wavefront four slots of each, lane by lane consecutive
+// pixels, so its reads are mostly neighbours; the slots meet in LDS for the
+// ordered sums.  With a lane doing all 24 slots of a pixel the code was long,
+// straight and cold in every launch, and few wavefronts had work (35 us for
+// one 64x2048 frame with the records read one after the other, 22 with all of
+// them requested first, now 8.5; 32x1024 20 -> 7.3; eight 128x2048 frames 28 ->
+// 19; 32 frames of 64x2048 keep the chip busy either way, 51 us).
+constexpr int kSlotWaves = 6;
+constexpr int kWaveSlots = 24 / kSlotWaves;
+static_assert(kWaveSlots == 4, "a wavefront's weights are one part of the record");
+
+__global__ __launch_bounds__(kSlotWaves* kWave) void k_jcp_slots(DevBuf d, Layout L) {
+    __shared__ float lw[24][kWave];     // u, then the weights
+    __shared__ float ltail[12][kWave];  // signed tail weights
+    __shared__ uint32_t lent[12][kWave];
     int tile, f;
     xcd_tile_frame(tile, f);
     const FrameDesc& fd = d.frames[f];
     const SegConst& s = fd.sc;
     const int nq = static_cast<int>(d.fs[f * kFsCount + kFsQueue]);
-    const int j = tile * blockDim.x + threadIdx.x;
-    if (j >= nq) return;
+    const int lane = lane_id();
+    const int w = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x) / kWave);
     const int H = s.H, W = s.W;
     const float4* px = d.pxyz + fd.pix_off;
     const size_t qo = (size_t)f * L.P;
     const int32_t* qm = d.qmap + qo;
     const int32_t* ql = d.qlist + qo;
     const int32_t* qrow = d.qrow + (size_t)f * (L.H + 1);
-    const int p = ql[j];
-    const int r = p / W, c = p % W;
-    const float4 core = px[p];
-    float4 nb[24];
-    int32_t nq_src[24];
-#pragma unroll
-    for (int i = 0; i < 24; ++i) {
-        const int np = min(max(r + kOffR[i], 0), H - 1) * W + min(max(c + kOffC[i], 0), W - 1);
-        nb[i] = px[np];
-        nq_src[i] = qm[np];
-    }
-    float u[24];
-    int32_t src[24];
-    float sum = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 24; ++i) {
-        const int dr = kOffR[i], dc = kOffC[i];
-        const int nr = r + dr, nc = c + dc;
-        if (nr >= 0 && nr < H && nc >= 0 && nc < W) {
-            const SlotVal v = eval_slot(s, p, core, nr * W + nc, nb[i], nq_src[i]);
-            u[i] = v.u;
-            src[i] = v.src;
-            if (v.near) sum += v.u;
-        } else {
-            // Stale slot: find the last earlier queue pixel for which this
-            // slot was inside the image.
-            const int rlo = max(0, -dr), rhi = min(H, H - dr);
-            const int clo = max(0, -dc), chi = min(W, W - dc);
-            // None in an image too small for the slot: rows rlo .. rhi - 1
-            // exist below.
-            int khi = rlo < rhi ? j - 1 : -1, klo = 0;
-            // First queue index at or after a row's first pixel: qrow.
-            if (rlo < rhi && rhi < H) khi = min(khi, qrow[rhi] - 1);
-            if (rlo < rhi && rlo > 0) klo = qrow[rlo];
-            int q = -1;
-            for (int k = khi; k >= klo && q < 0; --k) {
-                const int pk = ql[k], qc = pk % W;
-                if (qc >= clo && qc < chi) q = pk;
-            }
-            if (q >= 0) {
-                const int np = (q / W + dr) * W + q % W + dc;
-                const SlotVal v = eval_slot(s, q, px[q], np, px[np], qm[np]);
-                u[i] = v.u;
-                src[i] = v.src;
+    const size_t P = static_cast<size_t>(L.P);
+    for (int j0 = tile * kWave; j0 < nq; j0 += static_cast<int>(gridDim.x) * kWave) {
+        const int j = min(j0 + lane, nq - 1);  // past the end: the last one again, not written
+        const bool mine = j0 + lane < nq;
+        const int p = ql[j];
+        const int r = p / W, c = p % W;
+        const float4 core = px[p];
+        float4 nb[kWaveSlots];
+        int32_t nq_src[kWaveSlots];
+    #pragma unroll
+        for (int k = 0; k < kWaveSlots; ++k) {
+            const int i = w * kWaveSlots + k;
+            const int np = min(max(r + kOffR[i], 0), H - 1) * W + min(max(c + kOffC[i], 0), W - 1);
+            nb[k] = px[np];
+            nq_src[k] = qm[np];
+        }
+        float u[kWaveSlots];
+        int32_t src[kWaveSlots];
+    #pragma unroll
+        for (int k = 0; k < kWaveSlots; ++k) {
+            const int dr = kOffR[w * kWaveSlots + k], dc = kOffC[w * kWaveSlots + k];
+            const int nr = r + dr, nc = c + dc;
+            SlotVal v{0.0f, kSrcUnknown, false};  // slots start at zero / UNKNOWN (segmenter.cpp:523-525)
+            if (nr >= 0 && nr < H && nc >= 0 && nc < W) {
+                v = eval_slot(s, p, core, nr * W + nc, nb[k], nq_src[k]);
             } else {
-                u[i] = 0.0f;  // slots start at zero / UNKNOWN (segmenter.cpp:523-525)
-                src[i] = kSrcUnknown;
+                // Stale slot: find the last earlier queue pixel for which this
+                // slot was inside the image.
+                const int rlo = max(0, -dr), rhi = min(H, H - dr);
+                const int clo = max(0, -dc), chi = min(W, W - dc);
+                // None in an image too small for the slot: rows rlo .. rhi - 1
+                // exist below.
+                int khi = rlo < rhi ? j - 1 : -1, klo = 0;
+                // First queue index at or after a row's first pixel: qrow.
+                if (rlo < rhi && rhi < H) khi = min(khi, qrow[rhi] - 1);
+                if (rlo < rhi && rlo > 0) klo = qrow[rlo];
+                int q = -1;
+                for (int e = khi; e >= klo && q < 0; --e) {
+                    const int pk = ql[e], qc = pk % W;
+                    if (qc >= clo && qc < chi) q = pk;
+                }
+                if (q >= 0) {
+                    const int np = (q / W + dr) * W + q % W + dc;
+                    v = eval_slot(s, q, px[q], np, px[np], qm[np]);
+                    v.near = false;  // no part of this pixel's sum
+                }
+            }
+            u[k] = v.u;
+            src[k] = v.src;
+            // What the sum takes: slots without a near neighbour add nothing
+            // (their u is +0 as the sum's start is, so adding it changes nothing).
+            lw[w * kWaveSlots + k][lane] = v.near ? v.u : 0.0f;
+        }
+        __syncthreads();
+        float sum = 0.0f;
+    #pragma unroll
+        for (int i = 0; i < 24; ++i) sum += lw[i][lane];
+        __syncthreads();
+        const bool ok = fabsf(sum) > 1.1920928955078125e-07f;  // FLT_EPSILON
+        // An infinite sum makes every weight 0 or NaN: the reference's comparison
+        // is false then, as it is without any weight.
+        const bool weigh = ok && sum < __builtin_inff();
+        uint4* rec = d.slot_rec + qo * kRecordParts + j;
+        float part[kWaveSlots];
+    #pragma unroll
+        for (int k = 0; k < kWaveSlots; ++k) {
+            const int i = w * kWaveSlots + k;
+            const float t = weigh ? u[k] / sum : 0.0f;
+            lw[i][lane] = t;
+            if (i < 12) {
+                part[k] = t;
+                lent[i][lane] = static_cast<uint32_t>((t > 0.0f ? src[k] : kSrcUnknown) + kLabelBase);
+            } else {
+                part[k] = src[k] == kSrcObstacle ? t : (src[k] == kSrcGround ? -t : 0.0f);
+                ltail[i - 12][lane] = part[k];
             }
         }
+        if (mine)
+            rec[(w < 3 ? w : w + 2) * P] = make_uint4(__float_as_uint(part[0]), __float_as_uint(part[1]),
+                                                      __float_as_uint(part[2]), __float_as_uint(part[3]));
+        __syncthreads();
+        if (w == 0 && mine) {
+            uint32_t flags = ok ? kRecOk : 0u;
+            float tail_sum = 0.0f, total = 0.0f;
+            uint32_t entry[12];
+        #pragma unroll
+            for (int i = 0; i < 12; ++i) {
+                const uint32_t e = lent[i][lane];
+                entry[i] = e & 0xffffu;
+                flags |= (e >> 16) << i;
+                const float t = ltail[i][lane];
+                tail_sum += t;
+                if (t != 0.0f) flags |= kRecTail;
+                total += lw[i][lane] + lw[12 + i][lane];
+            }
+            // The pixel's own weights sum to 1; stale ones come on top, divided by a
+            // sum they are not part of.
+            if (total > 1.5f) flags |= min(((__float_as_uint(total) >> 23) & 0xffu) - 126u, 140u) << kRecScale;
+            rec[3 * P] = make_uint4(entry[0] | entry[1] << 16, entry[2] | entry[3] << 16, entry[4] | entry[5] << 16,
+                                    entry[6] | entry[7] << 16);
+            rec[4 * P] =
+                make_uint4(entry[8] | entry[9] << 16, entry[10] | entry[11] << 16, __float_as_uint(tail_sum), flags);
+        }
+        __syncthreads();
     }
-    const bool ok = fabsf(sum) > 1.1920928955078125e-07f;  // FLT_EPSILON
-    // An infinite sum makes every weight 0 or NaN: the reference's comparison
-    // is false then, as it is without any weight.
-    const bool weigh = ok && sum < __builtin_inff();
-    float head[12], tail[12];
-    uint32_t entry[12];
-    uint32_t flags = ok ? kRecOk : 0u;
-    float tail_sum = 0.0f, total = 0.0f;
-#pragma unroll
-    for (int i = 0; i < 12; ++i) {
-        const float w = weigh ? u[i] / sum : 0.0f;
-        const uint32_t e = static_cast<uint32_t>((w > 0.0f ? src[i] : kSrcUnknown) + kLabelBase);
-        head[i] = w;
-        entry[i] = e & 0xffffu;
-        flags |= (e >> 16) << i;
-        const float t = weigh ? u[12 + i] / sum : 0.0f;
-        tail[i] = src[12 + i] == kSrcObstacle ? t : (src[12 + i] == kSrcGround ? -t : 0.0f);
-        tail_sum += tail[i];
-        if (tail[i] != 0.0f) flags |= kRecTail;
-        total += w + t;
-    }
-    // The pixel's own weights sum to 1; stale ones come on top, divided by a
-    // sum they are not part of.
-    if (total > 1.5f) flags |= min(((__float_as_uint(total) >> 23) & 0xffu) - 126u, 140u) << kRecScale;
-    uint4* rec = d.slot_rec + qo * kRecordParts + j;
-    const size_t P = static_cast<size_t>(L.P);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        rec[k * P] = make_uint4(__float_as_uint(head[4 * k]), __float_as_uint(head[4 * k + 1]),
-                                __float_as_uint(head[4 * k + 2]), __float_as_uint(head[4 * k + 3]));
-        rec[(5 + k) * P] = make_uint4(__float_as_uint(tail[4 * k]), __float_as_uint(tail[4 * k + 1]),
-                                      __float_as_uint(tail[4 * k + 2]), __float_as_uint(tail[4 * k + 3]));
-    }
-    rec[3 * P] = make_uint4(entry[0] | entry[1] << 16, entry[2] | entry[3] << 16, entry[4] | entry[5] << 16,
-                            entry[6] | entry[7] << 16);
-    rec[4 * P] = make_uint4(entry[8] | entry[9] << 16, entry[10] | entry[11] << 16, __float_as_uint(tail_sum), flags);
 }
 
 constexpr int kSolveThreads = 512;
@@ -660,7 +676,6 @@ void launch_jcp(lp_context* c, int B) {
     DevBuf& d = c->d;
     const Layout& L = c->L;
     hipStream_t st = c->stream;
-    const int pb = (L.P + 255) / 256;
     stage_mark(c, "jcp_queue");
     const int mt = c->mark_tile;
     if (mt == 64)
@@ -669,11 +684,13 @@ void launch_jcp(lp_context* c, int B) {
         hipLaunchKernelGGL(k_jcp_mark<128>, dim3(L.H * ((L.W + 127) / 128), B), dim3(128), 0, st, d, L);
     else
         hipLaunchKernelGGL(k_jcp_mark<256>, dim3(L.H * ((L.W + 255) / 256), B), dim3(256), 0, st, d, L);
-    const int qt = (L.P + kQueueTile - 1) / kQueueTile;  // at most blk_stride tiles
-    hipLaunchKernelGGL(k_jcp_count, dim3(qt, B), dim3(kQueueThreads), 0, st, d, L);
-    hipLaunchKernelGGL(k_jcp_fill, dim3(qt, B), dim3(kQueueThreads), 0, st, d, L);
+    hipLaunchKernelGGL(k_jcp_fill, dim3((L.qruns + kFillTile - 1) / kFillTile, B), dim3(kFillThreads), 0, st, d, L);
     stage_mark(c, "jcp_slots");
-    hipLaunchKernelGGL(k_jcp_slots, dim3(pb, B), dim3(256), 0, st, d, L);
+    // A workgroup for each 64 pixels of a frame's queue when they are few; on
+    // larger batches about 4096 in all, several turns each (most of a frame's
+    // pixels are not queued, so one for each 64 of them would mostly be empty).
+    hipLaunchKernelGGL(k_jcp_slots, dim3(std::min((L.P + kWave - 1) / kWave, std::max(64, 4096 / B)), B),
+                       dim3(kSlotWaves * kWave), 0, st, d, L);
     stage_mark(c, "jcp_solve");
     hipLaunchKernelGGL(k_jcp_solve, dim3(B), dim3(kSolveThreads), 0, st, d, L);
     stage_mark(c, "labels");
