@@ -1364,8 +1364,8 @@ __global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, const dou
 // all its threads.  The place of its run's vertices in the frame's hull array
 // is the sum of the vertex counts before it, which it adds up itself.  (As
 // three launches, a scan of the counts, the small clusters and the listed large
-// ones, each waited for its slowest cluster: one 64x2048 frame 46 -> 25 us, one
-// 32x1024 frame 37 -> 11 us, eight mixed frames at a time 61 -> 44 us.)  Runs
+// ones, each waited for its slowest cluster: one 64x2048 frame 46 -> 25 us, now 20,
+// one 32x1024 frame 37 -> 11 us, eight mixed frames at a time 61 -> 44 us.)  Runs
 // of one or two clusters, the case of few frames, leave most wavefronts idle,
 // so there a cluster of more than kLocalShortSize members has the workgroup
 // (32x1024 31 -> 11 us); longer runs would take many such clusters in turns.
@@ -1385,10 +1385,28 @@ __device__ __forceinline__ uint32_t xy_hash(double x, double y) {
     return static_cast<uint32_t>(h);
 }
 
-template <int kVMax>
+// An obstacle's coordinates are floats, a standalone list's doubles.
+__device__ __forceinline__ uint32_t xy_hash(float x, float y) {
+    uint32_t h = f2u(x + 0.0f) * 0x9E3779B1u ^ f2u(y + 0.0f) * 0x85EBCA77u;
+    return h ^ h >> 15;
+}
+
+template <typename T>
+__device__ __forceinline__ void member_coords(const DevBuf& d, const double2* list_xy, size_t ob, uint32_t base,
+                                              int32_t m, T& x, T& y) {
+    if constexpr (sizeof(T) == 4) {
+        x = d.ox[ob + m];
+        y = d.oy[ob + m];
+    } else {
+        x = list_xy[base + m].x;
+        y = list_xy[base + m].y;
+    }
+}
+
+template <int kVMax, typename T>
 struct LocalLds {
-    double vx[kVMax];
-    double vy[kVMax];
+    T vx[kVMax];
+    T vy[kVMax];
     int32_t canon[kVMax];
     int32_t sorted[kVMax];
     int32_t table[2 * kVMax];
@@ -1410,9 +1428,14 @@ __device__ __forceinline__ void local_sync() {
         __syncthreads();
 }
 
-// A cluster of at most kVMax hull vertices, by kThreads threads.
-template <int kThreads, int kVMax>
-__device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d, const double2* list_xy, size_t ob,
+// A cluster of at most kVMax hull vertices, by kThreads threads.  What this
+// waits for in the largest cluster of a frame (6528 members and 125 vertices in
+// one of 64x2048): the members' coordinates and their hash; the vertices'
+// order, which a lane per vertex compared with all others one by one; the
+// members' bins, which were a chain of LDS reads each.  All three cut down, the
+// launch took 25.5 -> 20.3 us for that frame and 121 -> 88 us for 32.
+template <int kThreads, int kVMax, typename T>
+__device__ __forceinline__ void local_ranks(LocalLds<kVMax, T>& s, const DevBuf& d, const double2* list_xy, size_t ob,
                                             size_t BN, const LocalCluster& k) {
     constexpr int kLocalHash = 2 * kVMax;
     const int tid = static_cast<int>(threadIdx.x) % kThreads;
@@ -1427,14 +1450,14 @@ __device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d,
     local_sync<kThreads>();
     for (int i = tid; i < V; i += kThreads) {
         const int32_t idx = d.hull_idx[ob + base + i];
-        double x, y;
-        member_xy(d, list_xy, ob, base, idx, x, y);
+        T x, y;
+        member_coords(d, list_xy, ob, base, idx, x, y);
         s.canon[i] = idx;
         s.vx[i] = x;
         s.vy[i] = y;
-        if (!list_xy) {
-            d.hcx[BN + ob + hoff + i] = x;
-            d.hcy[BN + ob + hoff + i] = y;
+        if (sizeof(T) == 4) {
+            d.hcx[BN + ob + hoff + i] = static_cast<double>(x);
+            d.hcy[BN + ob + hoff + i] = static_cast<double>(y);
         }
         uint32_t h = xy_hash(x, y) & hmask;  // load <= 1/2: a free slot exists
         while (atomicCAS(&s.table[h], -1, i) != -1) h = (h + 1) & hmask;
@@ -1443,7 +1466,7 @@ __device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d,
     // Smallest member index per vertex coordinates.
     for (int q0 = tid; q0 < size; q0 += kThreads * kLocalUnroll) {
         int32_t m[kLocalUnroll];
-        double mx[kLocalUnroll], my[kLocalUnroll];
+        T mx[kLocalUnroll], my[kLocalUnroll];
 #pragma unroll
         for (int u = 0; u < kLocalUnroll; ++u) {
             const int q = q0 + u * kThreads;
@@ -1451,7 +1474,7 @@ __device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d,
         }
 #pragma unroll
         for (int u = 0; u < kLocalUnroll; ++u)
-            if (m[u] >= 0) member_xy(d, list_xy, ob, base, m[u], mx[u], my[u]);
+            if (m[u] >= 0) member_coords(d, list_xy, ob, base, m[u], mx[u], my[u]);
 #pragma unroll
         for (int u = 0; u < kLocalUnroll; ++u) {
             if (m[u] < 0) continue;
@@ -1464,14 +1487,32 @@ __device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d,
     }
     local_sync<kThreads>();
     // Sorted order of the vertex indices (ties, i.e. one point reported
-    // twice, in vertex order).
-    for (int i = tid; i < V; i += kThreads) {
+    // twice, in vertex order).  With threads to spare, several take a vertex
+    // and compare it with a part of the others each.
+    const int parts = max(1, kThreads / max(V, 1));
+    if (parts > 1) {
+        for (int i = tid; i < V; i += kThreads) s.table[i] = 0;
+        local_sync<kThreads>();
+    }
+    for (int t = tid; t < V * parts; t += kThreads) {
+        const int i = t % V, part = t / V;
         const int32_t ci = s.canon[i];
+        const int j1 = V * (part + 1) / parts;
         int pos = 0;
-        for (int j = 0; j < V; ++j) {
+#pragma unroll 8
+        for (int j = V * part / parts; j < j1; ++j) {
             const int32_t cj = s.canon[j];
             pos += (cj < ci || (cj == ci && j < i)) ? 1 : 0;
         }
+        if (parts > 1)
+            atomicAdd(&s.table[i], pos);
+        else
+            s.table[i] = pos;
+    }
+    local_sync<kThreads>();
+    for (int i = tid; i < V; i += kThreads) {
+        const int pos = s.table[i];
+        const int32_t ci = s.canon[i];
         s.sorted[pos] = ci;
         s.spos[i] = static_cast<int16_t>(pos);
         d.hull_idx[ob + base + i] = ci;
@@ -1482,6 +1523,27 @@ __device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d,
     // bin: each run of equal bins adds its length once.
     int steps = 0;
     while ((1 << steps) <= V) ++steps;
+    // Many members: a table over the index range says where each of its
+    // buckets starts among the sorted indices, and a member walks from there.
+    const bool bucketed = size > kThreads * kLocalUnroll / 2 && V > 8;
+    const int32_t idx0 = V > 0 ? s.sorted[0] : 0, idx1 = V > 0 ? s.sorted[V - 1] : 0;
+    int shift = 0;
+    while (((idx1 - idx0) >> shift) >= kLocalHash) ++shift;
+    if (bucketed) {
+        for (int t = tid; t < kLocalHash; t += kThreads) {
+            int lo = 0, hi = V;
+            for (int st = 0; st < steps; ++st) {
+                if (lo >= hi) break;
+                const int mid = (lo + hi) >> 1;
+                if (s.sorted[mid] - idx0 <= static_cast<int64_t>(t) << shift)
+                    lo = mid + 1;
+                else
+                    hi = mid;
+            }
+            s.table[t] = lo;
+        }
+        local_sync<kThreads>();
+    }
     // Wave-uniform trip count: the run detection below reads all lanes.
     for (int q0 = w * kWave + lane; q0 - lane < size; q0 += kThreads * kLocalUnroll) {
         int32_t m[kLocalUnroll];
@@ -1493,7 +1555,16 @@ __device__ __forceinline__ void local_ranks(LocalLds<kVMax>& s, const DevBuf& d,
             lo[u] = 0;
             hi[u] = V;
         }
-        for (int st = 0; st < steps; ++st) {
+        if (bucketed) {
+#pragma unroll
+            for (int u = 0; u < kLocalUnroll; ++u) {
+                if (m[u] >= idx0) lo[u] = m[u] >= idx1 ? V : s.table[(m[u] - idx0) >> shift];
+            }
+#pragma unroll
+            for (int u = 0; u < kLocalUnroll; ++u)
+                while (lo[u] < V && s.sorted[lo[u]] <= m[u]) ++lo[u];
+        }
+        for (int st = bucketed ? steps : 0; st < steps; ++st) {
 #pragma unroll
             for (int u = 0; u < kLocalUnroll; ++u) {
                 if (lo[u] < hi[u]) {
@@ -1574,12 +1645,12 @@ __device__ __forceinline__ void local_ranks_many(const DevBuf& d, const double2*
     }
 }
 
-template <int kThreads>
+template <int kThreads, typename T>
 __global__ __launch_bounds__(kThreads) void k_hull_local(DevBuf d, Layout L, const double2* list_xy) {
     constexpr int kWaves = kThreads / kWave;
     __shared__ union {
-        LocalLds<kLocalMax> large;
-        LocalLds<kLocalSmallV> small[kWaves];
+        LocalLds<kLocalMax, T> large;
+        LocalLds<kLocalSmallV, T> small[kWaves];
     } lds;
     __shared__ LocalCluster run[kWaves];
     __shared__ uint32_t sums[kWaves + 1];
@@ -1617,14 +1688,14 @@ __global__ __launch_bounds__(kThreads) void k_hull_local(DevBuf d, Layout L, con
         }
         __syncthreads();
         auto small = [&](int q) { return run[q].V <= kLocalSmallV && run[q].size <= small_size; };
-        if (w < cnt && small(w)) local_ranks<kWave, kLocalSmallV>(lds.small[w], d, list_xy, ob, BN, run[w]);
+        if (w < cnt && small(w)) local_ranks<kWave, kLocalSmallV, T>(lds.small[w], d, list_xy, ob, BN, run[w]);
         __syncthreads();
         for (int q = 0; q < cnt; ++q) {
             if (small(q)) continue;
             if (run[q].V > kLocalMax)
                 local_ranks_many<kThreads>(d, list_xy, ob, BN, run[q]);
             else
-                local_ranks<kThreads, kLocalMax>(lds.large, d, list_xy, ob, BN, run[q]);
+                local_ranks<kThreads, kLocalMax, T>(lds.large, d, list_xy, ob, BN, run[q]);
             __syncthreads();
         }
     }
@@ -1711,10 +1782,15 @@ void launch_hull(lp_context* c, int B, const double2* list_xy) {
     // A wavefront for about each cluster, and at most 256 workgroups a frame,
     // so that a run holds few clusters while the chip has room.
     stage_mark(c, "hull_local");
-    if (wide)
-        hipLaunchKernelGGL(k_hull_local<1024>, dim3(local_grid(1024), B), dim3(1024), 0, st, d, L, list_xy);
+    auto launch_local = [&](auto kernel, int threads) {
+        hipLaunchKernelGGL(kernel, dim3(local_grid(threads), B), dim3(threads), 0, st, d, L, list_xy);
+    };
+    if (list_xy)
+        launch_local(k_hull_local<1024, double>, 1024);
+    else if (wide)
+        launch_local(k_hull_local<1024, float>, 1024);
     else
-        hipLaunchKernelGGL(k_hull_local<512>, dim3(local_grid(512), B), dim3(512), 0, st, d, L, list_xy);
+        launch_local(k_hull_local<512, float>, 512);
 }
 
 }  // namespace lp
