@@ -609,13 +609,14 @@ int stage_frames(lp_context* c, const lp_cloud* clouds, const CluConst& cc, cons
 
 int run_pipeline(lp_context* c, int B, bool segment_only) {
     c->L.B_active = B;
+    const bool radius_rule = c->staged_filtered && !segment_only && !c->noise_kdtree;
     if (c->staged_filtered && !segment_only) {
         if (c->noise_kdtree)
             launch_noise_kdtree(c, B, true);
         else
             launch_noise(c, B, true);
     }
-    launch_segment_front(c, B);
+    launch_segment_front(c, B, radius_rule);
     launch_jcp(c, B);
     if (!segment_only) {
         launch_cluster(c, B, true);
@@ -1339,7 +1340,7 @@ int lp_cluster(lp_context* c, const lp_clusterer_config* cfg, const lp_cloud* cl
     if (st != LP_OK) return st;
     c->num_frames = 1;
     c->L.B_active = 1;
-    launch_clear(c, 1);
+    launch_clear(c, 1, false);
     launch_cluster(c, 1, false);
     LP_HIP(hipGetLastError());
     Outputs out(c);

@@ -35,13 +35,14 @@ void launch_mt19937(uint32_t* out, int count, hipStream_t st);
 void launch_hash_reset(lp_context* c, int B, const int32_t* slots, int count_slot);
 // Clears every hash slot of the context (at creation).
 void launch_hash_init(lp_context* c);
-void launch_segment_front(lp_context* c, int B);
+void launch_segment_front(lp_context* c, int B, bool cleared);
 void launch_jcp(lp_context* c, int B);
 void launch_cluster(lp_context* c, int B, bool from_split);
 // Ring indices of the scan-ordered cloud staged as frame 0 (x, y).
 void launch_ring_info(lp_context* c, int n);
-// Fill kernel of the per-batch device state (first stage of every run).
-void launch_clear(lp_context* c, int B);
+// Fill kernel of the per-batch device state (first stage of every run); with
+// `noise` also of the radius rule's, which runs ahead of the segmenter.
+void launch_clear(lp_context* c, int B, bool noise);
 // Per-cluster hulls; `list_xy` (standalone lists only) holds the lists'
 // coordinates as (x, y) pairs for the canonical choice among identical points.
 void launch_hull(lp_context* c, int B, const double2* list_xy = nullptr);

@@ -84,25 +84,6 @@ __device__ __forceinline__ float noise_dist(const float4& t, const float4& p) {
     return d0 * d0 + (d1 * d1 + (d2 * d2 + 0.0f));
 }
 
-// The hash slots are clean between uses: every user
-// resets the slots it occupied when it is done (k_hash_reset), so only the
-// column bits and the counters are cleared here.
-__global__ void k_noise_clear(DevBuf d, Layout L) {
-    const int f = blockIdx.y;
-    const int stride = gridDim.x * blockDim.x;
-    const int t0 = blockIdx.x * blockDim.x + threadIdx.x;
-    for (int q = t0; q < kNoiseOccWords; q += stride) d.nocc[(size_t)f * kNoiseOccWords + q] = 0;
-    if (t0 == 0) {
-        d.fs[f * kFsCount + kFsKept] = 0;
-        d.fs[f * kFsCount + kFsNoise] = 0;
-        d.fs[f * kFsCount + kFsNoiseOpen] = 0;
-        d.fs[f * kFsCount + kFsNoiseHard] = 0;
-        d.fs[f * kFsCount + kFsNoiseCells] = 0;
-        d.fs[f * kFsCount + kFsNoisePlaced] = 0;
-        d.fs[f * kFsCount + kFsNoiseErr] = 0;
-    }
-}
-
 constexpr int kNearWindow = 8;  // input-order neighbours tested on each side
 
 constexpr int kPrepRows = 2;  // points per thread: consecutive runs of 256, their atomics in flight together
@@ -595,8 +576,8 @@ void launch_noise(lp_context* c, int B, bool compact) {
     const Layout& L = c->L;
     hipStream_t st = c->stream;
     const int nb = (L.N + 255) / 256;
+    launch_clear(c, B, true);  // for the segmenter too, which does not clear again
     stage_mark(c, "noise");
-    hipLaunchKernelGGL(k_noise_clear, dim3(256, B), dim3(256), 0, st, d, L);
     hipLaunchKernelGGL(k_noise_prep, dim3((L.N + kPrepTile - 1) / kPrepTile, B), dim3(256), 0, st, d, L);
     // About the cells of a 64x2048 frame per 32 workgroups.
     hipLaunchKernelGGL(k_noise_cells, dim3(std::min(nb, 64), B), dim3(256), 0, st, d, L);

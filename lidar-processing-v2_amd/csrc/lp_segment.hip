@@ -25,8 +25,11 @@ constexpr uint32_t kEmptyZ = 0x7fc00000u;           // NaN marks an empty cell
 // ---------------------------------------------------------------------------
 // Per-batch clear (fill kernels instead of memsets so the whole sequence can
 // be captured in a graph).  The voxel hash is clean on entry (its previous
-// users reset the slots they occupied).
-__global__ void k_clear(DevBuf d, Layout L) {
+// users reset the slots they occupied).  Ahead of the noise filter it clears
+// the filter's column bits and counters as well (a launch of their own took 4
+// to 9 us of a 64x2048 frame); after it (the KD-tree search) the filter's
+// counts stay.
+__global__ void k_clear(DevBuf d, Layout L, bool noise) {
     const int f = blockIdx.y;
     const FrameDesc fd = d.frames[f];
     const int cells = fd.sc.cells;
@@ -37,7 +40,9 @@ __global__ void k_clear(DevBuf d, Layout L) {
     for (int c = t0; c < cells; c += stride) d.cell_count[(size_t)f * L.cell_stride + c] = 0;
     for (int p = t0; p < P; p += stride) d.pix_key[fd.pix_off + p] = ~0ull;
     for (int k = t0; k < kRansacIters; k += stride) d.hyp_count[f * kRansacIters + k] = 0;
-    if (t0 < kFsKept) d.fs[f * kFsCount + t0] = 0;  // the noise filter's counts run ahead of this clear
+    if (noise)
+        for (int q = t0; q < kNoiseOccWords; q += stride) d.nocc[(size_t)f * kNoiseOccWords + q] = 0;
+    if (t0 < (noise ? static_cast<int>(kFsCount) : static_cast<int>(kFsKept))) d.fs[f * kFsCount + t0] = 0;
 }
 
 // ---------------------------------------------------------------------------
@@ -838,12 +843,12 @@ __global__ __launch_bounds__(256) void k_pixel_label(DevBuf d, Layout L) {
 }
 
 // ---------------------------------------------------------------------------
-void launch_segment_front(lp_context* c, int B) {
+void launch_segment_front(lp_context* c, int B, bool cleared) {
     DevBuf& d = c->d;
     const Layout& L = c->L;
     hipStream_t st = c->stream;
     const int nb = (L.N + 255) / 256;
-    launch_clear(c, B);
+    if (!cleared) launch_clear(c, B, false);
     stage_mark(c, "project");
     const int wg = c->point_wg;
     if (c->persistent)
@@ -876,9 +881,9 @@ void launch_segment_front(lp_context* c, int B) {
     hipLaunchKernelGGL(k_pixel_label, dim3((L.P + 255) / 256, B), dim3(256), 0, st, d, L);
 }
 
-void launch_clear(lp_context* c, int B) {
+void launch_clear(lp_context* c, int B, bool noise) {
     stage_mark(c, "clear");
-    hipLaunchKernelGGL(k_clear, dim3(256, B), dim3(256), 0, c->stream, c->d, c->L);
+    hipLaunchKernelGGL(k_clear, dim3(256, B), dim3(256), 0, c->stream, c->d, c->L, noise);
 }
 
 // k_hash_reset clears the slots a stage occupied; k_hash_init clears every slot
