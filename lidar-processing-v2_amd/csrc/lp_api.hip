@@ -875,8 +875,7 @@ int create_lane(const lp_capacity* cap, lp_context** out) {
     layout_bytes(L, &c->d, static_cast<char*>(c->arena));
     launch_mt19937(c->d.mt_raw, kMtRawCount, c->stream);
     launch_hash_init(c);
-    e = hipMemsetAsync(c->d.fs, 0, L.B * kFsCount * sizeof(uint32_t), c->stream);
-    if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+    e = hipStreamSynchronize(c->stream);
     if (e != hipSuccess) {
         lp_context_destroy(c);
         return fail(LP_ERR_HIP, std::string("context init: ") + hipGetErrorString(e));

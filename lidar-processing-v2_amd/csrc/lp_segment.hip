@@ -887,12 +887,13 @@ void launch_clear(lp_context* c, int B, bool noise) {
 }
 
 // k_hash_reset clears the slots a stage occupied; k_hash_init clears every slot
-// (context creation).
+// and the frames' scalars (context creation).
 __global__ void k_hash_reset(DevBuf d, Layout L, const int32_t* slots, int count_slot) {
     reset_slots(d, L, blockIdx.y, slots, count_slot, blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x);
 }
 
 __global__ void k_hash_init(DevBuf d, Layout L) {
+    for (int q = blockIdx.x * blockDim.x + threadIdx.x; q < L.B * kFsCount; q += gridDim.x * blockDim.x) d.fs[q] = 0;
     const size_t total = (size_t)L.B * L.hash_cap;
     for (size_t o = blockIdx.x * (size_t)blockDim.x + threadIdx.x; o < total; o += (size_t)gridDim.x * blockDim.x) {
         d.hslot[o] = HashSlot{-1, 0u, 0, kHashMinClean};
