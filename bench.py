@@ -74,10 +74,10 @@ def bytes_extended(n_raw, n, p, n_obs, voxels, hull_vertices, clusters):
 def kernel_bytes_8d(kernel, n, p, n_obs, voxels, hull_vertices):
     """The share of bytes_8d each kernel moves (per frame): the projection
     reads the points, the pixel labels write the range image and the row
-    solve reads it, the labels kernel writes the labels, the spherical
-    conversion reads the obstacle points and the component labels write
-    their cluster labels, the voxel insert writes the hash, and the hull
-    rounds read the hull inputs and produce the vertices."""
+    solve reads it, the labels kernel writes the labels, the obstacle split
+    reads the obstacle points and the cluster labels are written for them,
+    the voxel insert writes the hash, and the first hull round reads the hull
+    inputs and produces the vertices of most clusters."""
     return {"k_project": 14 * n, "k_pixel_label": 5 * p, "k_jcp_solve": 5 * p, "k_seg_labels": 4 * n,
             "k_obs_gather": 12 * n_obs, "k_cluster_label": 4 * n_obs, "k_voxel_insert": 8 * voxels,
             "k_hull_round": 8 * n_obs + 16 * hull_vertices}.get(kernel, 0)
