@@ -227,7 +227,11 @@ __device__ __forceinline__ void cand_min(CandMin& m, double area, int pos, int c
 // running minimum of polygonizer.cpp:257).  After the first candidate of the
 // overall smallest area m only areas below float(m) replace, so the last of
 // those is the answer; without one it is that first candidate, if m is below
-// the float of the smallest area before it.
+// the float of the smallest area before it.  If it is not (the sides of a
+// straight wall give areas that agree in float), the last candidate below the
+// float of the smallest area before it is found from prefix minima over the
+// walk, NT elements at a time; that case took the walk by one lane before
+// (eight 128x2048 frames with facades 112 -> 27 us, 32 of 64x2048 68 -> 43).
 constexpr int kWalkSerial = -2;
 
 template <int NT>
@@ -287,24 +291,25 @@ __device__ int choose_candidate(const double2* V, const double* area, int n, int
     for (int q = 0; q <= j0 >> 5; ++q) pairs += __popc(par[q]);
     if (pairs > cap) return kWalkSerial;
     // Candidates of the walk's pairs: visit(position, vertex, offset bit).
-    auto candidates = [&](auto visit) {
-        for (int t = j0 + tid; t < elements; t += NT) {
-            const int i = row_of(t), j = t - i + 1;
-            if (early && i == j0 && j == n - 1) continue;
-            int before = t - j0;
-            for (int q = 0; q < i >> 5; ++q) before += __popc(par[q]);
-            before += __popc(par[i >> 5] & ((1u << (i & 31)) - 1u));
-            const bool twin = j == J[i] && ((par[i >> 5] >> (i & 31)) & 1u);
-            const bool wrapped = i == j0 && j == n - 1;
-            for (int p = 0; p <= (twin ? 1 : 0); ++p) {
-                const int a = p && wrapped ? wrap(i + 1, n) : i;
-                const int b = wrap(p && !wrapped ? j + 1 : j, n);
-                visit(4 * (before + p) + 0, a, 0);
-                visit(4 * (before + p) + 1, a, 1);
-                visit(4 * (before + p) + 2, b, 0);
-                visit(4 * (before + p) + 3, b, 1);
-            }
+    auto candidates_at = [&](int t, auto visit) {
+        const int i = row_of(t), j = t - i + 1;
+        if (early && i == j0 && j == n - 1) return;
+        int before = t - j0;
+        for (int q = 0; q < i >> 5; ++q) before += __popc(par[q]);
+        before += __popc(par[i >> 5] & ((1u << (i & 31)) - 1u));
+        const bool twin = j == J[i] && ((par[i >> 5] >> (i & 31)) & 1u);
+        const bool wrapped = i == j0 && j == n - 1;
+        for (int p = 0; p <= (twin ? 1 : 0); ++p) {
+            const int a = p && wrapped ? wrap(i + 1, n) : i;
+            const int b = wrap(p && !wrapped ? j + 1 : j, n);
+            visit(4 * (before + p) + 0, a, 0);
+            visit(4 * (before + p) + 1, a, 1);
+            visit(4 * (before + p) + 2, b, 0);
+            visit(4 * (before + p) + 3, b, 1);
         }
+    };
+    auto candidates = [&](auto visit) {
+        for (int t = j0 + tid; t < elements; t += NT) candidates_at(t, visit);
     };
     auto area_of = [&](int v, int up) { return area[up ? v : (v == 0 ? n - 1 : v - 1)]; };
     // Candidate of the smallest area, the first of equal ones.
@@ -353,7 +358,58 @@ __device__ int choose_candidate(const double2* V, const double* area, int n, int
         __syncthreads();
     }
     if (later.pos >= 0) return later.cand;
-    return m.area < static_cast<double>(static_cast<float>(later.area)) ? m.cand : kWalkSerial;
+    if (m.area < static_cast<double>(static_cast<float>(later.area))) return m.cand;
+    double carry = __builtin_inf();  // smallest area of the elements before these NT
+    CandMin last{0.0, -1, -1};
+    for (int t0 = j0; t0 < elements; t0 += NT) {
+        const int t = t0 + tid;
+        double mine = __builtin_inf();
+        if (t < elements) candidates_at(t, [&](int, int v, int up) { mine = fmin(mine, area_of(v, up)); });
+        double incl = mine;
+#pragma unroll
+        for (int o = 1; o < kWave; o <<= 1) {
+            const double x = __shfl_up(incl, o, kWave);
+            if (lane_id() >= o) incl = fmin(incl, x);
+        }
+        double run = __shfl_up(incl, 1, kWave);
+        run = fmin(lane_id() > 0 ? run : __builtin_inf(), carry);
+        double total = __shfl(incl, kWave - 1, kWave);
+        if (NT > kWave) {
+            if (lane_id() == 0) red[tid / kWave].area = total;
+            __syncthreads();
+            for (int q = 0; q < NT / kWave; ++q) {
+                if (q < tid / kWave) run = fmin(run, red[q].area);
+                total = fmin(total, red[q].area);
+            }
+            __syncthreads();
+        }
+        carry = fmin(carry, total);
+        if (t < elements)
+            candidates_at(t, [&](int pos, int v, int up) {
+                const double a = area_of(v, up);
+                if (a < static_cast<double>(static_cast<float>(run))) {
+                    last.pos = pos;
+                    last.cand = 2 * v + up;
+                }
+                run = fmin(run, a);
+            });
+    }
+#pragma unroll
+    for (int o = kWave / 2; o > 0; o >>= 1) {
+        const int p = __shfl_xor(last.pos, o, kWave), c = __shfl_xor(last.cand, o, kWave);
+        if (p > last.pos) {
+            last.pos = p;
+            last.cand = c;
+        }
+    }
+    if (NT > kWave) {
+        if (lane_id() == 0) red[tid / kWave] = last;
+        __syncthreads();
+        for (int q = 0; q < NT / kWave; ++q)
+            if (red[q].pos > last.pos) last = red[q];
+        __syncthreads();
+    }
+    return last.cand;
 }
 
 // The same by one lane: the reference's walk and its sequential rule.  False
