@@ -361,7 +361,10 @@ __device__ int prune_chain(const double* X, const double* Y, uint16_t* L, uint16
 
 constexpr int kPrunePasses = 6;
 constexpr int kMergeChain = 32;  // half lists longer than this take the wavefront chain
-constexpr int kBigPrunePasses = 32;
+// What is left after the rounds is nearly convex: pruning drops few points a
+// pass, and one wavefront goes through the whole list for it (with up to 32
+// passes the launch took 80 to 110 us for eight 128x2048 frames, 54 with 4).
+constexpr int kBigPrunePasses = 4;
 constexpr int kWavesPerBlock = 4;
 constexpr int kHullRounds = 3;
 constexpr int kHullBig = 4096;  // candidates one workgroup finishes after the rounds
