@@ -1701,6 +1701,9 @@ __global__ __launch_bounds__(kThreads) void k_hull_local(DevBuf d, Layout L, con
                 local_ranks<kThreads, kLocalMax, T>(lds.large, d, list_xy, ob, BN, run[q]);
             __syncthreads();
         }
+        // Every wavefront has looked at the whole run (small clusters are
+        // passed over without a barrier) before the next one replaces it.
+        __syncthreads();
     }
 }
 
