@@ -429,7 +429,7 @@ size_t layout_bytes(const Layout& L, DevBuf* d, char* base) {
     go(x.hcy, 2 * B * N);
     go(x.hci, 2 * B * N);
     go(x.hc_count, 2 * B * N);
-    go(x.hc_open, B * N);
+    go(x.hc_open, B * N + 1);  // standalone lists: their offsets, one more than there are lists
     go(x.hull_idx, B * N);
     go(x.hull_count, B * N);
     go(x.hull_off, B * N);

@@ -179,7 +179,7 @@ struct DevBuf {
     double* hcy;
     int32_t* hci;            // candidate obstacle index
     uint32_t* hc_count;      // per cluster candidates (two buffers)
-    uint32_t* hc_open;       // clusters of more than one chunk
+    uint32_t* hc_open;       // clusters of more than one chunk; before the run: the offsets of standalone lists
     // Per chunk of the first hull round (written by its plan): its cluster,
     // with bit 31 set when the chunk is the cluster's only one (= cell_items,
     // free in the hull stage); its index in the cluster and, from bit 16, its

@@ -44,6 +44,17 @@ def test_list_runs(oracle, order):
         assert np.array_equal(h, oracle.convex_hull(x, y))
 
 
+@pytest.mark.parametrize("count", [64, 4096])
+def test_as_many_lists_as_points(count):
+    """One-point lists that fill the context: there is one offset more than
+    points."""
+    rng = np.random.default_rng(count)
+    with N.Context(max_points=count) as ctx:
+        for lists in (count, count - 1, count):
+            st, hulls = ctx.convex_hulls([rng.normal(0, 9, (2, 1)) for _ in range(lists)])
+            assert st == 0 and all(np.array_equal(h, [0]) for h in hulls)
+
+
 def _frame(seed, posts):
     """Lone points all around, each a cluster of its own or of a few, and eight
     arcs of 72 columns, every point of which is a hull vertex.  An arc's first
