@@ -13,9 +13,12 @@
 // Here: voxel keys go into an open-addressing HBM hash set by atomicCAS
 // (one dense id per occupied voxel, per-voxel point count and minimum point
 // index by atomics on the voxel's own slot), components come from a
-// lock-free union-find over dense ids (in global memory by the whole grid for
-// few frames, in LDS by one workgroup per frame for many), and a component's
-// label is the rank of its first point among the surviving components'.
+// lock-free union-find over dense ids (in LDS by one workgroup per frame, in
+// global memory by the whole grid when a frame's voxels do not fit there), and
+// a component's label is the rank of its first point among the surviving
+// components'.
+#include <algorithm>
+
 #include "lp_kernels.h"
 #include "lp_joins.h"
 #include "lp_queue.h"
@@ -551,76 +554,205 @@ __device__ __forceinline__ int32_t root_of_point(const DevBuf& d, size_t ob, siz
 
 // Clusters in the order of their first point (the reference numbers them in
 // input order): a component is a cluster when it has at least min_size points,
-// and its first point is its minimum obstacle index.  One workgroup per frame
-// marks the first points of the frame's few hundred components in an LDS
-// bitmap (kRankPoints points at a time), ranks them by the bits before them,
-// and writes each cluster's size, member offset and empty cursors and each
-// root's label.  Before, two passes over all points, each following three
-// dependent gathers, numbered the clusters (with the offsets' scan 22 -> 5
-// us for one 64x2048 frame).
+// and its first point is its minimum obstacle index.  Two forms, by the number
+// of obstacles a frame can have (launch_cluster):
+//
+// Up to kRankPoints: one workgroup per frame marks the first points of the
+// frame's components in an LDS bitmap, ranks them by the bits before them, and
+// writes each cluster's size, member offset and empty cursors and each root's
+// label (standalone, the labels only).  A frame has a few hundred components,
+// for which the two passes below and the offsets' scan took 22 us of a 64x2048
+// frame and this takes 5.  Where nearly every point is a component, it waits
+// for the roots' gathers, eight a thread in flight: a standalone call with
+// 200 000 isolated points takes 264 us, 387 with one gather at a time.
 constexpr int kRankThreads = 1024;
 constexpr int kRankItems = 8;
 constexpr int kRankWords = kRankThreads * kRankItems;
 constexpr int kRankPoints = kRankWords * 32;
+constexpr int kRankRoots = 8;  // roots per thread and turn
 
+// visit(root, first point, size) for every component, R roots per thread and
+// turn.  (Most frames have one turn of one root: the unrolled code, cold in
+// every launch, would cost them 0.7 us.)
+template <int R, typename Visit>
+__device__ __forceinline__ void for_components(const DevBuf& d, size_t ob, int roots, Visit visit) {
+    for (int i0 = threadIdx.x; i0 < roots; i0 += kRankThreads * R) {
+        int32_t r[R], first[R];
+        uint32_t size[R];
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            const int i = i0 + u * kRankThreads;
+            r[u] = i < roots ? d.vroots[ob + i] : -1;
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u) {
+            if (r[u] < 0) continue;
+            first[u] = d.vmin[ob + r[u]];
+            size[u] = d.vcnt[ob + r[u]];
+        }
+#pragma unroll
+        for (int u = 0; u < R; ++u)
+            if (r[u] >= 0) visit(r[u], first[u], size[u]);
+    }
+}
+
+// Member offsets: the exclusive sums of the K sizes, R per thread and turn.
+template <int R>
+__device__ __forceinline__ void member_offsets(const DevBuf& d, size_t ob, int K, uint32_t* lds) {
+    uint32_t off = 0;
+    for (int base = 0; base < K; base += kRankThreads * R) {
+        const int b = base + static_cast<int>(threadIdx.x) * R;
+        uint32_t v[R];
+        uint32_t mine = 0;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            v[k] = b + k < K ? d.cl_size[ob + b + k] : 0u;
+            mine += v[k];
+        }
+        uint32_t total;
+        uint32_t at = block_exclusive_sum<kRankThreads>(mine, lds, &total) + off;
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            if (b + k < K) d.cl_off[ob + b + k] = at;
+            at += v[k];
+        }
+        off += total;
+    }
+}
+
+template <bool kOffsets>
 __global__ __launch_bounds__(kRankThreads) void k_component_rank(DevBuf d, Layout L) {
     __shared__ uint32_t bits[kRankWords];
     __shared__ uint32_t before[kRankWords];
     __shared__ uint32_t lds[kRankThreads / kWave + 1];
     const int f = blockIdx.x;
     const int tid = threadIdx.x;
-    const int nobs = static_cast<int>(d.fs[f * kFsCount + kFsObstacles]);
     const int roots = static_cast<int>(d.fs[f * kFsCount + kFsRoots]);
     const uint32_t min_size = d.cc->min_size;
     const size_t ob = (size_t)f * L.N;
-    uint32_t carry = 0;
-    for (int base = 0; base < nobs; base += kRankPoints) {
-        for (int q = tid; q < kRankWords; q += kRankThreads) bits[q] = 0;
-        __syncthreads();
-        for (int i = tid; i < roots; i += kRankThreads) {
-            const int32_t r = d.vroots[ob + i];
-            const int at = d.vmin[ob + r] - base;
-            if (d.vcnt[ob + r] >= min_size && at >= 0 && at < kRankPoints) atomicOr(&bits[at >> 5], 1u << (at & 31));
-        }
-        __syncthreads();
-        uint32_t sum = 0;
+    // visit(root, first point, size) for every component.
+    auto components = [&](auto visit) {
+        if (roots <= 2 * kRankThreads)
+            for_components<1>(d, ob, roots, visit);
+        else
+            for_components<kRankRoots>(d, ob, roots, visit);
+    };
+    for (int q = tid; q < kRankWords; q += kRankThreads) bits[q] = 0;
+    __syncthreads();
+    components([&](int32_t, int32_t at, uint32_t size) {
+        if (size >= min_size) atomicOr(&bits[at >> 5], 1u << (at & 31));
+    });
+    __syncthreads();
+    uint32_t sum = 0;
 #pragma unroll
-        for (int k = 0; k < kRankItems; ++k) sum += static_cast<uint32_t>(__popc(bits[tid * kRankItems + k]));
-        uint32_t total;
-        uint32_t ex = block_exclusive_sum<kRankThreads>(sum, lds, &total) + carry;
+    for (int k = 0; k < kRankItems; ++k) sum += static_cast<uint32_t>(__popc(bits[tid * kRankItems + k]));
+    uint32_t clusters;
+    uint32_t ex = block_exclusive_sum<kRankThreads>(sum, lds, &clusters);
 #pragma unroll
-        for (int k = 0; k < kRankItems; ++k) {
-            before[tid * kRankItems + k] = ex;
-            ex += static_cast<uint32_t>(__popc(bits[tid * kRankItems + k]));
+    for (int k = 0; k < kRankItems; ++k) {
+        before[tid * kRankItems + k] = ex;
+        ex += static_cast<uint32_t>(__popc(bits[tid * kRankItems + k]));
+    }
+    __syncthreads();
+    components([&](int32_t r, int32_t at, uint32_t size) {
+        if (size < min_size) {
+            d.vlab[ob + r] = -1;
+            return;
         }
-        __syncthreads();
-        for (int i = tid; i < roots; i += kRankThreads) {
-            const int32_t r = d.vroots[ob + i];
-            const uint32_t size = d.vcnt[ob + r];
-            const int at = d.vmin[ob + r] - base;
-            if (size < min_size) d.vlab[ob + r] = -1;
-            if (size < min_size || at < 0 || at >= kRankPoints) continue;
-            const uint32_t lab = before[at >> 5] + static_cast<uint32_t>(__popc(bits[at >> 5] & ((1u << (at & 31)) - 1u)));
+        const uint32_t lab = before[at >> 5] + static_cast<uint32_t>(__popc(bits[at >> 5] & ((1u << (at & 31)) - 1u)));
+        if (kOffsets) {
             d.cl_size[ob + lab] = size;
             d.cl_cursor[ob + lab] = 0;
             d.hc_count[ob + lab] = 0;  // the round-0 hull input count (first buffer)
-            d.vlab[ob + r] = static_cast<int32_t>(lab);
         }
-        carry += total;
-        __syncthreads();
+        d.vlab[ob + r] = static_cast<int32_t>(lab);
+    });
+    if (tid == 0) d.fs[f * kFsCount + kFsClusters] = clusters;
+    if (!kOffsets) return;
+    __syncthreads();
+    const int K = static_cast<int>(clusters);
+    if (K <= kRankThreads)
+        member_offsets<1>(d, ob, K, lds);
+    else
+        member_offsets<kRankItems>(d, ob, K, lds);
+}
+
+// Beyond kRankPoints: two passes of the whole grid over tiles of 2048
+// obstacles (eight rows of 256), the first points of every tile and then their
+// numbers after the tiles before; the offsets are scanned afterwards.  (The
+// form above in turns of kRankPoints, each over all components, took 6.1 ms of
+// a standalone call with a million isolated points and 74 ms with four million;
+// with these the calls take 0.84 and 3.3 ms.)
+constexpr int kCompThreads = 256;
+constexpr int kCompRows = 8;
+constexpr int kCompTile = kCompThreads * kCompRows;
+
+// The thread's points that are a component's first, of them the clusters'.
+__device__ __forceinline__ uint32_t first_points(const DevBuf& d, size_t ob, size_t ho, int base, int nobs,
+                                                 uint32_t min_size, int32_t (&root)[kCompRows],
+                                                 uint32_t (&size)[kCompRows], uint32_t& clusters) {
+    uint32_t m = 0;
+    clusters = 0;
+#pragma unroll
+    for (int k = 0; k < kCompRows; ++k) {
+        const int q = base + k * kCompThreads + static_cast<int>(threadIdx.x);
+        if (q >= nobs) continue;
+        root[k] = root_of_point(d, ob, ho, q);
+        size[k] = d.vcnt[ob + root[k]];
+        if (d.vmin[ob + root[k]] != q) continue;
+        m |= 1u << k;
+        if (size[k] >= min_size) clusters |= 1u << k;
     }
-    if (tid == 0) d.fs[f * kFsCount + kFsClusters] = carry;
-    // Member offsets: the exclusive sums of the sizes.
-    const int K = static_cast<int>(carry);
-    uint32_t off = 0;
-    for (int base = 0; base < K; base += kRankThreads) {
-        const int k = base + tid;
-        const uint32_t v = k < K ? d.cl_size[ob + k] : 0u;
-        uint32_t total;
-        const uint32_t ex = block_exclusive_sum<kRankThreads>(v, lds, &total) + off;
-        if (k < K) d.cl_off[ob + k] = ex;
-        off += total;
+    return m;
+}
+
+__global__ __launch_bounds__(kCompThreads) void k_component_count(DevBuf d, Layout L) {
+    __shared__ uint32_t lds[kCompThreads / kWave + 1];
+    const int f = blockIdx.y;
+    const int nobs = static_cast<int>(d.fs[f * kFsCount + kFsObstacles]);
+    const int base = blockIdx.x * kCompTile;
+    if (base >= nobs) return;
+    int32_t root[kCompRows];
+    uint32_t size[kCompRows], clusters;
+    first_points(d, (size_t)f * L.N, (size_t)f * L.hash_cap, base, nobs, d.cc->min_size, root, size, clusters);
+    uint32_t total;
+    block_exclusive_sum<kCompThreads>(static_cast<uint32_t>(__popc(clusters)), lds, &total);
+    if (threadIdx.x == 0) d.blk[(size_t)f * L.blk_stride + blockIdx.x] = total;
+}
+
+__global__ __launch_bounds__(kCompThreads) void k_component_number(DevBuf d, Layout L) {
+    __shared__ uint32_t lds[kCompRows * kCompThreads / kWave + 1];
+    const int f = blockIdx.y;
+    const int nobs = static_cast<int>(d.fs[f * kFsCount + kFsObstacles]);
+    const int tile = blockIdx.x;
+    const int base = tile * kCompTile;
+    if (base >= nobs) {
+        if (tile == 0 && threadIdx.x == 0) d.fs[f * kFsCount + kFsClusters] = 0;
+        return;
     }
+    const uint32_t* blk = d.blk + (size_t)f * L.blk_stride;
+    uint32_t pre = 0;
+    for (int i = threadIdx.x; i < tile; i += kCompThreads) pre += blk[i];
+    uint32_t pre_total;
+    block_exclusive_sum<kCompThreads>(pre, lds, &pre_total);
+    const size_t ob = (size_t)f * L.N;
+    int32_t root[kCompRows];
+    uint32_t size[kCompRows], clusters;
+    const uint32_t first = first_points(d, ob, (size_t)f * L.hash_cap, base, nobs, d.cc->min_size, root, size, clusters);
+    uint32_t pos[kCompRows];
+    const uint32_t total = tile_compact<kCompThreads, kCompRows>(clusters, pos, lds);
+#pragma unroll
+    for (int k = 0; k < kCompRows; ++k) {
+        if (!((first >> k) & 1u)) continue;
+        const uint32_t lab = pre_total + pos[k];
+        const bool cluster = (clusters >> k) & 1u;
+        d.vlab[ob + root[k]] = cluster ? static_cast<int32_t>(lab) : -1;
+        if (!cluster) continue;
+        d.cl_size[ob + lab] = size[k];
+        d.cl_cursor[ob + lab] = 0;
+        d.hc_count[ob + lab] = 0;
+    }
+    if (threadIdx.x == 0 && base + kCompTile >= nobs) d.fs[f * kFsCount + kFsClusters] = pre_total + total;
 }
 
 // True when the obstacle at input index i (pixel pix of a frame W pixels
@@ -739,7 +871,20 @@ void launch_cluster(lp_context* c, int B, bool from_split) {
     hipLaunchKernelGGL(k_voxel_neighbours, dim3(nb, B), dim3(256), 0, st, d, L);
     hipLaunchKernelGGL(k_voxel_cc, dim3(B), dim3(1024), 0, st, d, L);
     hipLaunchKernelGGL(k_voxel_stats, dim3(nb, B), dim3(256), 0, st, d, L);
-    hipLaunchKernelGGL(k_component_rank, dim3(B), dim3(kRankThreads), 0, st, d, L);
+    // Obstacles a frame can have: of the split, each has a pixel of its own (by
+    // the capacity, so that a graph holds for every batch); standalone, the
+    // cloud's points.
+    const int most = from_split ? std::min(L.N, L.P) : c->frames.front().n;
+    if (most > kRankPoints) {
+        const int ct = (L.N + kCompTile - 1) / kCompTile;
+        hipLaunchKernelGGL(k_component_count, dim3(ct, B), dim3(kCompThreads), 0, st, d, L);
+        hipLaunchKernelGGL(k_component_number, dim3(ct, B), dim3(kCompThreads), 0, st, d, L);
+        if (from_split) launch_scan(c, B, d.cl_size, d.cl_off, L.N, kCountSlot, kFsClusters, -1);
+    } else if (from_split) {
+        hipLaunchKernelGGL(k_component_rank<true>, dim3(B), dim3(kRankThreads), 0, st, d, L);
+    } else {
+        hipLaunchKernelGGL(k_component_rank<false>, dim3(B), dim3(kRankThreads), 0, st, d, L);
+    }
     if (from_split) {
         hipLaunchKernelGGL(k_cluster_label<true>, dim3(nb, B), dim3(256), 0, st, d, L);
     } else {
