@@ -368,6 +368,23 @@ constexpr int kBigPrunePasses = 4;
 constexpr int kWavesPerBlock = 4;
 constexpr int kHullRounds = 3;
 constexpr int kHullBig = 4096;  // candidates one workgroup finishes after the rounds
+// Candidates up to which one workgroup takes a cluster through the rounds, and
+// what each of several takes of more.  Of points whose chunks lose so little
+// that kHullBig is in question the rounds of fewer would leave half a percent
+// more in shares; of more, what the rounds bring down to kHullBig at all shares
+// bring lower (by their last round), so no cluster is refused for them.
+constexpr int kHullTogether = 6144;
+constexpr int kHullShare = 2048;
+// hc_open entries: a cluster (below 2^24, as points are) and which of the
+// workgroups that take its shares in turn.
+constexpr int kHullTakerBit = 24;
+constexpr uint32_t kHullTakers = 256;
+constexpr uint32_t kSecondBuffer = 1u << 31;
+
+// Workgroups that take a cluster of n candidates through the rounds.
+__device__ __forceinline__ uint32_t hull_shares(uint32_t n) {
+    return n <= static_cast<uint32_t>(kHullTogether) ? 1u : (n + kHullShare - 1) / kHullShare;
+}
 
 // Andrew's monotone chain over the n points P[0..n) (sorted by (x, y, idx))
 // with sign-exact orientation (polygonizer.cpp:66-90).  Writes the hull to
@@ -672,8 +689,10 @@ __device__ int sort_dedupe_chunk(double* X, double* Y, int32_t* I, uint16_t* P, 
 // it fits: that chunk's hull is final).  hc_chunk_c / hc_chunk_i / hc_chunk_b
 // receive each chunk's cluster, index and size, and the cluster's first
 // candidate, the frame's total goes to kFsHullChunks, and the clusters of more
-// than one chunk are listed in hc_open for the rounds after the first.  It also
-// clears the hull counts and flags and the second buffer's candidate counts.
+// than one chunk are listed in hc_open for the rounds after the first, once for
+// every workgroup that may take a share of them there (fewer than one per 256
+// points).  It also clears the hull counts and flags and the second buffer's
+// candidate counts.
 constexpr int kPlanThreads = 1024;
 constexpr int kPlanItems = 4;
 
@@ -700,7 +719,14 @@ __global__ __launch_bounds__(kPlanThreads) void k_hull_plan(DevBuf d, Layout L) 
                 d.hc_count[BN + ob + c] = 0;
                 cn[q] = d.hc_count[ob + c];
                 v[q] = cn[q] <= static_cast<uint32_t>(kHullChunk) ? 1u : (cn[q] + kHullChunk - 1) / kHullChunk;
+                // (An add of one is one atomic for the wavefront.)
                 if (v[q] > 1) d.hc_open[ob + atomicAdd(&d.fs[f * kFsCount + kFsHullOpen], 1u)] = static_cast<uint32_t>(c);
+                if (cn[q] > static_cast<uint32_t>(kHullTogether)) {
+                    const uint32_t more = min(hull_shares(cn[q]), kHullTakers) - 1;
+                    uint32_t* open = d.hc_open + ob + atomicAdd(&d.fs[f * kFsCount + kFsHullOpen], more);
+#pragma nounroll
+                    for (uint32_t k = 0; k < more; ++k) open[k] = static_cast<uint32_t>(c) | (k + 1) << kHullTakerBit;
+                }
                 local += v[q];
             }
         }
@@ -997,8 +1023,19 @@ __global__ __launch_bounds__(256, 3) void k_hull_round(DevBuf d, Layout L) {
 // table of one 64x2048 frame 39 -> 21 us; eight 128x2048 frames at a time 129
 // -> 101 us).  512 threads for few frames: with 256 the clusters of more than four chunks take
 // their chunks in turns (the eight frames 120 us), 1024 leave one workgroup to
-// a CU (one frame 32 us).  Workgroups from `tiles` on clear the voxel table's
-// used slots, which no later kernel reads.
+// a CU (one frame 32 us).
+// A cluster with more candidates than kHullTogether is shared among workgroups:
+// taken by one, 65 000 points of a wall with 2 cm of noise made a 64x2048 frame
+// 658 us, now 440, and the candidates of a whole wall with 1 mm 2.42 ms, now
+// 0.44 (both 0.65 with the launches per round).  A share goes through its rounds
+// alone, one more than a whole cluster since its chunks meet only each other,
+// and what is left of it lies at its place in the buffers; the first words of
+// the cluster's part of hc_chunk_b say how much and in which buffer, for
+// k_hull_big.  What is left of a whole cluster is in the second buffer.
+// Workgroups from `tiles` on clear the voxel table's used slots, which no later
+// kernel reads.
+static_assert(kHullRounds % 2 == 1, "what the rounds leave is in the second buffer");
+
 template <int kThreads>
 __global__ __launch_bounds__(kThreads) void k_hull_merge(DevBuf d, Layout L, int tiles) {
     __shared__ ChunkLds lds[kThreads / kWave];
@@ -1015,30 +1052,47 @@ __global__ __launch_bounds__(kThreads) void k_hull_merge(DevBuf d, Layout L, int
     const size_t ob = (size_t)f * L.N;
     const size_t BN = (size_t)L.B * L.N;
     for (uint32_t j = tile; j < open; j += tiles) {
-        const int c = static_cast<int>(d.hc_open[ob + j]);
+        const uint32_t entry = d.hc_open[ob + j];
+        const int c = static_cast<int>(entry & ((1u << kHullTakerBit) - 1u));
         const uint32_t base = d.cl_off[ob + c];
-        uint32_t cnt = d.hc_count[BN + ob + c];
-        bool final_chunk = false;
-        for (int r = 1; r < kHullRounds && !final_chunk; ++r) {
-            const size_t in = (size_t)(r & 1) * BN + ob + base, out = (size_t)((r + 1) & 1) * BN + ob + base;
-            final_chunk = cnt <= static_cast<uint32_t>(kHullChunk);
-            if (threadIdx.x == 0) next = 0;
-            __syncthreads();
-            for (uint32_t lo = w * kHullChunk; lo < cnt; lo += kThreads / kWave * kHullChunk) {
-                const int n = static_cast<int>(min(cnt - lo, static_cast<uint32_t>(kHullChunk)));
-                const int kk = chunk_hull(lds[w], d, L, f, c, in + lo, n);
-                if (final_chunk)
-                    put_hull(lds[w], d, ob, c, base, kk);
-                else
-                    put_candidates(lds[w], d, out, &next, kk);
-                wave_sync();
+        const uint32_t all = d.hc_count[BN + ob + c];
+        const uint32_t shares = hull_shares(all);
+        const bool whole = shares == 1;
+        const int rounds = whole ? kHullRounds : kHullRounds + 1;
+        for (uint32_t share = entry >> kHullTakerBit; share < shares; share += kHullTakers) {
+            const uint32_t first = share * kHullShare;
+            uint32_t cnt = whole ? all : min(all - first, static_cast<uint32_t>(kHullShare));
+            bool last = false;  // the candidates are one chunk
+            uint32_t buffer = 1;
+            for (int r = 1; r < rounds && !last; ++r) {
+                const size_t in = buffer * BN + ob + base + first, out = (buffer ^ 1) * BN + ob + base + first;
+                last = cnt <= static_cast<uint32_t>(kHullChunk);
+                if (threadIdx.x == 0) next = 0;
+                __syncthreads();
+                for (uint32_t lo = w * kHullChunk; lo < cnt; lo += kThreads / kWave * kHullChunk) {
+                    const int n = static_cast<int>(min(cnt - lo, static_cast<uint32_t>(kHullChunk)));
+                    const int kk = chunk_hull(lds[w], d, L, f, c, in + lo, n);
+                    if (whole && last)
+                        put_hull(lds[w], d, ob, c, base, kk);
+                    else
+                        put_candidates(lds[w], d, out, &next, kk);
+                    wave_sync();
+                }
+                __syncthreads();
+                cnt = next;
+                buffer ^= 1;
+                __syncthreads();
             }
-            __syncthreads();
-            cnt = next;
-            __syncthreads();
+            if (!(whole && last) && threadIdx.x == 0) {
+                // The count of a whole cluster still makes one share of it, should
+                // another taker look.
+                if (whole)
+                    d.hc_count[BN + ob + c] = cnt;
+                else
+                    d.hc_chunk_b[ob + base + share] = cnt | (buffer ? kSecondBuffer : 0u);
+                atomicAdd(&d.fs[f * kFsCount + kFsHullLeft], 1u);
+            }
         }
-        // Left to k_hull_big, which reads the buffer the last round wrote.
-        if (!final_chunk && threadIdx.x == 0) d.hc_count[(size_t)(kHullRounds & 1) * BN + ob + c] = cnt;
     }
 }
 
@@ -1171,9 +1225,44 @@ __device__ void ref_hull(const DevBuf& d, const Layout& L, const double2* list_x
     __syncthreads();
 }
 
+// What the rounds left of a shared cluster, from its part of the candidate
+// buffers (the second one `second` entries after the first) to X, Y, I; returns
+// how many points that is, of which the first kHullBig are there.  By the 1024
+// threads of k_hull_big, with their share of its LDS; out of line, or its
+// registers would spill those of the chains.
+__device__ __attribute__((noinline)) uint32_t gather_shares(const double* cx, const double* cy, const int32_t* ci,
+                                                            size_t second, const uint32_t* words, uint32_t shares,
+                                                            double* X, double* Y, int32_t* I, uint32_t* lds) {
+    uint32_t* word = lds;
+    uint32_t* at = lds + 1024;
+    const uint32_t tid = threadIdx.x;
+    uint32_t cnt = 0;
+    for (uint32_t s0 = 0; s0 < shares && cnt <= static_cast<uint32_t>(kHullBig); s0 += 1024) {
+        const uint32_t mine = s0 + tid < shares ? words[s0 + tid] : 0u;
+        uint32_t total;
+        const uint32_t before = block_exclusive_sum<1024>(mine & ~kSecondBuffer, lds + 2 * 1024, &total);
+        word[tid] = mine;
+        at[tid] = cnt + before;
+        __syncthreads();
+        // A wavefront copies what a share left.
+        for (uint32_t q = tid / kWave; q < min(shares - s0, 1024u); q += 1024 / kWave) {
+            const uint32_t left = word[q] & ~kSecondBuffer, to = at[q];
+            const size_t src = (word[q] & kSecondBuffer ? second : 0) + static_cast<size_t>(s0 + q) * kHullShare;
+            for (uint32_t i = tid % kWave; i < left && to + i < static_cast<uint32_t>(kHullBig); i += kWave) {
+                X[to + i] = cx[src + i];
+                Y[to + i] = cy[src + i];
+                I[to + i] = ci[src + i];
+            }
+        }
+        cnt += total;
+        __syncthreads();
+    }
+    return cnt;
+}
+
 // Clusters whose candidates still exceed one chunk after the rounds (hulls
-// with hundreds of vertices): one workgroup sorts up to kHullBig candidates
-// in LDS and chains them.
+// with hundreds of vertices) and what is left of shared ones: one workgroup
+// sorts up to kHullBig candidates in LDS and chains them.
 // The same workgroups then redo the flagged clusters (ref_hull).
 __global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, const double2* list_xy) {
     __shared__ double X[kHullBig];
@@ -1187,13 +1276,14 @@ __global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, const dou
     __shared__ bool nlist_done;
     __shared__ int open_list[1024];
     __shared__ int open_n;
+    __shared__ uint32_t share_lds[2 * 1024 + 1024 / kWave + 1];
     const int f = blockIdx.y;
     const int K = static_cast<int>(d.fs[f * kFsCount + kFsClusters]);
     const int tid = threadIdx.x;
     const size_t ob = (size_t)f * L.N;
     const size_t BN = (size_t)L.B * L.N;
-    constexpr int r_in = kHullRounds;
-    const size_t in_b = (size_t)(r_in & 1) * BN;
+    // Mostly nothing is left and no cluster is flagged.
+    if (!d.fs[f * kFsCount + kFsHullLeft] && !d.fs[f * kFsCount + kFsHullInexact]) return;
     // Workgroup x takes the clusters c = x (mod gridDim.x): its threads test
     // 1024 of them at once and list those without a hull yet.
     const int T = static_cast<int>(gridDim.x);
@@ -1206,24 +1296,28 @@ __global__ __launch_bounds__(1024) void k_hull_big(DevBuf d, Layout L, const dou
         const int nopen = open_n;
         for (int jo = 0; jo < nopen; ++jo) {
             const int c = open_list[jo];
-            const uint32_t cnt = d.hc_count[in_b + ob + c];
+            const uint32_t base = d.cl_off[ob + c];
+            uint32_t cnt = d.hc_count[BN + ob + c];
+            const uint32_t shares = hull_shares(cnt);
+            if (shares == 1) {
+                for (uint32_t i = tid; i < min(cnt, static_cast<uint32_t>(kHullBig)); i += 1024) {
+                    const size_t src = BN + ob + base + i;
+                    X[i] = d.hcx[src];
+                    Y[i] = d.hcy[src];
+                    I[i] = d.hci[src];
+                }
+            } else {
+                const size_t at = ob + base;
+                cnt = gather_shares(d.hcx + at, d.hcy + at, d.hci + at, BN, d.hc_chunk_b + at, shares, X, Y, I, share_lds);
+            }
             if (cnt > static_cast<uint32_t>(kHullBig)) {
                 if (tid == 0) atomicOr(&d.fs[f * kFsCount + kFsErr], kErrHullCapacity);
                 continue;
             }
             const int n = static_cast<int>(cnt);
-            const uint32_t base = d.cl_off[ob + c];
             int m = 1;
             while (m < n) m <<= 1;
-            for (int i = tid; i < m; i += 1024) {
-                if (i < n) {
-                    const size_t src = in_b + ob + base + i;
-                    X[i] = d.hcx[src];
-                    Y[i] = d.hcy[src];
-                    I[i] = d.hci[src];
-                }
-                P[i] = static_cast<uint16_t>(i);
-            }
+            for (int i = tid; i < m; i += 1024) P[i] = static_cast<uint16_t>(i);
             __syncthreads();
             for (int k = 2; k <= m; k <<= 1) {
                 for (int j = k >> 1; j > 0; j >>= 1) {
@@ -1728,6 +1822,7 @@ __global__ void k_hull_lists_init(DevBuf d, Layout L, const int32_t* offsets, in
         d.fs[kFsHullInexact] = 0;
         d.fs[kFsHullRounded] = 0;
         d.fs[kFsHullOpen] = 0;
+        d.fs[kFsHullLeft] = 0;
     }
     if (t < K) {
         d.cl_off[t] = static_cast<uint32_t>(offsets[t]);

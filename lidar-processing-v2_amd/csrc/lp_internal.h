@@ -179,11 +179,12 @@ struct DevBuf {
     double* hcy;
     int32_t* hci;            // candidate obstacle index
     uint32_t* hc_count;      // per cluster candidates (two buffers)
-    uint32_t* hc_open;       // clusters of more than one chunk; before the run: the offsets of standalone lists
+    uint32_t* hc_open;       // clusters of more than one chunk, once per taker; before the run: the offsets of standalone lists
     // Per chunk of the first hull round (written by its plan): its cluster,
     // with bit 31 set when the chunk is the cluster's only one (= cell_items,
     // free in the hull stage); its index in the cluster and, from bit 16, its
-    // point count (= cell_zkey); the cluster's first candidate.
+    // point count (= cell_zkey); the cluster's first candidate.  After that
+    // round hc_chunk_b holds, per share of a cluster, what the later ones left.
     int32_t* hc_chunk_c;
     uint32_t* hc_chunk_i;
     uint32_t* hc_chunk_b;
@@ -249,7 +250,8 @@ enum FsSlot : int {
     kFsErr,
     kFsBoxes,          // clusters with a box
     kFsNoisePlaced,    // cell-sorted places given to cells
-    kFsHullOpen,       // clusters of more than one chunk
+    kFsHullOpen,       // entries of hc_open
+    kFsHullLeft,       // clusters and shares of which the rounds left more than a chunk
     kFsCellPoints,     // points in polar cells
     kFsCellsSmall,     // non-empty polar cells of up to 16 points
     kFsCellsLarge,     // larger ones
