@@ -859,7 +859,7 @@ int create_lane(const lp_capacity* cap, lp_context** out) {
     // Every point could occupy its own cell or voxel: the table holds N keys
     // at the chosen worst-case load.
     L.hash_cap = 1 << ceil_log2(static_cast<int64_t>(std::ceil(L.N / static_cast<double>(cap->hash_load_factor))));
-    L.blk_stride = std::max((std::max({L.N, L.P, L.hash_cap}) + 2047) / 2048, (L.N + 1023) / 1024) + 1;
+    L.blk_stride = (L.N + 1023) / 1024 + 1;
     L.box_stride = L.N / 3 + 1024;
     L.obs_rows = (L.N + 63) / 64;
     L.qruns = L.H * ((L.W + 63) / 64);

@@ -193,10 +193,6 @@ __device__ __forceinline__ uint32_t ord_f32(float f) {
     const uint32_t u = f2u(f);
     return (u & 0x80000000u) ? ~u : (u | 0x80000000u);
 }
-__device__ __forceinline__ uint64_t ord_f64(double d) {
-    const uint64_t u = __builtin_bit_cast(uint64_t, d);
-    return (u & 0x8000000000000000ULL) ? ~u : (u | 0x8000000000000000ULL);
-}
 
 // ---- wavefront (64 lanes) helpers --------------------------------------
 constexpr int kWave = 64;
@@ -378,35 +374,7 @@ __device__ __forceinline__ T block_exclusive_sum(T v, T* lds, T* total) {
     return res;
 }
 
-// Places in a counter for R rows of flags: one atomic add by the lowest
-// flagged lane for the whole wavefront; each flagged lane's place is the
-// counter before the add plus the flagged (row, lane) pairs before it, rows
-// in order.
-template <int R>
-__device__ __forceinline__ void wave_reserve(uint32_t* ctr, const bool (&flag)[R], uint32_t (&out)[R]) {
-    uint64_t m[R];
-    uint64_t any = 0;
-    uint32_t total = 0;
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        m[s] = __ballot(flag[s]);
-        any |= m[s];
-        total += static_cast<uint32_t>(__popcll(m[s]));
-    }
-    uint32_t base = 0;
-    if (total) {
-        const int first = static_cast<int>(__ffsll(static_cast<unsigned long long>(any))) - 1;
-        if (lane_id() == first) base = atomicAdd(ctr, total);
-        base = __shfl(base, first, kWave);
-    }
-#pragma unroll
-    for (int s = 0; s < R; ++s) {
-        out[s] = base + lanes_below(m[s]);
-        base += static_cast<uint32_t>(__popcll(m[s]));
-    }
-}
-
-// wave_reserve for a whole workgroup: one atomic add per workgroup
+// Places in a counter for R rows of flags: one atomic add per workgroup
 // (per-frame counters hit by every wavefront are a contention point).  All
 // threads of the workgroup call it; `lds` holds blockDim.x / 64 + 1 words.
 // Places are in (wavefront, row, lane) order.

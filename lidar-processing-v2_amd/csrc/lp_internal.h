@@ -22,7 +22,6 @@ constexpr int kSmallCell = 512;       // cells up to this size are sorted by one
 constexpr int kSlotRecordBytes = 128;  // JCP slots of a queue pixel
 constexpr int kBigCell = 8192;        // larger cells: one workgroup; beyond: capacity error
 constexpr int kHullChunk = 256;       // points per chunk-hull wave
-constexpr int kHullFinal = 8192;      // candidates a final hull workgroup can hold
 constexpr int kNoiseOccWords = 1024 * 1024 / 32;  // noise filter: 1024 x 1024 column bits per frame
 constexpr int32_t kHashMinClean = 0x7fffffff;     // aux of a free hash slot (the voxel minimum's identity)
 
@@ -274,7 +273,7 @@ struct Layout {
     int32_t cell_stride;    // cells per frame (capacity)
     int32_t cand_stride;    // slices*4 capacity
     int32_t hash_cap;       // power of two
-    int32_t blk_stride;     // scan block sums per frame
+    int32_t blk_stride;     // tile totals per frame (tiles of at least 1024 points)
     int32_t box_stride;     // oriented boxes per frame (capacity)
     int32_t obs_rows;       // runs of 64 points per frame
     int32_t qruns;          // runs of 64 columns per frame

@@ -21,7 +21,7 @@ int spread_streams(const std::vector<lp_context*>& contexts);
 void stage_mark(lp_context* c, const char* name);
 
 // Which per-frame count bounds a scan.
-enum ScanCount : int { kCountPoints = 0, kCountPixels = 1, kCountSlot = 2, kCountHash = 3, kCountRawPoints = 4 };
+enum ScanCount : int { kCountPoints = 0, kCountRawPoints, kCountSlot };
 
 // Exclusive scan of `in` into `out` for every frame of the batch; frame f
 // covers in[f*stride .. f*stride + count_f).  The total goes to

@@ -11,11 +11,9 @@ constexpr int kScanThreads = 256;
 constexpr int kScanItems = 8;
 constexpr int kScanTile = kScanThreads * kScanItems;
 
-__device__ __forceinline__ int scan_count(const DevBuf& d, const Layout& L, int f, ScanCount kind, int slot) {
+__device__ __forceinline__ int scan_count(const DevBuf& d, int f, ScanCount kind, int slot) {
     const FrameDesc& fd = d.frames[f];
     if (kind == kCountPoints) return fd.n;
-    if (kind == kCountPixels) return fd.sc.H * fd.sc.W;
-    if (kind == kCountHash) return L.hash_cap;
     if (kind == kCountRawPoints) return fd.n_raw;
     return static_cast<int>(d.fs[f * kFsCount + slot]);
 }
@@ -24,7 +22,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_reduce(DevBuf d, Layout L
                                                               ScanCount kind, int slot) {
     __shared__ uint32_t lds[kScanThreads / kWave + 1];
     const int f = blockIdx.y;
-    const int n = scan_count(d, L, f, kind, slot);
+    const int n = scan_count(d, f, kind, slot);
     const int base = blockIdx.x * kScanTile;
     if (base >= n) return;
     uint32_t s = 0;
@@ -45,7 +43,7 @@ __global__ __launch_bounds__(kScanThreads) void k_scan_down(DevBuf d, Layout L, 
                                                             int total_slot) {
     __shared__ uint32_t lds[kScanThreads / kWave + 1];
     const int f = blockIdx.y;
-    const int n = scan_count(d, L, f, kind, slot);
+    const int n = scan_count(d, f, kind, slot);
     const int tile = blockIdx.x;
     const int base = tile * kScanTile;
     if (base >= n) {

@@ -172,12 +172,6 @@ __global__ void k_cell_fill(DevBuf d, Layout L) {
     d.cell_zkey[(size_t)f * L.N + pos] = ord_f32(d.z[gi]);
 }
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 // Bitonic sort of m (power of two) u32 keys in LDS by NT cooperating
 // threads (tid in [0, NT)); SYNC() orders the stages.
 template <int NT, typename Sync>
